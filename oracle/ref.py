@@ -28,8 +28,8 @@ def available() -> bool:
 
 
 def build(ref_root: str = "/root/reference") -> bool:
-    """Compile the oracle library when the reference tree is present."""
-    if not os.path.isdir(ref_root):
+    """Compile the oracle library when the reference's sources are present."""
+    if not os.path.isdir(os.path.join(ref_root, "src", "pypolymlp", "cxx", "src")):
         return False
     subprocess.run(["make", "-s", "-j8", f"REF_ROOT={ref_root}"], cwd=HERE, check=True)
     return True
