@@ -457,12 +457,16 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
     std::vector<double> pos_dev((size_t)n_atoms * 3), trans;
     std::vector<int> tr_off(n_st + 1, 0), atom_st(n_atoms);
     size_t poff = 0;
-    max_atoms = 0;
+    max_atoms = max_trans = 0;
+    CellInfo info;
+    const bool may_bin = n_st == 1 && n_atoms >= 1024;
     for (int s = 0; s < n_st; ++s) {
         const int n = n_atoms_in[s];
         max_atoms = std::max(max_atoms, n);
         std::vector<double> tr, prev;
-        cell_translations(axes + 9 * (size_t)s, pos + poff, n, cutoff, tr, prev);
+        cell_translations(axes + 9 * (size_t)s, pos + poff, n, cutoff, tr, prev,
+                          may_bin ? &info : nullptr);
+        max_trans = std::max(max_trans, (int)(tr.size() / 3));
         for (int j = 0; j < n; ++j)
             for (int a = 0; a < 3; ++a) pos_dev[3 * (size_t)(atom_off[s] + j) + a] = prev[(size_t)a * n + j];
         trans.insert(trans.end(), tr.begin(), tr.end());
@@ -492,10 +496,7 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
     check_hip(hipMemcpyAsync(d_row_off.ptr, row_off.data(), (n_st + 1) * 4, hipMemcpyHostToDevice, st), "copy");
     // cell-list search for one large structure whose cell spans >= 3 bins of
     // width rc along every lattice direction
-    if (n_st == 1 && n_atoms >= 1024) {
-        CellInfo info;
-        std::vector<double> tr, prev;
-        cell_translations(axes, pos, n_atoms, cutoff, tr, prev, &info);
+    if (may_bin) {
         double inv[9];
         {
             const double* a = info.axis;
@@ -524,77 +525,83 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
             grid.tindex = (const int*)d_tindex.ptr;
         }
     }
-    n_pairs = build_list(false, d_nb_off, d_nb_j, d_nb_t, d_nb_d, nb_off);
+    build_lists();
     max_pairs_atom = 0;
     for (int i = 0; i < n_atoms; ++i) max_pairs_atom = std::max(max_pairs_atom, nb_off[i + 1] - nb_off[i]);
 }
 
-void BatchHandle::prepare_bins() {
-    Device& dev = device();
-    hipStream_t st = dev.stream;
-    const int nbins = grid.nb[0] * grid.nb[1] * grid.nb[2];
-    d_bin.alloc((size_t)n_atoms * 4), d_wrap.alloc((size_t)n_atoms * 12);
-    d_bin_start.alloc((size_t)(nbins + 1) * 4), d_bin_sorted.alloc((size_t)n_atoms * 4);
-    DevBuf cnt, cur;
-    cnt.alloc((size_t)nbins * 4), cur.alloc((size_t)nbins * 4);
-    check_hip(hipMemsetAsync(cnt.ptr, 0, (size_t)nbins * 4, st), "memset");
-    check_hip(hipMemsetAsync(cur.ptr, 0, (size_t)nbins * 4, st), "memset");
-    launch_bin_assign(st, n_atoms, (const double*)d_pos.ptr, grid, (int*)d_bin.ptr, (int*)d_wrap.ptr,
-                      (int*)cnt.ptr);
-    check_hip(hipGetLastError(), "bin assign launch");
-    std::vector<int> c(nbins), start(nbins + 1, 0);
-    check_hip(hipMemcpyAsync(c.data(), cnt.ptr, (size_t)nbins * 4, hipMemcpyDeviceToHost, st), "copy");
+static constexpr double kPairTol = 1e-10;
+
+void BatchHandle::build_lists() {
+    hipStream_t st = device().stream;
+    const double cut2 = cutoff * cutoff;
+    const double tol = kPairTol, tol2 = tol * tol;
+    const double* dpos = (const double*)d_pos.ptr;
+    const double* dtr = (const double*)d_trans.ptr;
+    DevBuf cnt, bin, wrap, bin_count, bin_start, bin_sorted, keys;
+    cnt.alloc((size_t)n_atoms * 8);
+    if (binned) {
+        const size_t nbins = (size_t)grid.nb[0] * grid.nb[1] * grid.nb[2];
+        bin.alloc((size_t)n_atoms * 4), wrap.alloc((size_t)n_atoms * 12);
+        bin_count.alloc(nbins * 4), bin_start.alloc((nbins + 1) * 4);
+        bin_sorted.alloc((size_t)n_atoms * bin_atom_bytes());
+        check_hip(hipMemsetAsync(bin_count.ptr, 0, nbins * 4, st), "memset");
+        launch_bin_atoms(st, n_atoms, dpos, grid, (int*)bin.ptr, (int*)wrap.ptr,
+                         (int*)bin_count.ptr, (int*)bin_start.ptr, bin_sorted.ptr);
+        check_hip(hipGetLastError(), "bin launch");
+        launch_bin_count(st, n_atoms, dpos, (const int*)bin.ptr, (const int*)bin_start.ptr,
+                         bin_sorted.ptr, grid, dtr, cut2, tol2, tol, (int*)cnt.ptr);
+    } else {
+        launch_list_count(st, n_atoms, max_atoms, (const int*)d_atom_st.ptr,
+                          (const int*)d_atom_off.ptr, dpos, (const int*)d_tr_off.ptr, dtr, cut2,
+                          tol2, tol, (int*)cnt.ptr);
+    }
+    check_hip(hipGetLastError(), "neighbor launch");
+    std::vector<int> c((size_t)2 * n_atoms);
+    check_hip(hipMemcpyAsync(c.data(), cnt.ptr, c.size() * 4, hipMemcpyDeviceToHost, st), "copy");
     check_hip(hipStreamSynchronize(st), "sync");
-    for (int b = 0; b < nbins; ++b) start[b + 1] = start[b] + c[b];
-    check_hip(hipMemcpyAsync(d_bin_start.ptr, start.data(), (size_t)(nbins + 1) * 4,
+    nb_off.assign(n_atoms + 1, 0), hb_off.assign(n_atoms + 1, 0);
+    int most = 0;
+    for (int i = 0; i < n_atoms; ++i) {
+        nb_off[i + 1] = nb_off[i] + c[i];
+        hb_off[i + 1] = hb_off[i] + c[n_atoms + i];
+        most = std::max(most, c[i]);
+    }
+    n_pairs = nb_off[n_atoms], n_half = hb_off[n_atoms];
+    const size_t M = std::max<long>(n_pairs, 1);
+    d_nb_off.alloc((size_t)(n_atoms + 1) * 4), d_hb_off.alloc((size_t)(n_atoms + 1) * 4);
+    d_nb_j.alloc(M * 4), d_nb_t.alloc(M * 4), d_nb_d.alloc(M * 24);
+    check_hip(hipMemcpyAsync(d_nb_off.ptr, nb_off.data(), (size_t)(n_atoms + 1) * 4,
                              hipMemcpyHostToDevice, st), "copy");
-    launch_bin_scatter(st, n_atoms, (const int*)d_bin.ptr, (const int*)d_bin_start.ptr, (int*)cur.ptr,
-                       (int*)d_bin_sorted.ptr);
-    check_hip(hipGetLastError(), "bin scatter launch");
+    check_hip(hipMemcpyAsync(d_hb_off.ptr, hb_off.data(), (size_t)(n_atoms + 1) * 4,
+                             hipMemcpyHostToDevice, st), "copy");
+    if (binned) {
+        const size_t kb = bin_key_bytes(n_pairs, most);
+        if (kb) keys.alloc(kb);
+        launch_bin_fill(st, n_atoms, most, dpos, (const int*)bin.ptr, (const int*)bin_start.ptr,
+                        bin_sorted.ptr, grid, dtr, cut2, tol2, tol, (const int*)d_nb_off.ptr,
+                        (int*)d_nb_j.ptr, (int*)d_nb_t.ptr, (double*)d_nb_d.ptr,
+                        kb ? keys.ptr : nullptr);
+    } else {
+        launch_list_fill(st, n_atoms, max_atoms, max_trans, (const int*)d_atom_st.ptr,
+                         (const int*)d_atom_off.ptr, dpos, (const int*)d_tr_off.ptr, dtr, cut2,
+                         tol2, (const int*)d_nb_off.ptr, (int*)d_nb_j.ptr, (int*)d_nb_t.ptr,
+                         (double*)d_nb_d.ptr);
+    }
+    check_hip(hipGetLastError(), "neighbor launch");
     check_hip(hipStreamSynchronize(st), "sync");
 }
 
-long BatchHandle::build_list(bool half, DevBuf& off, DevBuf& nj, DevBuf& nt, DevBuf& nd,
-                             std::vector<int>& host_off) {
-    Device& dev = device();
-    hipStream_t st = dev.stream;
-    const double cut2 = cutoff * cutoff;
-    const double tol = 1e-10, tol2 = tol * tol;
-    if (binned && !d_bin.ptr) prepare_bins();
-    DevBuf cnt;
-    cnt.alloc((size_t)n_atoms * 4);
-    auto run = [&](int* c, const int* o, int* j, int* t, double* d) {
-        if (binned)
-            launch_bin_pairs(st, n_atoms, half ? 1 : 0, (const double*)d_pos.ptr, (const int*)d_bin.ptr,
-                             (const int*)d_wrap.ptr, (const int*)d_bin_start.ptr,
-                             (const int*)d_bin_sorted.ptr, grid, (const double*)d_trans.ptr, cut2,
-                             tol2, tol, c, o, j, t, d);
-        else if (half)
-            launch_neighbor_half(st, n_atoms, (int*)d_atom_st.ptr, (int*)d_atom_off.ptr,
-                                 (double*)d_pos.ptr, (int*)d_tr_off.ptr, (double*)d_trans.ptr, cut2,
-                                 tol2, tol, c, o, j, t, d);
-        else
-            launch_neighbor_full(st, n_atoms, (int*)d_atom_st.ptr, (int*)d_atom_off.ptr,
-                                 (double*)d_pos.ptr, (int*)d_tr_off.ptr, (double*)d_trans.ptr, cut2,
-                                 tol2, c, o, j, t, d);
-        check_hip(hipGetLastError(), "neighbor launch");
-    };
-    run((int*)cnt.ptr, nullptr, nullptr, nullptr, nullptr);
-    std::vector<int> c(n_atoms);
-    check_hip(hipMemcpyAsync(c.data(), cnt.ptr, (size_t)n_atoms * 4, hipMemcpyDeviceToHost, st), "copy");
-    check_hip(hipStreamSynchronize(st), "sync");
-    host_off.assign(n_atoms + 1, 0);
-    for (int i = 0; i < n_atoms; ++i) host_off[i + 1] = host_off[i] + c[i];
-    const long M = host_off[n_atoms];
-    off.alloc((size_t)(n_atoms + 1) * 4);
-    nj.alloc(std::max<long>(M, 1) * 4);
-    nt.alloc(std::max<long>(M, 1) * 4);
-    nd.alloc(std::max<long>(M, 1) * 24);
-    check_hip(hipMemcpyAsync(off.ptr, host_off.data(), (size_t)(n_atoms + 1) * 4,
-                             hipMemcpyHostToDevice, st), "copy");
-    run(nullptr, (const int*)off.ptr, (int*)nj.ptr, (int*)nt.ptr, (double*)nd.ptr);
-    check_hip(hipStreamSynchronize(st), "sync");
-    return M;
+void BatchHandle::ensure_half() {
+    if (has_half) return;
+    hipStream_t st = device().stream;
+    const size_t M = std::max<long>(n_half, 1);
+    d_hb_j.alloc(M * 4), d_hb_t.alloc(M * 4), d_hb_d.alloc(M * 24);
+    launch_half_list(st, n_atoms, kPairTol, (const int*)d_nb_off.ptr, (const int*)d_nb_j.ptr,
+                     (const int*)d_nb_t.ptr, (const double*)d_nb_d.ptr, (const int*)d_hb_off.ptr,
+                     (int*)d_hb_j.ptr, (int*)d_hb_t.ptr, (double*)d_hb_d.ptr);
+    check_hip(hipGetLastError(), "half list launch");
+    has_half = true;
 }
 
 BatchDev BatchHandle::view() const {
@@ -1004,17 +1011,16 @@ int plm_neighbor(const double* axis, const double* pos_c, int n, double cutoff, 
     PLM_TRY({
         std::vector<int> types(n, 0);
         BatchHandle b(nullptr, cutoff, 1, axis, pos_c, types.data(), &n);
-        DevBuf off, nj, nt, nd;
-        std::vector<int> host_off;
-        const long M = half ? b.build_list(true, off, nj, nt, nd, host_off) : b.n_pairs;
-        if (!half) host_off = b.nb_off;
+        if (half) b.ensure_half();
+        const long M = half ? b.n_half : b.n_pairs;
+        const std::vector<int>& host_off = half ? b.hb_off : b.nb_off;
         *n_pairs = M;
         if (capacity < M || !offset) return PLM_OK;
         Device& dev = device();
         hipStream_t st = dev.stream;
-        const DevBuf& J = half ? nj : b.d_nb_j;
-        const DevBuf& T = half ? nt : b.d_nb_t;
-        const DevBuf& D = half ? nd : b.d_nb_d;
+        const DevBuf& J = half ? b.d_hb_j : b.d_nb_j;
+        const DevBuf& T = half ? b.d_hb_t : b.d_nb_t;
+        const DevBuf& D = half ? b.d_hb_d : b.d_nb_d;
         std::memcpy(offset, host_off.data(), (size_t)(n + 1) * 4);
         if (neigh) check_hip(hipMemcpyAsync(neigh, J.ptr, M * 4, hipMemcpyDeviceToHost, st), "copy");
         if (trans_id) check_hip(hipMemcpyAsync(trans_id, T.ptr, M * 4, hipMemcpyDeviceToHost, st), "copy");

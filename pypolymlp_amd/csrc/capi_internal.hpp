@@ -130,12 +130,13 @@ struct ModelHandle {
 struct BatchHandle {
     ModelHandle* model;  // may be null for neighbour-list-only use
     double cutoff = 0.0;
-    int n_st = 0, n_atoms = 0, max_atoms = 0, max_pairs_atom = 0;
+    int n_st = 0, n_atoms = 0, max_atoms = 0, max_trans = 0, max_pairs_atom = 0;
     long n_pairs = 0;
-    std::vector<int> atom_off, row_off, types, nb_off;
+    std::vector<int> atom_off, row_off, types, nb_off, hb_off;
     DevBuf d_types, d_pos, d_trans, d_tr_off, d_atom_st, d_atom_off, d_row_off;
     DevBuf d_nb_off, d_nb_j, d_nb_t, d_nb_d;
-    // half neighbour list (evaluation), built on first use
+    // half neighbour list (evaluation), built from the full one on first use
+    // (its offsets with the full list)
     bool has_half = false;
     long n_half = 0;
     DevBuf d_hb_off, d_hb_j, d_hb_t, d_hb_d;
@@ -143,15 +144,13 @@ struct BatchHandle {
     bool binned = false;
     BinGridHost grid{};
     unsigned long long serial = 0;  // creation number (identifies the batch's rows)
-    DevBuf d_tindex, d_bin, d_wrap, d_bin_start, d_bin_sorted;
+    DevBuf d_tindex;
     BatchHandle(ModelHandle* m, double cutoff, int n_st, const double* axes, const double* pos,
                 const int* types, const int* n_atoms);
     BatchDev view() const;
     void ensure_half();
-    // neighbour list (full or half) into the given buffers; returns pair count
-    long build_list(bool half, DevBuf& off, DevBuf& nj, DevBuf& nt, DevBuf& nd,
-                    std::vector<int>& host_off);
-    void prepare_bins();
+    // the full neighbour list and the offsets of both lists
+    void build_lists();
 };
 
 struct XPlan {

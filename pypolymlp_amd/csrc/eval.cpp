@@ -170,13 +170,6 @@ void upload_potential(ModelHandle& m) {
     ++m.pot_version;
 }
 
-void BatchHandle::ensure_half() {
-    if (has_half) return;
-    std::vector<int> off;
-    n_half = build_list(true, d_hb_off, d_hb_j, d_hb_t, d_hb_d, off);
-    has_half = true;
-}
-
 // Work buffers of one evaluation; out = [energies | forces (3 per atom) | stresses (6)].
 static void alloc_eval(const ModelHandle& m, const BatchHandle& b, bool fp64, DevBuf& a_buf,
                        DevBuf& pse, DevBuf& psf, DevBuf& out, size_t& n_out) {

@@ -125,13 +125,8 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     up(d_atom_st, zeros.data(), (size_t)n * 4);
     up(d_atom_off, atom_off, 8);
     up(d_row_off, row_off, 8);
-    int* cnt_f = d_cnt;
-    int* cnt_h = d_cnt + n;
-    launch_neighbor_full(st, n, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2, cnt_f,
-                         nullptr, nullptr, nullptr, nullptr);
-    check_hip(hipGetLastError(), "neighbor launch");
-    launch_neighbor_half(st, n, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2, tol,
-                         cnt_h, nullptr, nullptr, nullptr, nullptr);
+    launch_list_count(st, n, n, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2, tol,
+                      d_cnt);
     check_hip(hipGetLastError(), "neighbor launch");
     std::vector<int> c((size_t)2 * n);
     check_hip(hipMemcpyAsync(c.data(), d_cnt, (size_t)n * 8, hipMemcpyDeviceToHost, st), "copy");
@@ -159,12 +154,12 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
 
     up(d_nb_off, off_f.data(), (size_t)(n + 1) * 4);
     up(d_hb_off, off_h.data(), (size_t)(n + 1) * 4);
-    launch_neighbor_full(st, n, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2,
-                         nullptr, d_nb_off, d_nb_j, d_nb_t, d_nb_d);
+    launch_list_fill(st, n, n, n_tr, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2,
+                     d_nb_off, d_nb_j, d_nb_t, d_nb_d);
     check_hip(hipGetLastError(), "neighbor launch");
-    launch_neighbor_half(st, n, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2, tol,
-                         nullptr, d_hb_off, d_hb_j, d_hb_t, d_hb_d);
-    check_hip(hipGetLastError(), "neighbor launch");
+    launch_half_list(st, n, tol, d_nb_off, d_nb_j, d_nb_t, d_nb_d, d_hb_off, d_hb_j, d_hb_t,
+                     d_hb_d);
+    check_hip(hipGetLastError(), "half list launch");
 
     BatchDev bd;
     bd.n_st = 1;

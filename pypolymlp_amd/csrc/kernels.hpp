@@ -10,29 +10,40 @@ namespace plm {
 struct XRowsParams;
 struct BlockWz;
 
-void launch_neighbor_full(hipStream_t st, int n, const int* atom_st, const int* st_atom_off,
-                          const double* pos, const int* tr_off, const double* trans, double cut2,
-                          double tol2, int* count, const int* nb_off, int* nb_j, int* nb_t,
-                          double* nb_d);
-void launch_neighbor_half(hipStream_t st, int n, const int* atom_st, const int* st_atom_off,
-                          const double* pos, const int* tr_off, const double* trans, double cut2,
-                          double tol2, double tol, int* count, const int* nb_off, int* nb_j,
-                          int* nb_t, double* nb_d);
+// Neighbour lists (kernels_nb.hip). count: full list counts of the n atoms,
+// then their half list counts. Every (j, T) of each structure:
+void launch_list_count(hipStream_t st, int n, int max_atoms, const int* atom_st,
+                       const int* st_atom_off, const double* pos, const int* tr_off,
+                       const double* trans, double cut2, double tol2, double tol, int* count);
+void launch_list_fill(hipStream_t st, int n, int max_atoms, int max_trans, const int* atom_st,
+                      const int* st_atom_off, const double* pos, const int* tr_off,
+                      const double* trans, double cut2, double tol2, const int* nb_off, int* nb_j,
+                      int* nb_t, double* nb_d);
 
+// a cell list of one large structure
 struct BinGridHost {
     int nb[3];
     int mexp[3];
     double inv[9];
     const int* tindex;  // device pointer
 };
-void launch_bin_assign(hipStream_t st, int n, const double* pos, const BinGridHost& g, int* bin,
-                       int* wrap, int* bin_count);
-void launch_bin_scatter(hipStream_t st, int n, const int* bin, const int* start, int* cursor,
-                        int* sorted);
-void launch_bin_pairs(hipStream_t st, int n, int half, const double* pos, const int* bin,
-                      const int* wrap, const int* start, const int* sorted, const BinGridHost& g,
-                      const double* trans, double cut2, double tol2, double tol, int* count,
-                      const int* nb_off, int* nb_j, int* nb_t, double* nb_d);
+size_t bin_atom_bytes();  // bytes per atom of the bin-ordered copy
+// bin_count: zero on entry
+void launch_bin_atoms(hipStream_t st, int n, const double* pos, const BinGridHost& g, int* bin,
+                      int* wrap, int* bin_count, int* start, void* sorted);
+void launch_bin_count(hipStream_t st, int n, const double* pos, const int* bin, const int* start,
+                      const void* sorted, const BinGridHost& g, const double* trans, double cut2,
+                      double tol2, double tol, int* count);
+// bytes of global sort keys the fill needs (0: they fit LDS)
+size_t bin_key_bytes(long n_pairs, int max_pairs_atom);
+void launch_bin_fill(hipStream_t st, int n, int max_pairs_atom, const double* pos, const int* bin,
+                     const int* start, const void* sorted, const BinGridHost& g,
+                     const double* trans, double cut2, double tol2, double tol, const int* nb_off,
+                     int* nb_j, int* nb_t, double* nb_d, void* keys);
+// the half list from the full one
+void launch_half_list(hipStream_t st, int n, double tol, const int* nb_off, const int* nb_j,
+                      const int* nb_t, const double* nb_d, const int* hb_off, int* hb_j, int* hb_t,
+                      double* hb_d);
 
 size_t anlm_smem(const ModelDev& md, int elem, int nthreads, int max_noconj);
 void launch_anlm(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd, void* a_full,

@@ -1,10 +1,7 @@
-// HIP kernels of the X path for gfx950: brute-force neighbour lists and the
-// order parameters a_{nlm,tp}(i).
+// HIP kernels of the X path for gfx950: the order parameters a_{nlm,tp}(i).
 //
-// Reference loop nests these kernels replace:
-//   NeighborFull          src/cxx/src/compute/neighbor_full.cpp:10-76
-//   NeighborHalf          src/cxx/src/compute/neighbor_half.cpp:10-100
-//   Local::compute_anlmtp_d (values, conjugate fill)  local.cpp:116-217
+// Reference loop nest these kernels replace:
+//   Local::compute_anlmtp_d (values, conjugate fill)  src/cxx/src/compute/local.cpp:116-217
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -19,117 +16,6 @@
 namespace plm {
 
 void check_hip(hipError_t e, const char* what);
-
-// ---------------------------------------------------------------------------
-// Neighbour list: one thread per atom i, brute force over (j, T) in the
-// reference's loop order (j ascending, translations in host order). The
-// distance predicate uses explicitly rounded FP64 operations so the pair set is
-// bit-identical to the reference's (no FMA contraction).
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ bool pair_test(const double* pi, const double* pj, const double* tr,
-                                          double cut2, double tol2, double* d) {
-    const double dxij = __dadd_rn(pj[0], -pi[0]);
-    const double dyij = __dadd_rn(pj[1], -pi[1]);
-    const double dzij = __dadd_rn(pj[2], -pi[2]);
-    const double dx = __dadd_rn(dxij, tr[0]);
-    const double dy = __dadd_rn(dyij, tr[1]);
-    const double dz = __dadd_rn(dzij, tr[2]);
-    const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-    d[0] = dx, d[1] = dy, d[2] = dz;
-    return r2 < cut2 && r2 > tol2;
-}
-
-__global__ void neighbor_full_kernel(int n_atoms_total, const int* __restrict__ atom_st,
-                                     const int* __restrict__ st_atom_off,
-                                     const double* __restrict__ pos,
-                                     const int* __restrict__ tr_off,
-                                     const double* __restrict__ trans, double cut2, double tol2,
-                                     int* __restrict__ count, const int* __restrict__ nb_off,
-                                     int* __restrict__ nb_j, int* __restrict__ nb_t,
-                                     double* __restrict__ nb_d) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_atoms_total) return;
-    const int s = atom_st[i];
-    const int a0 = st_atom_off[s], a1 = st_atom_off[s + 1];
-    const int t0 = tr_off[s], t1 = tr_off[s + 1];
-    const double* pi = pos + 3 * (size_t)i;
-    int c = 0;
-    int out = nb_off ? nb_off[i] : 0;
-    for (int j = a0; j < a1; ++j) {
-        const double* pj = pos + 3 * (size_t)j;
-        for (int t = t0; t < t1; ++t) {
-            double d[3];
-            if (pair_test(pi, pj, trans + 3 * (size_t)t, cut2, tol2, d)) {
-                if (nb_off) {
-                    nb_j[out] = j;
-                    nb_t[out] = t - t0;
-                    nb_d[3 * (size_t)out] = d[0];
-                    nb_d[3 * (size_t)out + 1] = d[1];
-                    nb_d[3 * (size_t)out + 2] = d[2];
-                    ++out;
-                }
-                ++c;
-            }
-        }
-    }
-    if (!nb_off) count[i] = c;
-}
-
-// Half list (neighbor_half.cpp:10-100): j < i, plus self images in the upper
-// half space of the translation.
-__global__ void neighbor_half_kernel(int n_atoms_total, const int* __restrict__ atom_st,
-                                     const int* __restrict__ st_atom_off,
-                                     const double* __restrict__ pos,
-                                     const int* __restrict__ tr_off,
-                                     const double* __restrict__ trans, double cut2, double tol2,
-                                     double tol, int* __restrict__ count,
-                                     const int* __restrict__ nb_off, int* __restrict__ nb_j,
-                                     int* __restrict__ nb_t, double* __restrict__ nb_d) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_atoms_total) return;
-    const int s = atom_st[i];
-    const int a0 = st_atom_off[s];
-    const int t0 = tr_off[s], t1 = tr_off[s + 1];
-    const double* pi = pos + 3 * (size_t)i;
-    int c = 0;
-    int out = nb_off ? nb_off[i] : 0;
-    auto emit = [&](int j, int t, const double* d) {
-        if (nb_off) {
-            nb_j[out] = j;
-            nb_t[out] = t - t0;
-            nb_d[3 * (size_t)out] = d[0];
-            nb_d[3 * (size_t)out + 1] = d[1];
-            nb_d[3 * (size_t)out + 2] = d[2];
-            ++out;
-        }
-        ++c;
-    };
-    for (int j = a0; j < i; ++j) {
-        const double* pj = pos + 3 * (size_t)j;
-        for (int t = t0; t < t1; ++t) {
-            double d[3];
-            if (pair_test(pi, pj, trans + 3 * (size_t)t, cut2, tol2, d)) emit(j, t, d);
-        }
-    }
-    for (int t = t0; t < t1; ++t) {
-        const double* tr = trans + 3 * (size_t)t;
-        const double dx = tr[0], dy = tr[1], dz = tr[2];
-        const double r2 =
-            __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-        if (r2 < cut2 && r2 > tol2) {
-            bool keep;
-            if (dz >= tol) keep = true;
-            else if (fabs(dz) < tol && dy >= tol) keep = true;
-            else if (fabs(dz) < tol && fabs(dy) < tol && dx >= tol) keep = true;
-            else keep = false;
-            if (keep) {
-                double d[3] = {dx, dy, dz};
-                emit(i, t, d);
-            }
-        }
-    }
-    if (!nb_off) count[i] = c;
-}
 
 // ---------------------------------------------------------------------------
 // Order parameters a_{nlm,tp}(i) (noconj accumulation + conjugate fill).
@@ -280,27 +166,6 @@ __global__ void __launch_bounds__(NT) anlm_reg_kernel(ModelDev md, BatchDev bd,
             out[k] = v;
         }
     }
-}
-
-// explicit instantiation via launchers
-void launch_neighbor_full(hipStream_t st, int n, const int* atom_st, const int* st_atom_off,
-                          const double* pos, const int* tr_off, const double* trans, double cut2,
-                          double tol2, int* count, const int* nb_off, int* nb_j, int* nb_t,
-                          double* nb_d) {
-    const int B = 128;
-    neighbor_full_kernel<<<(n + B - 1) / B, B, 0, st>>>(n, atom_st, st_atom_off, pos, tr_off,
-                                                        trans, cut2, tol2, count, nb_off, nb_j,
-                                                        nb_t, nb_d);
-}
-
-void launch_neighbor_half(hipStream_t st, int n, const int* atom_st, const int* st_atom_off,
-                          const double* pos, const int* tr_off, const double* trans, double cut2,
-                          double tol2, double tol, int* count, const int* nb_off, int* nb_j,
-                          int* nb_t, double* nb_d) {
-    const int B = 128;
-    neighbor_half_kernel<<<(n + B - 1) / B, B, 0, st>>>(n, atom_st, st_atom_off, pos, tr_off,
-                                                        trans, cut2, tol2, tol, count, nb_off,
-                                                        nb_j, nb_t, nb_d);
 }
 
 size_t anlm_smem(const ModelDev& md, int elem, int nthreads, int max_noconj) {
