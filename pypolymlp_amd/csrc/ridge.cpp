@@ -9,15 +9,20 @@
 
 #include "capi_internal.hpp"
 #include "profile.hpp"
+#include "solve_batch.hpp"
 
 namespace plm {
 
-void launch_cholesky(hipStream_t st, double* A, int ld, int n_pad, int* info);
-void launch_chol_solve(hipStream_t st, const double* L, int ld, int n_pad, double* z);
-void launch_residual(hipStream_t st, const double* A, int ld, int n, double alpha, const double* x,
-                     const double* b, double* r);
-void launch_add_diag(hipStream_t st, double* A, int ld, int n, double add);
-void launch_axpy(hipStream_t st, int n, const double* d, double* x);
+void launch_cholesky(hipStream_t st, const MatBatch& mb, int n_sys, int ld, int n_pad,
+                     double* side);
+void launch_chol_solve(hipStream_t st, const MatBatch& mb, int n_sys, int ld, int n_pad, double* z,
+                       double* y);
+void launch_residual(hipStream_t st, const double* A, int ld, int n, const MatBatch& mb, int n_sys,
+                     const double* x, const double* b, size_t b_stride, double* r);
+void launch_shifted_copy(hipStream_t st, const double* A, int ld, int n, const MatBatch& mb,
+                         int n_sys);
+void launch_pad_system(hipStream_t st, const double* src, int n, int n_pad, double* A);
+void launch_axpy(hipStream_t st, int n, int ld, int n_sys, const double* d, double* x);
 int solve_block();
 
 void launch_gram_system(hipStream_t st, const double* G, int ldg, int F, const double* s,
@@ -32,6 +37,9 @@ void launch_symv(hipStream_t st, const double* A, int lda, int n, const double* 
 // cache: factors of successful alphas are kept in it while it has room
 // (kFactorBudget) and, for alphas it already holds, reused instead of
 // factoring again.
+// Up to kMatBatch alphas go through each launch together: one factorization is
+// bound by its chain of panels, which leaves most of the chip idle (five alphas
+// at F = 2,277 take little longer than one).
 static constexpr size_t kFactorBudget = 32ull << 30;
 
 static void ridge_core(int F, int np, const DevBuf& A0, const DevBuf& b, const double* alphas,
@@ -39,49 +47,73 @@ static void ridge_core(int F, int np, const DevBuf& A0, const DevBuf& b, const d
                        FactorCache* cache = nullptr) {
     hipStream_t st = device().stream;
     const size_t mat = (size_t)np * np * 8;
-    auto Af = std::make_unique<DevBuf>();
-    DevBuf x, r, di;
-    x.alloc(np * 8), r.alloc(np * 8), di.alloc(4);
-    for (int k = 0; k < n_alpha; ++k) {
-        const double a = alphas[k];
-        const DevBuf* L = nullptr;
-        if (cache)
-            for (const auto& e : cache->f)
-                if (e.first == a) L = e.second.get();
-        int hi = 0;
-        if (!L) {
-            Af->alloc(mat);
-            check_hip(hipMemcpyAsync(Af->ptr, A0.ptr, mat, hipMemcpyDeviceToDevice, st), "copy");
-            launch_add_diag(st, (double*)Af->ptr, np, F, a);
-            check_hip(hipMemsetAsync(di.ptr, 0, 4, st), "memset");
+    int group = std::min(n_alpha, kMatBatch);
+    // several factors at once only where they take at most half of the free memory
+    if (group > 1 && group * mat > (1ull << 30)) {
+        size_t free_b = 0, total = 0;
+        check_hip(hipMemGetInfo(&free_b, &total), "memory info");
+        while (group > 1 && group * mat > free_b / 2) --group;
+    }
+    std::vector<std::unique_ptr<DevBuf>> Af(group);
+    DevBuf x, y, r, side, di;
+    x.alloc((size_t)group * np * 8), y.alloc((size_t)group * np * 8), r.alloc((size_t)group * np * 8);
+    di.alloc(kMatBatch * sizeof(int));
+    for (int k0 = 0; k0 < n_alpha; k0 += group) {
+        const int n = std::min(group, n_alpha - k0);
+        MatBatch all{}, fresh{};
+        int n_fresh = 0, slot[kMatBatch];
+        for (int q = 0; q < n; ++q) {
+            all.alpha[q] = alphas[k0 + q];
+            slot[q] = -1;
+            if (cache)
+                for (const auto& e : cache->f)
+                    if (e.first == alphas[k0 + q]) all.a[q] = (double*)e.second->ptr;
+            if (all.a[q]) continue;
+            if (!Af[q]) Af[q] = std::make_unique<DevBuf>();
+            Af[q]->alloc(mat);
+            all.a[q] = (double*)Af[q]->ptr;
+            slot[q] = n_fresh;
+            fresh.a[n_fresh] = all.a[q], fresh.alpha[n_fresh] = alphas[k0 + q];
+            ++n_fresh;
+        }
+        int hi[kMatBatch] = {};
+        if (n_fresh > 0) {
+            fresh.info = (int*)di.ptr;
+            side.alloc((size_t)n_fresh * np * 64 * 8);
+            check_hip(hipMemsetAsync(di.ptr, 0, kMatBatch * sizeof(int), st), "memset");
+            launch_shifted_copy(st, (const double*)A0.ptr, np, F, fresh, n_fresh);
             {
                 ProfScope ps("cholesky", st);
-                launch_cholesky(st, (double*)Af->ptr, np, np, (int*)di.ptr);
+                launch_cholesky(st, fresh, n_fresh, np, np, (double*)side.ptr);
             }
             check_hip(hipGetLastError(), "cholesky launch");
-            check_hip(hipMemcpyAsync(&hi, di.ptr, 4, hipMemcpyDeviceToHost, st), "copy");
-            check_hip(hipStreamSynchronize(st), "sync");
-            L = Af.get();
+            check_hip(hipMemcpyAsync(hi, di.ptr, n_fresh * sizeof(int), hipMemcpyDeviceToHost, st), "copy");
         }
         {
             ProfScope ps("chol_solve", st);
-            const double* bk = (const double*)b.ptr + k * b_stride;
-            check_hip(hipMemcpyAsync(x.ptr, bk, np * 8, hipMemcpyDeviceToDevice, st), "copy");
-            launch_chol_solve(st, (const double*)L->ptr, np, np, (double*)x.ptr);
+            const double* bk = (const double*)b.ptr + k0 * b_stride;
+            for (int q = 0; q < n; ++q)
+                check_hip(hipMemcpyAsync((double*)x.ptr + (size_t)q * np, bk + q * b_stride, np * 8,
+                                         hipMemcpyDeviceToDevice, st), "copy");
+            launch_chol_solve(st, all, n, np, np, (double*)x.ptr, (double*)y.ptr);
             // one step of iterative refinement
-            check_hip(hipMemsetAsync(r.ptr, 0, np * 8, st), "memset");
-            launch_residual(st, (double*)A0.ptr, np, F, a, (double*)x.ptr, bk, (double*)r.ptr);
-            launch_chol_solve(st, (const double*)L->ptr, np, np, (double*)r.ptr);
-            launch_axpy(st, F, (double*)r.ptr, (double*)x.ptr);
+            check_hip(hipMemsetAsync(r.ptr, 0, (size_t)n * np * 8, st), "memset");
+            launch_residual(st, (const double*)A0.ptr, np, F, all, n, (const double*)x.ptr, bk,
+                            b_stride, (double*)r.ptr);
+            launch_chol_solve(st, all, n, np, np, (double*)r.ptr, (double*)y.ptr);
+            launch_axpy(st, F, np, n, (const double*)r.ptr, (double*)x.ptr);
         }
         check_hip(hipGetLastError(), "solve launch");
-        check_hip(hipMemcpyAsync(coeffs + (size_t)k * F, x.ptr, (size_t)F * 8, hipMemcpyDeviceToHost, st), "copy");
+        for (int q = 0; q < n; ++q)
+            check_hip(hipMemcpyAsync(coeffs + (size_t)(k0 + q) * F, (double*)x.ptr + (size_t)q * np,
+                                     (size_t)F * 8, hipMemcpyDeviceToHost, st), "copy");
         check_hip(hipStreamSynchronize(st), "sync");
-        info[k] = hi;
-        if (cache && L == Af.get() && hi == 0 && cache->bytes + mat <= kFactorBudget) {
-            cache->bytes += mat;
-            cache->f.emplace_back(a, std::move(Af));
-            Af = std::make_unique<DevBuf>();
+        for (int q = 0; q < n; ++q) {
+            info[k0 + q] = slot[q] >= 0 ? hi[slot[q]] : 0;
+            if (cache && slot[q] >= 0 && info[k0 + q] == 0 && cache->bytes + mat <= kFactorBudget) {
+                cache->bytes += mat;
+                cache->f.emplace_back(alphas[k0 + q], std::move(Af[q]));
+            }
         }
     }
 }
@@ -91,16 +123,19 @@ void ridge_solve(int F, const double* xtx, const double* xty, const double* alph
     if (F <= 0 || n_alpha <= 0) throw std::invalid_argument("empty ridge problem");
     const int B = solve_block();
     const int np = (F + B - 1) / B * B;
-    const size_t mat = (size_t)np * np * 8;
-    std::vector<double> h((size_t)np * np, 0.0);
-    for (int i = 0; i < F; ++i) std::memcpy(&h[(size_t)i * np], xtx + (size_t)i * F, (size_t)F * 8);
-    for (int i = F; i < np; ++i) h[(size_t)i * np + i] = 1.0;
-    std::vector<double> hb(np, 0.0);
-    std::memcpy(hb.data(), xty, (size_t)F * 8);
+    hipStream_t st = device().stream;
     DevBuf A0, b;
-    A0.alloc(mat), b.alloc(np * 8);
-    check_hip(hipMemcpy(A0.ptr, h.data(), mat, hipMemcpyHostToDevice), "copy");
-    check_hip(hipMemcpy(b.ptr, hb.data(), np * 8, hipMemcpyHostToDevice), "copy");
+    A0.alloc((size_t)np * np * 8), b.alloc(np * 8);
+    {
+        DevBuf src;  // padded on the device
+        src.alloc((size_t)F * F * 8);
+        check_hip(hipMemcpyAsync(src.ptr, xtx, (size_t)F * F * 8, hipMemcpyHostToDevice, st), "copy");
+        launch_pad_system(st, (const double*)src.ptr, F, np, (double*)A0.ptr);
+        check_hip(hipGetLastError(), "pad launch");
+        check_hip(hipMemsetAsync(b.ptr, 0, np * 8, st), "memset");
+        check_hip(hipMemcpyAsync(b.ptr, xty, (size_t)F * 8, hipMemcpyHostToDevice, st), "copy");
+        check_hip(hipStreamSynchronize(st), "sync");
+    }
     ridge_core(F, np, A0, b, alphas, n_alpha, coeffs, info);
 }
 
