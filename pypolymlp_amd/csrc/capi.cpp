@@ -32,16 +32,104 @@ void check_hip(hipError_t e, const char* what) {
         throw DeviceError(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// ---------------------------------------------------------------------------
+// Device memory pool. A fit allocates and frees tens of GB; freed device memory
+// is not at once available again, so that repeated passes slowed down from 157
+// ms to 0.4-4 s each once they had gone through the card's memory. Released
+// blocks are kept up to an eighth of the device memory (the oldest given back
+// beyond that), all of them but 1 GiB are given back when no buffer is in use,
+// and all when an allocation fails.
+// ---------------------------------------------------------------------------
+namespace {
+
+class DevPool {
+    struct Block {
+        void* ptr;
+        unsigned long long tick;  // release order
+    };
+    std::mutex mu;
+    std::multimap<size_t, Block> idle;          // by size
+    std::map<void*, size_t> in_use;             // block sizes
+    size_t cached = 0, bound = 0;
+    unsigned long long tick = 0;
+
+    // give blocks back, oldest first, until at most keep bytes are cached
+    void trim(size_t keep) {
+        while (cached > keep) {
+            auto old = idle.begin();
+            for (auto it = idle.begin(); it != idle.end(); ++it)
+                if (it->second.tick < old->second.tick) old = it;
+            (void)hipFree(old->second.ptr);
+            cached -= old->first;
+            idle.erase(old);
+        }
+    }
+
+  public:
+    void* take(size_t n) {
+        // whole pages; whole allocation units of the driver above 1 MiB
+        const size_t unit = n < (1u << 20) ? 4096 : (2u << 20);
+        const size_t size = (n + unit - 1) / unit * unit;
+        std::lock_guard<std::mutex> lock(mu);
+        // the smallest idle block that is at most a quarter (small: three times) too large
+        auto it = idle.lower_bound(size);
+        if (it != idle.end() && it->first <= (size < (1u << 20) ? 4 * size : size + size / 4)) {
+            void* p = it->second.ptr;
+            in_use[p] = it->first;
+            cached -= it->first;
+            idle.erase(it);
+            return p;
+        }
+        void* p = nullptr;
+        hipError_t e = hipMalloc(&p, size);
+        if (e == hipErrorOutOfMemory && cached > 0) {
+            (void)hipGetLastError();
+            trim(0);
+            e = hipMalloc(&p, size);
+        }
+        check_hip(e, "hipMalloc");
+        in_use[p] = size;
+        return p;
+    }
+    void give(void* p) {
+        std::lock_guard<std::mutex> lock(mu);
+        auto it = in_use.find(p);
+        if (it == in_use.end()) return;
+        if (bound == 0) {
+            size_t f = 0, total = 0;
+            bound = hipMemGetInfo(&f, &total) == hipSuccess ? total / 8 : (4ull << 30);
+        }
+        idle.emplace(it->second, Block{p, ++tick});
+        cached += it->second;
+        in_use.erase(it);
+        trim(in_use.empty() ? std::min<size_t>(bound, 1ull << 30) : bound);
+    }
+    size_t cached_bytes() {
+        std::lock_guard<std::mutex> lock(mu);
+        return cached;
+    }
+};
+
+// not destroyed: the runtime may be gone before static destructors run
+DevPool& pool() {
+    static DevPool* p = new DevPool;
+    return *p;
+}
+
+}  // namespace
+
+size_t pool_cached_bytes() { return pool().cached_bytes(); }
+
 DevBuf::~DevBuf() { release(); }
 void DevBuf::release() {
-    if (ptr) (void)hipFree(ptr);
+    if (ptr) pool().give(ptr);
     ptr = nullptr, bytes = 0;
 }
 void DevBuf::alloc(size_t n) {
     if (n <= bytes && ptr) return;
     release();
     if (n == 0) n = 16;
-    check_hip(hipMalloc(&ptr, n), "hipMalloc");
+    ptr = pool().take(n);
     bytes = n;
 }
 
@@ -455,7 +543,7 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
     row_off.assign(n_st + 1, 0);
     for (int s = 0; s < n_st; ++s) row_off[s + 1] = row_off[s] + 7 + 3 * n_atoms_in[s];
     std::vector<double> pos_dev((size_t)n_atoms * 3), trans;
-    std::vector<int> tr_off(n_st + 1, 0), atom_st(n_atoms);
+    std::vector<int> tr_off(n_st + 1, 0);
     size_t poff = 0;
     max_atoms = max_trans = 0;
     CellInfo info;
@@ -471,29 +559,12 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
             for (int a = 0; a < 3; ++a) pos_dev[3 * (size_t)(atom_off[s] + j) + a] = prev[(size_t)a * n + j];
         trans.insert(trans.end(), tr.begin(), tr.end());
         tr_off[s + 1] = tr_off[s] + (int)(tr.size() / 3);
-        for (int j = 0; j < n; ++j) atom_st[atom_off[s] + j] = s;
         poff += 3 * (size_t)n;
     }
     types.assign(types_in, types_in + n_atoms);
     if (m)
         for (int t : types)
             if (t < 0 || t >= m->host.n_type()) throw std::invalid_argument("atom type out of range");
-    d_types.alloc(n_atoms * 4);
-    d_pos.alloc(pos_dev.size() * 8);
-    d_trans.alloc(std::max<size_t>(trans.size(), 3) * 8);
-    d_tr_off.alloc((n_st + 1) * 4);
-    d_atom_st.alloc(n_atoms * 4);
-    d_atom_off.alloc((n_st + 1) * 4);
-    d_row_off.alloc((n_st + 1) * 4);
-    hipStream_t st = dev.stream;
-    check_hip(hipMemcpyAsync(d_types.ptr, types.data(), n_atoms * 4, hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_pos.ptr, pos_dev.data(), pos_dev.size() * 8, hipMemcpyHostToDevice, st), "copy");
-    if (!trans.empty())
-        check_hip(hipMemcpyAsync(d_trans.ptr, trans.data(), trans.size() * 8, hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_tr_off.ptr, tr_off.data(), (n_st + 1) * 4, hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_atom_st.ptr, atom_st.data(), n_atoms * 4, hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_atom_off.ptr, atom_off.data(), (n_st + 1) * 4, hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_row_off.ptr, row_off.data(), (n_st + 1) * 4, hipMemcpyHostToDevice, st), "copy");
     // cell-list search for one large structure whose cell spans >= 3 bins of
     // width rc along every lattice direction
     if (may_bin) {
@@ -519,15 +590,41 @@ BatchHandle::BatchHandle(ModelHandle* m, double cutoff_, int n_st_, const double
         if (ok) {
             binned = true;
             for (int a = 0; a < 9; ++a) grid.inv[a] = inv[a];
-            d_tindex.alloc(info.tindex.size() * 4);
-            check_hip(hipMemcpy(d_tindex.ptr, info.tindex.data(), info.tindex.size() * 4,
-                                hipMemcpyHostToDevice), "copy");
-            grid.tindex = (const int*)d_tindex.ptr;
         }
     }
-    build_lists();
-    max_pairs_atom = 0;
-    for (int i = 0; i < n_atoms; ++i) max_pairs_atom = std::max(max_pairs_atom, nb_off[i + 1] - nb_off[i]);
+    // the inputs in one upload
+    std::vector<unsigned char> in;
+    auto reserve = [&](size_t bytes) {
+        const size_t at = in.size();
+        in.resize(at + (bytes + 15) / 16 * 16);
+        return at;
+    };
+    auto put = [&](const void* src, size_t bytes) {
+        const size_t at = reserve(bytes);
+        if (bytes) std::memcpy(in.data() + at, src, bytes);
+        return at;
+    };
+    in.reserve((size_t)n_atoms * 32 + trans.size() * 8 + info.tindex.size() * 4 +
+               (size_t)n_st * 12 + 256);
+    const size_t at_pos = put(pos_dev.data(), pos_dev.size() * 8);
+    const size_t at_trans = put(trans.data(), trans.size() * 8);
+    const size_t at_types = put(types.data(), (size_t)n_atoms * 4);
+    const size_t at_st = reserve((size_t)n_atoms * 4);
+    for (int s = 0; s < n_st; ++s)
+        std::fill((int*)(in.data() + at_st) + atom_off[s], (int*)(in.data() + at_st) + atom_off[s + 1], s);
+    const size_t at_ao = put(atom_off.data(), (size_t)(n_st + 1) * 4);
+    const size_t at_ro = put(row_off.data(), (size_t)(n_st + 1) * 4);
+    const size_t at_to = put(tr_off.data(), (size_t)(n_st + 1) * 4);
+    const size_t at_ti = put(info.tindex.data(), binned ? info.tindex.size() * 4 : 0);
+    d_in.alloc(in.size());
+    check_hip(hipMemcpyAsync(d_in.ptr, in.data(), in.size(), hipMemcpyHostToDevice, dev.stream), "copy");
+    const unsigned char* base = (const unsigned char*)d_in.ptr;
+    d_pos = (const double*)(base + at_pos), d_trans = (const double*)(base + at_trans);
+    d_types = (const int*)(base + at_types), d_atom_st = (const int*)(base + at_st);
+    d_atom_off = (const int*)(base + at_ao), d_row_off = (const int*)(base + at_ro);
+    d_tr_off = (const int*)(base + at_to);
+    grid.tindex = (const int*)(base + at_ti);
+    build_lists();  // waits for the stream, so the upload's source may go
 }
 
 static constexpr double kPairTol = 1e-10;
@@ -536,8 +633,6 @@ void BatchHandle::build_lists() {
     hipStream_t st = device().stream;
     const double cut2 = cutoff * cutoff;
     const double tol = kPairTol, tol2 = tol * tol;
-    const double* dpos = (const double*)d_pos.ptr;
-    const double* dtr = (const double*)d_trans.ptr;
     DevBuf cnt, bin, wrap, bin_count, bin_start, bin_sorted, keys;
     cnt.alloc((size_t)n_atoms * 8);
     if (binned) {
@@ -546,50 +641,42 @@ void BatchHandle::build_lists() {
         bin_count.alloc(nbins * 4), bin_start.alloc((nbins + 1) * 4);
         bin_sorted.alloc((size_t)n_atoms * bin_atom_bytes());
         check_hip(hipMemsetAsync(bin_count.ptr, 0, nbins * 4, st), "memset");
-        launch_bin_atoms(st, n_atoms, dpos, grid, (int*)bin.ptr, (int*)wrap.ptr,
+        launch_bin_atoms(st, n_atoms, d_pos, grid, (int*)bin.ptr, (int*)wrap.ptr,
                          (int*)bin_count.ptr, (int*)bin_start.ptr, bin_sorted.ptr);
         check_hip(hipGetLastError(), "bin launch");
-        launch_bin_count(st, n_atoms, dpos, (const int*)bin.ptr, (const int*)bin_start.ptr,
-                         bin_sorted.ptr, grid, dtr, cut2, tol2, tol, (int*)cnt.ptr);
+        launch_bin_count(st, n_atoms, d_pos, (const int*)bin.ptr, (const int*)bin_start.ptr,
+                         bin_sorted.ptr, grid, d_trans, cut2, tol2, tol, (int*)cnt.ptr);
     } else {
-        launch_list_count(st, n_atoms, max_atoms, (const int*)d_atom_st.ptr,
-                          (const int*)d_atom_off.ptr, dpos, (const int*)d_tr_off.ptr, dtr, cut2,
-                          tol2, tol, (int*)cnt.ptr);
+        launch_list_count(st, n_atoms, max_atoms, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans,
+                          cut2, tol2, tol, (int*)cnt.ptr);
     }
     check_hip(hipGetLastError(), "neighbor launch");
-    std::vector<int> c((size_t)2 * n_atoms);
-    check_hip(hipMemcpyAsync(c.data(), cnt.ptr, c.size() * 4, hipMemcpyDeviceToHost, st), "copy");
+    d_off.alloc((size_t)(n_atoms + 1) * 8);
+    launch_list_offsets(st, n_atoms, (int*)cnt.ptr, (int*)d_off.ptr);
+    check_hip(hipGetLastError(), "offset launch");
+    std::vector<int> off((size_t)2 * (n_atoms + 1));
+    check_hip(hipMemcpyAsync(off.data(), d_off.ptr, off.size() * 4, hipMemcpyDeviceToHost, st), "copy");
     check_hip(hipStreamSynchronize(st), "sync");
-    nb_off.assign(n_atoms + 1, 0), hb_off.assign(n_atoms + 1, 0);
-    int most = 0;
-    for (int i = 0; i < n_atoms; ++i) {
-        nb_off[i + 1] = nb_off[i] + c[i];
-        hb_off[i + 1] = hb_off[i] + c[n_atoms + i];
-        most = std::max(most, c[i]);
-    }
+    nb_off.assign(off.begin(), off.begin() + n_atoms + 1);
+    hb_off.assign(off.begin() + n_atoms + 1, off.end());
+    max_pairs_atom = 0;
+    for (int i = 0; i < n_atoms; ++i) max_pairs_atom = std::max(max_pairs_atom, nb_off[i + 1] - nb_off[i]);
     n_pairs = nb_off[n_atoms], n_half = hb_off[n_atoms];
     const size_t M = std::max<long>(n_pairs, 1);
-    d_nb_off.alloc((size_t)(n_atoms + 1) * 4), d_hb_off.alloc((size_t)(n_atoms + 1) * 4);
     d_nb_j.alloc(M * 4), d_nb_t.alloc(M * 4), d_nb_d.alloc(M * 24);
-    check_hip(hipMemcpyAsync(d_nb_off.ptr, nb_off.data(), (size_t)(n_atoms + 1) * 4,
-                             hipMemcpyHostToDevice, st), "copy");
-    check_hip(hipMemcpyAsync(d_hb_off.ptr, hb_off.data(), (size_t)(n_atoms + 1) * 4,
-                             hipMemcpyHostToDevice, st), "copy");
     if (binned) {
-        const size_t kb = bin_key_bytes(n_pairs, most);
+        const size_t kb = bin_key_bytes(n_pairs, max_pairs_atom);
         if (kb) keys.alloc(kb);
-        launch_bin_fill(st, n_atoms, most, dpos, (const int*)bin.ptr, (const int*)bin_start.ptr,
-                        bin_sorted.ptr, grid, dtr, cut2, tol2, tol, (const int*)d_nb_off.ptr,
-                        (int*)d_nb_j.ptr, (int*)d_nb_t.ptr, (double*)d_nb_d.ptr,
+        launch_bin_fill(st, n_atoms, max_pairs_atom, d_pos, (const int*)bin.ptr,
+                        (const int*)bin_start.ptr, bin_sorted.ptr, grid, d_trans, cut2, tol2, tol,
+                        d_nb_off(), (int*)d_nb_j.ptr, (int*)d_nb_t.ptr, (double*)d_nb_d.ptr,
                         kb ? keys.ptr : nullptr);
     } else {
-        launch_list_fill(st, n_atoms, max_atoms, max_trans, (const int*)d_atom_st.ptr,
-                         (const int*)d_atom_off.ptr, dpos, (const int*)d_tr_off.ptr, dtr, cut2,
-                         tol2, (const int*)d_nb_off.ptr, (int*)d_nb_j.ptr, (int*)d_nb_t.ptr,
+        launch_list_fill(st, n_atoms, max_atoms, max_trans, d_atom_st, d_atom_off, d_pos, d_tr_off,
+                         d_trans, cut2, tol2, d_nb_off(), (int*)d_nb_j.ptr, (int*)d_nb_t.ptr,
                          (double*)d_nb_d.ptr);
     }
     check_hip(hipGetLastError(), "neighbor launch");
-    check_hip(hipStreamSynchronize(st), "sync");
 }
 
 void BatchHandle::ensure_half() {
@@ -597,8 +684,8 @@ void BatchHandle::ensure_half() {
     hipStream_t st = device().stream;
     const size_t M = std::max<long>(n_half, 1);
     d_hb_j.alloc(M * 4), d_hb_t.alloc(M * 4), d_hb_d.alloc(M * 24);
-    launch_half_list(st, n_atoms, kPairTol, (const int*)d_nb_off.ptr, (const int*)d_nb_j.ptr,
-                     (const int*)d_nb_t.ptr, (const double*)d_nb_d.ptr, (const int*)d_hb_off.ptr,
+    launch_half_list(st, n_atoms, kPairTol, d_nb_off(), (const int*)d_nb_j.ptr,
+                     (const int*)d_nb_t.ptr, (const double*)d_nb_d.ptr, d_hb_off(),
                      (int*)d_hb_j.ptr, (int*)d_hb_t.ptr, (double*)d_hb_d.ptr);
     check_hip(hipGetLastError(), "half list launch");
     has_half = true;
@@ -608,12 +695,12 @@ BatchDev BatchHandle::view() const {
     BatchDev b;
     b.n_st = n_st;
     b.n_atoms_total = n_atoms;
-    b.st_atom_off = (const int*)d_atom_off.ptr;
-    b.st_row_off = (const int*)d_row_off.ptr;
-    b.types = (const int*)d_types.ptr;
-    b.atom_st = (const int*)d_atom_st.ptr;
-    b.pos = (const double*)d_pos.ptr;
-    b.nb_off = (const int*)d_nb_off.ptr;
+    b.st_atom_off = d_atom_off;
+    b.st_row_off = d_row_off;
+    b.types = d_types;
+    b.atom_st = d_atom_st;
+    b.pos = d_pos;
+    b.nb_off = d_nb_off();
     b.nb_j = (const int*)d_nb_j.ptr;
     b.nb_d = (const double*)d_nb_d.ptr;
     return b;

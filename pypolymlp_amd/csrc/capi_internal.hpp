@@ -27,6 +27,9 @@ struct DeviceError : std::runtime_error {
 
 void check_hip(hipError_t e, const char* what);
 
+// Device memory from the library's pool (capi.cpp): released blocks are kept
+// for later buffers of all handles. Everything the library enqueues goes
+// through one stream, so a block may be handed on while work on it is queued.
 struct DevBuf {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -37,6 +40,7 @@ struct DevBuf {
     void alloc(size_t n);
     void release();
 };
+size_t pool_cached_bytes();  // device memory held by the pool's free blocks
 
 struct Device {
     bool init = false;
@@ -124,6 +128,7 @@ struct ModelHandle {
     // work buffers of eager evaluations (order parameters, head sums, results),
     // kept and grown across calls; eval_mutex serialises the calls that use them
     DevBuf ev_a, ev_pse, ev_psf, ev_out;
+    std::vector<double> ev_host;
     std::mutex eval_mutex;
 };
 
@@ -133,18 +138,23 @@ struct BatchHandle {
     int n_st = 0, n_atoms = 0, max_atoms = 0, max_trans = 0, max_pairs_atom = 0;
     long n_pairs = 0;
     std::vector<int> atom_off, row_off, types, nb_off, hb_off;
-    DevBuf d_types, d_pos, d_trans, d_tr_off, d_atom_st, d_atom_off, d_row_off;
-    DevBuf d_nb_off, d_nb_j, d_nb_t, d_nb_d;
+    DevBuf d_in;  // the inputs, uploaded in one copy; the pointers below are into it
+    const int *d_types = nullptr, *d_tr_off = nullptr, *d_atom_st = nullptr,
+              *d_atom_off = nullptr, *d_row_off = nullptr;
+    const double *d_pos = nullptr, *d_trans = nullptr;
+    DevBuf d_off;  // list offsets: n_atoms + 1 of the full list, then of the half list
+    DevBuf d_nb_j, d_nb_t, d_nb_d;
+    const int* d_nb_off() const { return (const int*)d_off.ptr; }
+    const int* d_hb_off() const { return (const int*)d_off.ptr + n_atoms + 1; }
     // half neighbour list (evaluation), built from the full one on first use
     // (its offsets with the full list)
     bool has_half = false;
     long n_half = 0;
-    DevBuf d_hb_off, d_hb_j, d_hb_t, d_hb_d;
+    DevBuf d_hb_j, d_hb_t, d_hb_d;
     // cell-list search (single large structure)
     bool binned = false;
     BinGridHost grid{};
     unsigned long long serial = 0;  // creation number (identifies the batch's rows)
-    DevBuf d_tindex;
     BatchHandle(ModelHandle* m, double cutoff, int n_st, const double* axes, const double* pos,
                 const int* types, const int* n_atoms);
     BatchDev view() const;

@@ -215,15 +215,16 @@ void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, con
 
 static void enqueue_eval(ModelHandle& m, BatchHandle& b, bool fp64, void* a_buf, void* pse,
                          void* psf, double* out, size_t n_out, hipStream_t st) {
-    enqueue_eval_dev(m, b.view(), (const int*)b.d_hb_off.ptr, (const int*)b.d_hb_j.ptr,
+    enqueue_eval_dev(m, b.view(), b.d_hb_off(), (const int*)b.d_hb_j.ptr,
                      (const double*)b.d_hb_d.ptr, (int)b.n_half, fp64, a_buf, pse, psf, out,
                      n_out, st);
 }
 
+// h: staging on the host (kept by the caller, so that its pages are in place)
 static void copy_out(const BatchHandle& b, const DevBuf& out, size_t n_out, hipStream_t st,
-                     double* energies, double* forces, double* stresses) {
+                     std::vector<double>& h, double* energies, double* forces, double* stresses) {
     const size_t A = b.n_atoms;
-    std::vector<double> h(n_out);
+    if (h.size() < n_out) h.resize(n_out);
     check_hip(hipMemcpyAsync(h.data(), out.ptr, n_out * 8, hipMemcpyDeviceToHost, st), "copy");
     check_hip(hipStreamSynchronize(st), "sync");
     if (energies) std::memcpy(energies, h.data(), (size_t)b.n_st * 8);
@@ -246,7 +247,7 @@ void eval_batch(ModelHandle& m, BatchHandle& b, bool fp64, double* energies, dou
     alloc_eval(m, b, fp64, m.ev_a, m.ev_pse, m.ev_psf, m.ev_out, n_out);
     enqueue_eval(m, b, fp64, m.ev_a.ptr, m.ev_pse.ptr, m.ev_psf.ptr, (double*)m.ev_out.ptr, n_out,
                  st);
-    copy_out(b, m.ev_out, n_out, st, energies, forces, stresses);
+    copy_out(b, m.ev_out, n_out, st, m.ev_host, energies, forces, stresses);
 }
 
 EvalGraph::~EvalGraph() {
@@ -287,7 +288,8 @@ void eval_graph_run(EvalGraph& g, int steps, double* energies, double* forces, d
         throw std::invalid_argument("model coefficients changed since the graph was captured");
     hipStream_t st = device().stream;
     for (int k = 0; k < steps; ++k) check_hip(hipGraphLaunch(g.exec, st), "graph launch");
-    copy_out(*g.b, g.out, g.n_out, st, energies, forces, stresses);
+    std::vector<double> h;
+    copy_out(*g.b, g.out, g.n_out, st, h, energies, forces, stresses);
 }
 
 void eval_single(ModelHandle& m, const double* axis, const double* pos_c, const int* types, int n,

@@ -15,6 +15,8 @@ struct BlockWz;
 void launch_list_count(hipStream_t st, int n, int max_atoms, const int* atom_st,
                        const int* st_atom_off, const double* pos, const int* tr_off,
                        const double* trans, double cut2, double tol2, double tol, int* count);
+// off: n + 1 offsets of the full lists, then n + 1 of the half lists
+void launch_list_offsets(hipStream_t st, int n, int* count, int* off);
 void launch_list_fill(hipStream_t st, int n, int max_atoms, int max_trans, const int* atom_st,
                       const int* st_atom_off, const double* pos, const int* tr_off,
                       const double* trans, double cut2, double tol2, const int* nb_off, int* nb_j,

@@ -50,6 +50,43 @@ __device__ __forceinline__ int wave_inclusive(int v, int lane) {
     return v;
 }
 
+// start[k] = sum of count[< k], start[n] = the total, for the counts of
+// workgroup blockIdx.x (n each); clear: the counts become zero
+__global__ void __launch_bounds__(1024) scan_kernel(int n, int* __restrict__ count,
+                                                    int* __restrict__ start, int clear) {
+    __shared__ int part[16];
+    count += (size_t)n * blockIdx.x, start += (size_t)(n + 1) * blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int base = 0;
+    for (int k0 = 0; k0 < n; k0 += 4096) {
+        const int k = k0 + 4 * threadIdx.x;
+        int c[4], sum = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            c[u] = k + u < n ? count[k + u] : 0;
+            sum += c[u];
+        }
+        const int incl = wave_inclusive(sum, lane);
+        if (lane == 63) part[wave] = incl;
+        __syncthreads();
+        int out = base + incl - sum, all = 0;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) out += part[w];
+            all += part[w];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < n) {
+                start[k + u] = out;
+                if (clear) count[k + u] = 0;
+                out += c[u];
+            }
+        base += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) start[n] = base;
+}
+
 // ---------------------------------------------------------------------------
 // All (j, T) of the structure. One workgroup per atom i (a wave per 64 atoms
 // of its structure, at most four), one lane per j: the difference r_j - r_i is
@@ -215,30 +252,6 @@ __global__ void bin_assign_kernel(int n, const double* __restrict__ pos, BinGrid
     const int id = (b[0] * g.nb[1] + b[1]) * g.nb[2] + b[2];
     bin[i] = id;
     atomicAdd(bin_count + id, 1);
-}
-
-// start[b] = sum of count[< b], start[nbins] = n; one workgroup
-__global__ void __launch_bounds__(1024) bin_scan_kernel(int nbins, int* __restrict__ count,
-                                                        int* __restrict__ start) {
-    __shared__ int part[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int base = 0;
-    for (int b0 = 0; b0 < nbins; b0 += 1024) {
-        const int b = b0 + threadIdx.x;
-        const int c = b < nbins ? count[b] : 0;
-        const int incl = wave_inclusive(c, lane);
-        if (lane == 63) part[wave] = incl;
-        __syncthreads();
-        int out = base + incl - c, all = 0;
-        for (int w = 0; w < 16; ++w) {
-            if (w < wave) out += part[w];
-            all += part[w];
-        }
-        if (b < nbins) start[b] = out, count[b] = 0;  // the counts become the scatter's cursors
-        base += all;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) start[nbins] = base;
 }
 
 __global__ void bin_scatter_kernel(int n, const int* __restrict__ bin, const int* __restrict__ start,
@@ -414,6 +427,10 @@ void launch_list_fill(hipStream_t st, int n, int max_atoms, int max_trans, const
             atom_st, st_atom_off, pos, tr_off, trans, cut2, tol2, nb_off, nb_j, nb_t, nb_d);
 }
 
+void launch_list_offsets(hipStream_t st, int n, int* count, int* off) {
+    scan_kernel<<<2, 1024, 0, st>>>(n, count, off, 0);
+}
+
 static BinGrid device_grid(const BinGridHost& gh) {
     BinGrid g;
     for (int a = 0; a < 3; ++a) g.nb[a] = gh.nb[a], g.mexp[a] = gh.mexp[a];
@@ -428,7 +445,7 @@ void launch_bin_atoms(hipStream_t st, int n, const double* pos, const BinGridHos
                       int* wrap, int* bin_count, int* start, void* sorted) {
     const int nbins = gh.nb[0] * gh.nb[1] * gh.nb[2];
     bin_assign_kernel<<<(n + 255) / 256, 256, 0, st>>>(n, pos, device_grid(gh), bin, wrap, bin_count);
-    bin_scan_kernel<<<1, 1024, 0, st>>>(nbins, bin_count, start);
+    scan_kernel<<<1, 1024, 0, st>>>(nbins, bin_count, start, 1);  // the counts become cursors
     bin_scatter_kernel<<<(n + 255) / 256, 256, 0, st>>>(n, bin, start, pos, wrap, bin_count,
                                                         static_cast<BinAtom*>(sorted));
 }

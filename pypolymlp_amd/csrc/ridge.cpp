@@ -52,6 +52,7 @@ static void ridge_core(int F, int np, const DevBuf& A0, const DevBuf& b, const d
     if (group > 1 && group * mat > (1ull << 30)) {
         size_t free_b = 0, total = 0;
         check_hip(hipMemGetInfo(&free_b, &total), "memory info");
+        free_b += pool_cached_bytes();
         while (group > 1 && group * mat > free_b / 2) --group;
     }
     std::vector<std::unique_ptr<DevBuf>> Af(group);

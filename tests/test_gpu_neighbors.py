@@ -86,3 +86,27 @@ def test_dense_cluster_sort_keys(n):
     assert np.array_equal(np.diff(hoff), full)
     keep = nb < np.repeat(full, n - 1)
     assert np.array_equal(hnb, nb[keep]) and np.array_equal(hd, d[keep])
+
+
+@pytest.mark.parametrize("name", ["bins", "thin"])
+def test_lists_beyond_one_scan_round(name):
+    """More atoms than one round of the offsets' prefix sum (4,096), by both
+    searches: some atoms' lists against the host, and every pair from both ends."""
+    n, rc = 4500, 4.0
+    axis, pos = cell(n, (34.0, 33.0, 32.0) if name == "bins" else (95.0, 95.0, 4.0), 5)
+    off, nb, tid, d = capi.neighbor(axis, pos, rc)
+    assert off[-1] == len(nb) and np.all(np.diff(off) >= 0)
+    tr, p = capi.cell_translations(axis, pos, rc)
+    for i in (0, 1, 1023, 4094, 4095, 4096, 4097, n - 1):
+        v = (p - p[:, i:i + 1]).T[:, None, :] + tr[None]
+        r2 = (v[..., 0] * v[..., 0] + v[..., 1] * v[..., 1]) + v[..., 2] * v[..., 2]
+        j, t = np.nonzero((r2 < rc * rc) & (r2 > 1e-20))
+        seg = slice(off[i], off[i + 1])
+        assert np.array_equal(nb[seg], j) and np.array_equal(tid[seg], t)
+        assert np.array_equal(d[seg], v[j, t])
+    i = np.repeat(np.arange(n), np.diff(off))
+    assert np.array_equal(np.sort(i * n + nb), np.sort(nb * n + i))
+    hoff, hnb, _, hd = capi.neighbor(axis, pos, rc, half=True)
+    low = nb < i
+    own = hnb == np.repeat(np.arange(n), np.diff(hoff))
+    assert np.array_equal(hnb[~own], nb[low]) and np.array_equal(hd[~own], d[low])
