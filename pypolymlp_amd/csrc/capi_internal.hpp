@@ -200,10 +200,10 @@ std::vector<long> poly_d_offsets(ModelHandle& m, const BatchHandle& b, int s0, i
 size_t poly_bytes(ModelHandle& m, const BatchHandle& b, int s0, int s1, bool fp64);
 size_t pair_record_bytes(const ModelHandle& m, bool fp64);
 
-// Work buffers of an accumulation: X of a sub-batch, its quantised slices,
-// and the X build's per-atom and per-pair buffers (grown as needed).
+// Work buffers of an accumulation: X of a sub-batch, its quantised slices, the
+// row splits of the FP64 Gram, and the X build's per-atom and per-pair buffers (grown as needed).
 struct AccumWork {
-    DevBuf xbuf, qbuf;
+    DevBuf xbuf, qbuf, part;
     XWork work;
 };
 

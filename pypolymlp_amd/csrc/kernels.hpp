@@ -156,8 +156,10 @@ void launch_pair(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& e
 // (gram_quant_bytes) then accumulate the exact Gram of the quantised X.
 void launch_set_column(hipStream_t st, bool fp64, void* X, int ld, int col, const double* y,
                        int rows);
+// part: gram_f64_part_bytes of scratch for the row splits (unused where that is 0)
+size_t gram_f64_part_bytes(int rows_pad, int F_pad);
 void launch_gram_f64(hipStream_t st, const double* X, int ld, int rows_pad, int F_pad, double* C,
-                     int ldc);
+                     int ldc, void* part);
 // Row q of the quantised matrix is row rmap[q] of X (zero where rmap[q] < 0).
 // Quantisation exponents are shared per column over chunks of rows: the first
 // h0 rows (a multiple of 64, at most gram_chunk_rows()), then

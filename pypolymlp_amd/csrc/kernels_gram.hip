@@ -23,69 +23,144 @@
 
 #include <stdexcept>
 
+#include <algorithm>
+
 #include "kernels.hpp"
+#include "solve_batch.hpp"
 
 namespace plm {
 
+void check_hip(hipError_t e, const char* what);
+
 typedef __attribute__((__vector_size__(4 * sizeof(double)))) double doublex4;
+typedef double doublex2 __attribute__((ext_vector_type(2)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-// Map a linear tile id to (bi, bj) with bi <= bj over nb blocks.
-__device__ __forceinline__ void tri_index(int t, int nb, int& bi, int& bj) {
-    // rows of the upper triangle: row bi has nb - bi tiles
-    int r = 0, rem = t;
-    while (rem >= nb - r) rem -= nb - r, ++r;
-    bi = r, bj = r + rem;
-}
-
 // ---------------------------------------------------------------------------
-// FP64: 64x64 output tile per 256-thread workgroup; each wave a 32x32 quarter
-// as 2x2 MFMA 16x16 blocks; K step 16 rows through LDS.
+// FP64: 128 x 128 output tile per 512-thread workgroup, each of the eight waves
+// a 64 x 32 part (4 x 2 MFMA blocks, 64 accumulator registers), two workgroups
+// a CU. 16 rows per stage through two LDS buffers (row pitch 144: the two rows
+// that half an operand read spans fall into the two halves of the banks), the
+// stage after next in registers. Bound by FP64 MFMA issue. A 64-wide tile reads
+// its panels at 8 flops a byte, which held the kernel at 42 TFLOP/s; this one
+// runs at 68 (F = 13,020, 35,190 rows: 139 -> 87 ms; a large library product
+// reaches 69); consecutive tiles of an XCD share panels in its L2.
+// Tiles tile0 .. tile0 + tiles; blockIdx.y: row split (launch_gram_f64), whose
+// results go to part.
 // ---------------------------------------------------------------------------
-constexpr int G64_T = 64;
-constexpr int G64_K = 16;
+constexpr int G64_T = 128, G64_K = 16, G64_P = 144;
+constexpr size_t kGram64Lds = (size_t)2 * 2 * G64_K * G64_P * 8;
+constexpr int kGram64Slots = 512;  // workgroups resident at once (two a CU)
 
-__global__ void __launch_bounds__(256) gram_f64_kernel(const double* __restrict__ X, int ld,
-                                                       int rows, int nb, double* __restrict__ C,
-                                                       int ldc) {
-    __shared__ double As[G64_K][G64_T + 1];
-    __shared__ double Bs[G64_K][G64_T + 1];
+template <bool SPLIT>
+__global__ void __launch_bounds__(512, 4) gram_f64_kernel(const double* __restrict__ X, int ld,
+                                                          int rows, int rows_split, int nb,
+                                                          int tile0, int tiles,
+                                                          double* __restrict__ C, int ldc,
+                                                          double* __restrict__ part) {
+    extern __shared__ __attribute__((aligned(16))) double sm64[];
+    const int per = (tiles + 7) >> 3;
+    const int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || t >= tiles) return;
     int bi, bj;
-    tri_index(blockIdx.x, nb, bi, bj);
+    tri_super_tile(tile0 + t, nb, bi, bj);
     const int I0 = bi * G64_T, J0 = bj * G64_T;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wi = (wave >> 1) * 32, wj = (wave & 1) * 32;
-    doublex4 acc[2][2];
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b) acc[a][b] = doublex4{0, 0, 0, 0};
-    for (int k0 = 0; k0 < rows; k0 += G64_K) {
-        __syncthreads();
-        for (int e = tid; e < G64_K * G64_T; e += 256) {
-            const int kk = e / G64_T, c = e % G64_T;
-            const size_t r = (size_t)(k0 + kk) * ld;
-            As[kk][c] = X[r + I0 + c];
-            Bs[kk][c] = X[r + J0 + c];
+    const int wi = (wave & 1) * 64, wj = (wave >> 1) * 32;
+    doublex4 acc[4][2];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[m][q] = doublex4{0, 0, 0, 0};
+    const int row0 = SPLIT ? blockIdx.y * rows_split : 0;
+    const int nst = (SPLIT ? min(rows_split, rows - row0) : rows) / G64_K;
+    // 16 rows x 64 pairs of columns a panel and stage, two pieces a thread
+    const double* pa = X + (size_t)(row0 + wave) * ld + I0 + 2 * lane;
+    const double* pb = X + (size_t)(row0 + wave) * ld + J0 + 2 * lane;
+    doublex2 ra[2], rb[2];
+    auto load = [&](int st) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            ra[u] = *reinterpret_cast<const doublex2*>(pa + (size_t)(G64_K * st + 8 * u) * ld);
+            rb[u] = *reinterpret_cast<const doublex2*>(pb + (size_t)(G64_K * st + 8 * u) * ld);
+        }
+    };
+    auto store = [&](int buf) {
+        double* a = sm64 + buf * 2 * G64_K * G64_P + wave * G64_P + 2 * lane;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            *reinterpret_cast<doublex2*>(a + 8 * u * G64_P) = ra[u];
+            *reinterpret_cast<doublex2*>(a + (G64_K + 8 * u) * G64_P) = rb[u];
+        }
+    };
+    load(0);
+    store(0);
+    load(min(1, nst - 1));
+    __syncthreads();
+    for (int st = 0; st < nst; ++st) {
+        const double* a = sm64 + (st & 1) * 2 * G64_K * G64_P + (lane >> 4) * G64_P + wi + (lane & 15);
+        const double* b = a + G64_K * G64_P - wi + wj;
+        store((st + 1) & 1);
+        load(min(st + 2, nst - 1));
+#pragma unroll
+        for (int ks = 0; ks < G64_K; ks += 4) {
+            double x[4], y[2];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) x[m] = a[ks * G64_P + 16 * m];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) y[q] = b[ks * G64_P + 16 * q];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    acc[m][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[m], y[q], acc[m][q], 0, 0, 0);
         }
         __syncthreads();
-        for (int ks = 0; ks < G64_K; ks += 4) {
-            const int kk = ks + (lane >> 4);
-            double a[2], b[2];
-            for (int m = 0; m < 2; ++m) a[m] = As[kk][wi + 16 * m + (lane & 15)];
-            for (int n = 0; n < 2; ++n) b[n] = Bs[kk][wj + 16 * n + (lane & 15)];
-            for (int m = 0; m < 2; ++m)
-                for (int n = 0; n < 2; ++n)
-                    acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], b[n], acc[m][n], 0, 0, 0);
+    }
+    // D[l/16 + 4v][l%16] of each 16 x 16 block
+    const int i0 = wi + (lane >> 4), j0 = wj + (lane & 15);
+    if constexpr (SPLIT) {
+        double* o = part + ((size_t)blockIdx.y * tiles + t) * G64_T * G64_T + i0 * G64_T + j0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[(16 * m + 4 * v) * G64_T + 16 * q] = acc[m][q][v];
+    } else {
+        double* o = C + (size_t)(I0 + i0) * ldc + J0 + j0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            double c[2][4];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) c[q][v] = o[(size_t)(16 * m + 4 * v) * ldc + 16 * q];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    o[(size_t)(16 * m + 4 * v) * ldc + 16 * q] = c[q][v] + acc[m][q][v];
         }
     }
-    // D[l/16 + 4v][l%16] of each 16x16 block
-    for (int m = 0; m < 2; ++m)
-        for (int n = 0; n < 2; ++n)
-            for (int v = 0; v < 4; ++v) {
-                const int i = I0 + wi + 16 * m + (lane >> 4) + 4 * v;
-                const int j = J0 + wj + 16 * n + (lane & 15);
-                C[(size_t)i * ldc + j] += acc[m][n][v];
-            }
+}
+
+// C += the splits' tiles, in their order
+__global__ void __launch_bounds__(256) gram_f64_sum_kernel(const double* __restrict__ part, int nb,
+                                                           int tile0, int tiles, int splits,
+                                                           double* __restrict__ C, int ldc) {
+    const int t = blockIdx.x;
+    int bi, bj;
+    tri_super_tile(tile0 + t, nb, bi, bj);
+    const int e = blockIdx.y * 512 + 2 * threadIdx.x;  // two of the tile's elements
+    doublex2 s = {0.0, 0.0};
+#pragma unroll 4
+    for (int k = 0; k < splits; ++k)
+        s += *reinterpret_cast<const doublex2*>(part + ((size_t)k * tiles + t) * G64_T * G64_T + e);
+    doublex2* c = reinterpret_cast<doublex2*>(C + (size_t)(bi * G64_T + e / G64_T) * ldc +
+                                              bj * G64_T + e % G64_T);
+    *c += s;
 }
 
 // ---------------------------------------------------------------------------
@@ -441,10 +516,53 @@ size_t gram_quant_bytes(int rows_pad, int h0, int ld) {
     return 3 * (size_t)rows_pad * ld + (size_t)n_chunks_of(rows_pad, h0) * ld * sizeof(int);
 }
 
+// The FP64 Gram's tiles go in whole rounds of resident workgroups; the rows of
+// the remaining tiles are split so that their round, too, fills the chip (F =
+// 13,020: 5,253 tiles are 10 rounds and 133 tiles, and an eleventh round cost
+// 1 of 88 ms; F = 2,277: 171 tiles in one launch left 85 CUs idle, 5.9 ms for
+// 33,800 rows against 3.5 ms in 11 splits). Each split keeps at least 512 rows.
+static int gram_f64_splits(int tiles, int rows) {
+    const int per = (tiles + 7) / 8, slots = kGram64Slots / 8;  // of one XCD
+    int best = 1;
+    double cost = 1e30;
+    for (int s = 1; s <= 32 && (s == 1 || rows / s >= 512); ++s) {
+        // rounds of 1 / s of the rows each, and the traffic of the partial tiles
+        const double c = (double)((per * s + slots - 1) / slots) / s + 0.002 * s;
+        if (c < cost) cost = c, best = s;
+    }
+    return best;
+}
+
+size_t gram_f64_part_bytes(int rows_pad, int F_pad) {
+    const int nb = F_pad / G64_T, rest = nb * (nb + 1) / 2 % kGram64Slots;
+    const int splits = gram_f64_splits(rest, rows_pad);
+    return splits == 1 ? 0 : (size_t)splits * rest * G64_T * G64_T * 8;
+}
+
 void launch_gram_f64(hipStream_t st, const double* X, int ld, int rows_pad, int F_pad, double* C,
-                     int ldc) {
-    const int nb = F_pad / G64_T;
-    gram_f64_kernel<<<nb * (nb + 1) / 2, 256, 0, st>>>(X, ld, rows_pad, nb, C, ldc);
+                     int ldc, void* part) {
+    if (F_pad % G64_T || rows_pad % G64_K) throw std::invalid_argument("FP64 Gram tile sizes");
+    const int nb = F_pad / G64_T, tiles = nb * (nb + 1) / 2;
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gram_f64_kernel<false>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGram64Lds),
+              "Gram shared memory");
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&gram_f64_kernel<true>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGram64Lds),
+              "Gram shared memory");
+    const int rest = tiles % kGram64Slots;
+    int splits = rest > 0 ? gram_f64_splits(rest, rows_pad) : 1;
+    const int whole = splits == 1 ? tiles : tiles - rest;
+    if (whole > 0)
+        gram_f64_kernel<false><<<(whole + 7) / 8 * 8, 512, kGram64Lds, st>>>(
+            X, ld, rows_pad, rows_pad, nb, 0, whole, C, ldc, nullptr);
+    if (splits == 1) return;
+    const int rs = ((rows_pad + splits - 1) / splits + G64_K - 1) / G64_K * G64_K;
+    splits = (rows_pad + rs - 1) / rs;  // none is empty
+    double* p = static_cast<double*>(part);
+    gram_f64_kernel<true><<<dim3((rest + 7) / 8 * 8, splits), 512, kGram64Lds, st>>>(
+        X, ld, rows_pad, rs, nb, whole, rest, C, ldc, p);
+    gram_f64_sum_kernel<<<dim3(rest, G64_T * G64_T / 512), 256, 0, st>>>(p, nb, whole, rest, splits,
+                                                                         C, ldc);
 }
 
 int gram_chunk_rows() { return kQChunk; }

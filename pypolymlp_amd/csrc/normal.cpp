@@ -144,9 +144,10 @@ void enqueue_accumulate(NormalHandle& acc, BatchHandle& b, const AccumPlan& plan
         launch_set_column(st, fp64, xb, ld, F, y + r0, (int)sb.rows);
         check_hip(hipGetLastError(), "target column");
         if (!plan.quant) {
+            if (const size_t n = gram_f64_part_bytes((int)sb.rows_pad, acc.F_pad)) ws.part.alloc(n);
             ProfScope ps("gram", st);
             launch_gram_f64(st, reinterpret_cast<const double*>(xb), ld, (int)sb.rows_pad,
-                            acc.F_pad, gram, acc.F_pad);
+                            acc.F_pad, gram, acc.F_pad, ws.part.ptr);
         } else {
             ws.qbuf.alloc(gram_quant_bytes((int)sb.rows_q, (int)sb.h0, ld));
             {
