@@ -196,7 +196,7 @@ int plm_api_sum_of_prod(plm_model* mp, int type, const double* anlm_re, const do
         pe.alloc((size_t)ps * 2 * elem);
         pf.alloc((size_t)ps * 2 * elem);
         launch_prodsum(st, fp64, m.md, m.ed, one.bd, one.a.ptr, m.max_nlm, pe.ptr, pf.ptr, ps,
-                       m.max_lin, 0);
+                       nullptr, m.max_lin, 0);
         check_hip(hipGetLastError(), "prodsum launch");
         // the sums are stored by head position; returned in the potential's order
         const int nh = m.ed.t[type].n_heads;

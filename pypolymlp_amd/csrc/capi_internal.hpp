@@ -127,7 +127,7 @@ struct ModelHandle {
     std::map<std::tuple<int, int, int>, GroupChoice> group_tuning;
     // work buffers of eager evaluations (order parameters, head sums, results),
     // kept and grown across calls; eval_mutex serialises the calls that use them
-    DevBuf ev_a, ev_pse, ev_psf, ev_out;
+    DevBuf ev_a, ev_eat, ev_psf, ev_part, ev_out;
     std::vector<double> ev_host;
     std::mutex eval_mutex;
 };
@@ -317,7 +317,7 @@ struct EvalGraph {
     bool fp64 = true;
     unsigned pot_version = 0;
     size_t n_out = 0;
-    DevBuf a_buf, pse, psf, out;
+    DevBuf a_buf, e_at, psf, part, out;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     EvalGraph() = default;
@@ -326,8 +326,8 @@ struct EvalGraph {
     ~EvalGraph();
 };
 void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, const int* hb_j,
-                      const double* hb_d, int n_half, bool fp64, void* a_buf, void* pse,
-                      void* psf, double* out, size_t n_out, hipStream_t st);
+                      const double* hb_d, int n_half, bool fp64, void* a_buf, double* e_at,
+                      void* psf, double* part, double* out, size_t n_out, hipStream_t st);
 void eval_graph_capture(EvalGraph& g);
 void eval_graph_run(EvalGraph& g, int steps, double* energies, double* forces, double* stresses);
 void eval_single(ModelHandle& m, const double* axis, const double* pos_c, const int* types, int n,

@@ -76,6 +76,11 @@ void upload_potential(ModelHandle& m) {
         if ((int)order[t].size() != n_heads)
             throw std::invalid_argument("evaluation heads do not match the potential");
     }
+    // the first head position of each type pair
+    std::vector<std::vector<int>> tp_first(nt, std::vector<int>(ntp, 0));
+    for (int t = 0; t < nt; ++t)
+        for (int tp = 1; tp < ntp; ++tp)
+            tp_first[t][tp] = tp_first[t][tp - 1] + (int)by_tp_t[t][tp - 1].size();
     // the type of atom j for an atom of type t and a type pair
     auto partner = [&](int t, int tp) {
         int found = -1;
@@ -106,29 +111,38 @@ void upload_potential(ModelHandle& m) {
             }
             off[r + 1] = (int)ce.size();
         }
-        // per type pair its heads and the first head of every Y key; hi and hj
-        // are head positions of atoms i and j
+        // per type pair its heads; hi and hj are head positions of atoms i and j
         const int nkey = m.md.n_lmh;
-        std::vector<int> hoff(ntp + 1, 0), koff((size_t)ntp * (nkey + 1), 0), nid, ylm, hi, hj;
+        std::vector<int> hoff(ntp + 1, 0), nid, ylm, hi, hj;
         std::vector<float> sj;
         std::vector<unsigned char> m0;
         for (int tp = 0; tp < ntp; ++tp) {
             const auto& heads = by_tp_t[t][tp];
             const int t2 = heads.empty() ? -1 : partner(t, tp);
             if (!heads.empty() && t2 < 0) throw std::invalid_argument("type pair without partner type");
-            int* ko = koff.data() + (size_t)tp * (nkey + 1);
             for (const auto& e : heads) {
                 if (gt && (e[1] < 0 || e[1] >= nkey)) throw std::invalid_argument("head Y key range");
                 if (e[3] < 0 || e[3] >= (int)m.head_rank[t2].size())
                     throw std::invalid_argument("head of atom j out of range");
-                if (gt) ++ko[e[1] + 1];
                 nid.push_back(e[0]), ylm.push_back(e[1]);
                 hi.push_back(m.head_rank[t][e[2]]), hj.push_back(m.head_rank[t2][e[3]]);
                 sj.push_back((float)e[4]), m0.push_back((unsigned char)e[5]);
             }
-            ko[0] = hoff[tp];
-            for (int k = 0; k < nkey; ++k) ko[k + 1] += ko[k];
             hoff[tp + 1] = (int)nid.size();
+            // the layout the per-lane pair loop relies on
+            const int cnt = (int)M.tp_to_n()[tp].size(), n_tp_heads = hoff[tp + 1] - hoff[tp];
+            if (n_tp_heads != 0 && n_tp_heads != (gt ? nkey : 1) * cnt)
+                throw std::invalid_argument("evaluation heads of a type pair");
+            for (int h = hoff[tp]; h < hoff[tp + 1]; ++h)
+                if (hi[h] != h || hj[h] - hj[hoff[tp]] != h - hoff[tp] ||
+                    nid[h] != (h - hoff[tp]) % cnt || (gt && ylm[h] != (h - hoff[tp]) / cnt) ||
+                    hj[hoff[tp]] != tp_first[t2][tp])
+                    throw std::invalid_argument("evaluation head order");
+        }
+        std::vector<int> ha(std::max(1, E.n_heads), 0);
+        for (int r = 0; r < E.n_heads; ++r) {
+            const int k = order[t][r];
+            ha[r] = gt ? T.noconj[k] | (T.nlm[T.noconj[k]].m == 0 ? 1 << 30 : 0) : k;
         }
         auto upv = [&](const auto& v) {
             using V = typename std::decay_t<decltype(v)>::value_type;
@@ -163,7 +177,7 @@ void upload_potential(ModelHandle& m) {
                           hj[h] | (sj[h] < 0.f ? 1 << 28 : 0) | (m0[h] ? 1 << 29 : 0)};
         }
         E.hd_off = upv(hoff);
-        E.hd_koff = upv(koff);
+        E.hd_a = upv(ha);
         E.hd_rec = static_cast<const int4*>(upv(rec));
     }
     m.pot_uploaded = true;
@@ -172,11 +186,12 @@ void upload_potential(ModelHandle& m) {
 
 // Work buffers of one evaluation; out = [energies | forces (3 per atom) | stresses (6)].
 static void alloc_eval(const ModelHandle& m, const BatchHandle& b, bool fp64, DevBuf& a_buf,
-                       DevBuf& pse, DevBuf& psf, DevBuf& out, size_t& n_out) {
+                       DevBuf& e_at, DevBuf& psf, DevBuf& part, DevBuf& out, size_t& n_out) {
     const int elem = fp64 ? 8 : 4;
     const size_t A = b.n_atoms;
     a_buf.alloc(A * m.max_nlm * 2 * elem);
-    pse.alloc(A * std::max(1, m.max_heads) * 2 * elem);
+    e_at.alloc(A * 8);
+    part.alloc(pair_part_bytes(m.md, (int)b.n_half, m.host.input().gtinv ? 0 : 1));
     psf.alloc(A * std::max(1, m.max_heads) * 2 * elem);
     n_out = (size_t)b.n_st + 3 * A + 6 * (size_t)b.n_st;
     out.alloc(n_out * 8);
@@ -186,8 +201,8 @@ static void alloc_eval(const ModelHandle& m, const BatchHandle& b, bool fp64, De
 // node when captured), then filled by the half-pair loop. bd carries the full
 // neighbour list (order parameters); hb_* the half list (pair loop).
 void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, const int* hb_j,
-                      const double* hb_d, int n_half, bool fp64, void* a_buf, void* pse,
-                      void* psf, double* out, size_t n_out, hipStream_t st) {
+                      const double* hb_d, int n_half, bool fp64, void* a_buf, double* e_at,
+                      void* psf, double* part, double* out, size_t n_out, hipStream_t st) {
     const int A = bd.n_atoms_total;
     launch_fill_zero(st, out, n_out);
     double* d_e = out;
@@ -201,22 +216,24 @@ void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, con
     check_hip(hipGetLastError(), "eval anlm launch");
     {
         ProfScope ps("eval_prodsum", st);
-        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, pse, psf,
-                       std::max(1, m.max_heads), m.max_lin, pair_model);
+        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, nullptr, psf,
+                       std::max(1, m.max_heads), e_at, m.max_lin, pair_model);
     }
     check_hip(hipGetLastError(), "prodsum launch");
     {
         ProfScope ps("eval_pair", st);
-        launch_pair(st, fp64, m.md, m.ed, bd, bd.atom_st, hb_off, hb_j, hb_d, n_half, pse, psf,
-                    std::max(1, m.max_heads), d_e, d_f, d_s, pair_model);
+        BatchDev hb = bd;
+        hb.nb_off = hb_off, hb.nb_j = hb_j, hb.nb_d = hb_d;
+        launch_pair(st, fp64, m.md, m.ed, hb, bd.atom_st, n_half, e_at, psf,
+                    std::max(1, m.max_heads), part, d_e, d_f, d_s, pair_model);
     }
     check_hip(hipGetLastError(), "pair launch");
 }
 
-static void enqueue_eval(ModelHandle& m, BatchHandle& b, bool fp64, void* a_buf, void* pse,
-                         void* psf, double* out, size_t n_out, hipStream_t st) {
+static void enqueue_eval(ModelHandle& m, BatchHandle& b, bool fp64, void* a_buf, double* e_at,
+                         void* psf, double* part, double* out, size_t n_out, hipStream_t st) {
     enqueue_eval_dev(m, b.view(), b.d_hb_off(), (const int*)b.d_hb_j.ptr,
-                     (const double*)b.d_hb_d.ptr, (int)b.n_half, fp64, a_buf, pse, psf, out,
+                     (const double*)b.d_hb_d.ptr, (int)b.n_half, fp64, a_buf, e_at, psf, part, out,
                      n_out, st);
 }
 
@@ -244,8 +261,8 @@ void eval_batch(ModelHandle& m, BatchHandle& b, bool fp64, double* energies, dou
     hipStream_t st = device().stream;
     std::lock_guard<std::mutex> lock(m.eval_mutex);
     size_t n_out = 0;
-    alloc_eval(m, b, fp64, m.ev_a, m.ev_pse, m.ev_psf, m.ev_out, n_out);
-    enqueue_eval(m, b, fp64, m.ev_a.ptr, m.ev_pse.ptr, m.ev_psf.ptr, (double*)m.ev_out.ptr, n_out,
+    alloc_eval(m, b, fp64, m.ev_a, m.ev_eat, m.ev_psf, m.ev_part, m.ev_out, n_out);
+    enqueue_eval(m, b, fp64, m.ev_a.ptr, (double*)m.ev_eat.ptr, m.ev_psf.ptr, (double*)m.ev_part.ptr, (double*)m.ev_out.ptr, n_out,
                  st);
     copy_out(b, m.ev_out, n_out, st, m.ev_host, energies, forces, stresses);
 }
@@ -260,15 +277,15 @@ void eval_graph_capture(EvalGraph& g) {
     BatchHandle& b = *g.b;
     prepare_eval(m, b);
     hipStream_t st = device().stream;
-    alloc_eval(m, b, g.fp64, g.a_buf, g.pse, g.psf, g.out, g.n_out);
+    alloc_eval(m, b, g.fp64, g.a_buf, g.e_at, g.psf, g.part, g.out, g.n_out);
     // one eager pass first: kernel attributes are set and every buffer exists
-    enqueue_eval(m, b, g.fp64, g.a_buf.ptr, g.pse.ptr, g.psf.ptr, (double*)g.out.ptr, g.n_out, st);
+    enqueue_eval(m, b, g.fp64, g.a_buf.ptr, (double*)g.e_at.ptr, g.psf.ptr, (double*)g.part.ptr, (double*)g.out.ptr, g.n_out, st);
     check_hip(hipStreamSynchronize(st), "sync");
     {
         ProfPause pause;
         check_hip(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "begin capture");
         try {
-            enqueue_eval(m, b, g.fp64, g.a_buf.ptr, g.pse.ptr, g.psf.ptr, (double*)g.out.ptr,
+            enqueue_eval(m, b, g.fp64, g.a_buf.ptr, (double*)g.e_at.ptr, g.psf.ptr, (double*)g.part.ptr, (double*)g.out.ptr,
                          g.n_out, st);
         } catch (...) {
             hipGraph_t tmp = nullptr;

@@ -110,7 +110,7 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     {
         Arena probe = ar;
         probe.take((size_t)n * m.max_nlm * 2 * elem);
-        probe.take((size_t)n * heads * 2 * elem);
+        probe.take((size_t)n * 8);
         probe.take((size_t)n * heads * 2 * elem);
         probe.take(n_out * 8);
         probe.take((size_t)(n + 1) * 8);
@@ -145,10 +145,11 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     double* d_nb_d = (double*)ar.take(Mf * 24);
     int* d_hb_off = (int*)ar.take((size_t)(n + 1) * 4);
     int* d_hb_j = (int*)ar.take(Mh * 4);
-    int* d_hb_t = (int*)ar.take(Mh * 4);
     double* d_hb_d = (double*)ar.take(Mh * 24);
+    double* part = (double*)ar.take(
+        pair_part_bytes(m.md, off_h[n], m.host.input().gtinv ? 0 : 1));
     void* a_buf = ar.take((size_t)n * m.max_nlm * 2 * elem);
-    void* pse = ar.take((size_t)n * heads * 2 * elem);
+    double* e_at = (double*)ar.take((size_t)n * 8);
     void* psf = ar.take((size_t)n * heads * 2 * elem);
     double* out = (double*)ar.take(n_out * 8);
 
@@ -157,7 +158,7 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     launch_list_fill(st, n, n, n_tr, d_atom_st, d_atom_off, d_pos, d_tr_off, d_trans, cut2, tol2,
                      d_nb_off, d_nb_j, d_nb_t, d_nb_d);
     check_hip(hipGetLastError(), "neighbor launch");
-    launch_half_list(st, n, tol, d_nb_off, d_nb_j, d_nb_t, d_nb_d, d_hb_off, d_hb_j, d_hb_t,
+    launch_half_list(st, n, tol, d_nb_off, d_nb_j, d_nb_t, d_nb_d, d_hb_off, d_hb_j, nullptr,
                      d_hb_d);
     check_hip(hipGetLastError(), "half list launch");
 
@@ -172,8 +173,8 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     bd.nb_off = d_nb_off;
     bd.nb_j = d_nb_j;
     bd.nb_d = d_nb_d;
-    enqueue_eval_dev(m, bd, d_hb_off, d_hb_j, d_hb_d, off_h[n], fp64, a_buf, pse, psf, out, n_out,
-                     st);
+    enqueue_eval_dev(m, bd, d_hb_off, d_hb_j, d_hb_d, off_h[n], fp64, a_buf, e_at, psf, part, out,
+                     n_out, st);
     std::vector<double> h(n_out);
     check_hip(hipMemcpyAsync(h.data(), out, n_out * 8, hipMemcpyDeviceToHost, st), "copy");
     check_hip(hipStreamSynchronize(st), "sync");

@@ -20,9 +20,11 @@ struct EvalTypeDev {
     const double2* pq_c;
     // half-pair contraction: heads of this type grouped by type pair
     const int* hd_off;      // [n_tp+1]
-    // gtinv: the heads of each type pair are ordered by Y key; hd_koff[tp (n_lmh + 1) + k]
-    // is the first head of key k of type pair tp
-    const int* hd_koff;
+    // gtinv: the heads of each type pair are ordered by Y key, then by radial
+    // function (head hd_off[tp] + key * rad_count[tp] + n_id), in both atoms' head sums
+    // per head, its order parameter (index into the atom's full list) with bit
+    // 30 set where m == 0 (weight 1/2 in the energy)
+    const int* hd_a;
     // per head, one 16-byte record: (radial n_id, ylm key, ilocal_noconj of the
     // head (atom i), jlocal_noconj (the same component seen from atom j) with
     // bit 28 set where (-1)^l = -1 and bit 29 where m == 0 (weight 1/2))

@@ -42,7 +42,7 @@ void launch_bin_fill(hipStream_t st, int n, int max_pairs_atom, const double* po
                      const int* start, const void* sorted, const BinGridHost& g,
                      const double* trans, double cut2, double tol2, double tol, const int* nb_off,
                      int* nb_j, int* nb_t, double* nb_d, void* keys);
-// the half list from the full one
+// the half list from the full one (hb_t may be null)
 void launch_half_list(hipStream_t st, int n, double tol, const int* nb_off, const int* nb_j,
                       const int* nb_t, const double* nb_d, const int* hb_off, int* hb_j, int* hb_t,
                       double* hb_d);
@@ -140,16 +140,21 @@ void launch_xrows(hipStream_t st, bool fp64, const ModelDev& md, const ColumnsDe
                   const PairRec& R, void* X, const double* roww, double* xe_sum, double* xe_sq);
 
 struct EvalDev;
+// prod_sum_f per atom and head into ps_f, and either prod_sum_e into ps_e or,
+// with ps_e null, the atoms' energies into e_at
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
                     const BatchDev& bd, const void* a_full, int a_stride, void* ps_e, void* ps_f,
-                    int ps_stride, int max_lin, int pair_model);
+                    int ps_stride, double* e_at, int max_lin, int pair_model);
 // x[0, n) = 0 by a kernel (a graph of it replays correctly; a memset node is avoided)
 void launch_fill_zero(hipStream_t st, double* x, size_t n);
-// half-pair loop over the n_half pairs of the half list (hb_off[n_atoms] = n_half)
+// half-pair loop over the n_half pairs of the half list, which bd carries as its
+// nb_off, nb_j and nb_d; the atoms' energies e_at added up per structure. part:
+// pair_part_bytes of scratch
+size_t pair_part_bytes(const ModelDev& md, int n_half, int pair_model);
 void launch_pair(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
-                 const BatchDev& bd, const int* atom_st, const int* hb_off, const int* hb_j,
-                 const double* hb_d, int n_half, const void* ps_e, const void* ps_f, int ps_stride,
-                 double* energy, double* forces, double* stress, int pair_model);
+                 const BatchDev& bd, const int* atom_st, int n_half, const double* e_at,
+                 const void* ps_f, int ps_stride, double* part, double* energy, double* forces,
+                 double* stress, int pair_model);
 
 // X^T X with the weighted targets in column F of X (ld >= F + 1, multiple of
 // 128; rows_pad multiple of 64). Mixed: quantise X into the int8 slice buffer

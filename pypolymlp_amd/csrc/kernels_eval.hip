@@ -35,13 +35,20 @@ void check_hip(hipError_t e, const char* what);
 // coefficient pair per term, one coalesced load per wave and iteration. A
 // lane writes the heads that begin and end in its chunk; the heads that cross
 // a chunk boundary are summed from the lanes' boundary slots in LDS.
+//
+// The pair loop needs prod_sum_f only. The energy is a sum over pairs of
+// f_n Re(Y (prod_sum_e(i) + (-1)^l prod_sum_e(j))), and the sum of f_n Y over an
+// atom's neighbours is its order parameter, so it is formed here per atom,
+//   e_i = sum_h w_h Re(a_h prod_sum_e[h])  (w_h = 1/2 where m = 0),
+// and no prod_sum_e is stored, which halves what the pair loop reads. HEADS_E:
+// prod_sum_e is written as well and the energy is not (plm_api_sum_of_prod).
 // ---------------------------------------------------------------------------
-template <class T, int NL>
+template <class T, int NL, bool HEADS_E>
 __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, BatchDev bd,
                                                      const Cpx<T>* __restrict__ a_full,
                                                      int a_stride, Cpx<T>* __restrict__ ps_e,
                                                      Cpx<T>* __restrict__ ps_f, int ps_stride,
-                                                     int pair_model) {
+                                                     double* __restrict__ e_at, int pair_model) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     // two slots per lane of head sums (4 values each) and their heads, the
     // atom's order parameters (a_stride complex values), then its features
@@ -71,7 +78,7 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
     }
     __syncthreads();
     const int lane = threadIdx.x;
-    Cpx<T>* oe = ps_e + (size_t)i * ps_stride;
+    Cpx<T>* oe = HEADS_E ? ps_e + (size_t)i * ps_stride : nullptr;
     Cpx<T>* of = ps_f + (size_t)i * ps_stride;
     const double scale = pair_model ? 0.5 : 1.0;
     // a head that begins and ends inside the lane's chunk is written at once;
@@ -79,25 +86,40 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
     // chunks) go to the lane's two slots, summed over lanes afterwards
     int cur = -1, first = -1;
     T er = T(0), ei = T(0), fr = T(0), fi = T(0);
+    double e_sum = 0.0;
+    auto add_energy = [&] {
+        if constexpr (!HEADS_E) {
+            const int ha = E.hd_a[cur];  // its order parameter, bit 30: m = 0
+            const Cpx<T> ac = a[ha & 0x3fffffff];
+            const double v = double(er) * double(ac.re) - double(ei) * double(ac.im);
+            e_sum += (ha >> 30) & 1 ? 0.5 * v : v;
+        }
+    };
     auto to_slot = [&](int sl) {
         sh[sl] = cur;
-        sv[4 * sl] = double(er), sv[4 * sl + 1] = double(ei);
+        if constexpr (HEADS_E) sv[4 * sl] = double(er), sv[4 * sl + 1] = double(ei);
         sv[4 * sl + 2] = double(fr), sv[4 * sl + 3] = double(fi);
     };
     sh[2 * lane] = sh[2 * lane + 1] = -1;
     for (int h = lane; h < E.n_heads; h += blockDim.x)
-        if (E.pot_off[h + 1] == E.pot_off[h]) oe[h] = {T(0), T(0)}, of[h] = {T(0), T(0)};
+        if (E.pot_off[h + 1] == E.pot_off[h]) {
+            if constexpr (HEADS_E) oe[h] = {T(0), T(0)};
+            of[h] = {T(0), T(0)};
+        }
     for (int it = 0; it < E.pq_iters; ++it) {
         const int4 k = E.pq_key[(size_t)it * NL + lane];
         const double2 c = E.pq_c[(size_t)it * NL + lane];
         const int head = (unsigned)k.y >> 16;
         if (head == 0xffff) break;  // the rest of this lane's chunk is padding
         if (head != cur) {
-            if (cur == first && cur >= 0) {
-                to_slot(2 * lane);
-            } else if (cur >= 0) {
-                oe[cur] = {T(scale * er), T(scale * ei)};
-                of[cur] = {T(scale * fr), T(scale * fi)};
+            if (cur >= 0) {
+                add_energy();
+                if (cur == first) {
+                    to_slot(2 * lane);
+                } else {
+                    if constexpr (HEADS_E) oe[cur] = {T(scale * er), T(scale * ei)};
+                    of[cur] = {T(scale * fr), T(scale * fi)};
+                }
             }
             if (first < 0) first = head;
             cur = head, er = ei = fr = fi = T(0);
@@ -119,7 +141,10 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
         er += pr.re * se, ei += pr.im * se;
         fr += pr.re * sf, fi += pr.im * sf;
     }
-    if (cur >= 0) to_slot(cur == first ? 2 * lane : 2 * lane + 1);
+    if (cur >= 0) {
+        add_energy();
+        to_slot(cur == first ? 2 * lane : 2 * lane + 1);
+    }
     __syncthreads();
     // slots in term order, empty ones skipped: the first slot of each head sums
     // the slots of that head and writes it
@@ -132,10 +157,21 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
         double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
         for (int q = sl; q < NS && (sh[q] == h || sh[q] < 0); ++q) {
             if (sh[q] < 0) continue;
-            s0 += sv[4 * q], s1 += sv[4 * q + 1], s2 += sv[4 * q + 2], s3 += sv[4 * q + 3];
+            if constexpr (HEADS_E) s0 += sv[4 * q], s1 += sv[4 * q + 1];
+            s2 += sv[4 * q + 2], s3 += sv[4 * q + 3];
         }
-        oe[h] = {T(scale * s0), T(scale * s1)};
+        if constexpr (HEADS_E) oe[h] = {T(scale * s0), T(scale * s1)};
         of[h] = {T(scale * s2), T(scale * s3)};
+    }
+    if constexpr (!HEADS_E) {
+        for (int off = 32; off > 0; off >>= 1) e_sum += __shfl_down(e_sum, off);
+        __syncthreads();  // the slots are read
+        if ((lane & 63) == 0) sv[lane >> 6] = e_sum;
+        __syncthreads();
+        if (lane == 0) {
+            for (int w = 1; w < NL / 64; ++w) e_sum += sv[w];
+            e_at[i] = scale * e_sum;
+        }
     }
 }
 
@@ -156,9 +192,7 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
                                                   const int* __restrict__ hb_off,
                                                   const int* __restrict__ hb_j,
                                                   const double* __restrict__ hb_d,
-                                                  const Cpx<T>* __restrict__ ps_e,
                                                   const Cpx<T>* __restrict__ ps_f, int ps_stride,
-                                                  double* __restrict__ energy,
                                                   double* __restrict__ forces,
                                                   double* __restrict__ stress, int pair_model) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -174,9 +208,8 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
     hb.nb_j = hb_j;
     hb.nb_d = hb_d;
     const int lane = threadIdx.x, pl = lane >> 3, sl = lane & 7;
-    const Cpx<T>* Pi_e = ps_e + (size_t)i * ps_stride;
     const Cpx<T>* Pi_f = ps_f + (size_t)i * ps_stride;
-    double e_acc = 0.0, fi_acc[3] = {0, 0, 0}, s_acc[6] = {0, 0, 0, 0, 0, 0};
+    double fi_acc[3] = {0, 0, 0}, s_acc[6] = {0, 0, 0, 0, 0, 0};
     for (int c0 = p0; c0 < p1; c0 += kEvPairs) {
         const int np = min(kEvPairs, p1 - c0);
         __syncthreads();  // the previous chunk's records are read
@@ -185,22 +218,20 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
         T* slot = pairs + (size_t)min(pl, np - 1) * L.stride;
         const T* ms = L.misc(slot);
         const bool live = pl < np && ms[4] != T(0);
-        // pair model: ea = energy sum, fxa = radial-derivative sum
-        T ea = T(0), fxa = T(0), fya = T(0), fza = T(0);
+        // pair model: fxa = radial-derivative sum
+        T fxa = T(0), fya = T(0), fza = T(0);
         int j = 0;
         if (live) {
             const int tp = int(ms[5]);
             j = hb_j[k];
             const T* fn = L.fn(slot);
             const T* fd = L.fd(slot);
-            const Cpx<T>* Pj_e = ps_e + (size_t)j * ps_stride;
             const Cpx<T>* Pj_f = ps_f + (size_t)j * ps_stride;
             const int h0 = E.hd_off[tp], h1 = E.hd_off[tp + 1];
             if (pair_model) {
                 for (int h = h0 + sl; h < h1; h += 8) {
                     const int4 hr = E.hd_rec[h];
                     const int nid = hr.x, hi = hr.z, hj = hr.w & 0x0fffffff;
-                    ea += fn[nid] * (Pi_e[hi].re + Pj_e[hj].re);
                     fxa += fd[nid] * (Pi_f[hi].re + Pj_f[hj].re);
                 }
             } else {
@@ -217,12 +248,9 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
                     const int hi = hr.z, hj = hr.w & 0x0fffffff;
                     const T sj = (hr.w >> 28) & 1 ? T(-1) : T(1);
                     const T w = (hr.w >> 29) & 1 ? T(0.5) : T(1);
-                    const Cpx<T> se = {(Pi_e[hi].re + Pj_e[hj].re * sj) * w,
-                                       (Pi_e[hi].im + Pj_e[hj].im * sj) * w};
                     const Cpx<T> sf = {(Pi_f[hi].re + Pj_f[hj].re * sj) * w,
                                        (Pi_f[hi].im + Pj_f[hj].im * sj) * w};
                     const Cpx<T> y = Y[key];
-                    ea += fv * (y.re * se.re - y.im * se.im);
                     const T d1r = fd[nid] * y.re * ir, d1i = fd[nid] * y.im * ir;
                     // val_a = -(d1 * d_a + fn * dY_a)
                     const Cpx<T> vx = {-(d1r * dx + fv * dY[3 * key].re), -(d1i * dx + fv * dY[3 * key].im)};
@@ -237,7 +265,6 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
         // the pair's sums over its 8 lanes
 #pragma unroll
         for (int off = 1; off < 8; off <<= 1) {
-            ea += __shfl_xor(ea, off);
             fxa += __shfl_xor(fxa, off);
             fya += __shfl_xor(fya, off);
             fza += __shfl_xor(fza, off);
@@ -246,7 +273,6 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
             // diff_ij: r_i - r_j - T, in FP64 for the forces' directions and the stress
             const double dx = -hb_d[3 * (size_t)k], dy = -hb_d[3 * (size_t)k + 1],
                          dz = -hb_d[3 * (size_t)k + 2];
-            const double eij = double(ea);
             double fx, fy, fz;
             if (pair_model) {
                 const double fij = -double(fxa) / sqrt(dx * dx + dy * dy + dz * dz);
@@ -254,7 +280,6 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
             } else {
                 fx = double(fxa), fy = double(fya), fz = double(fza);
             }
-            e_acc += eij;
             fi_acc[0] += fx, fi_acc[1] += fy, fi_acc[2] += fz;
             atomicAdd(forces + 3 * (size_t)j, -fx);
             atomicAdd(forces + 3 * (size_t)j + 1, -fy);
@@ -265,13 +290,11 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
     }
     // wave reduction (64 lanes)
     for (int off = 32; off > 0; off >>= 1) {
-        e_acc += __shfl_down(e_acc, off);
         for (int a = 0; a < 3; ++a) fi_acc[a] += __shfl_down(fi_acc[a], off);
         for (int a = 0; a < 6; ++a) s_acc[a] += __shfl_down(s_acc[a], off);
     }
     if (lane == 0) {
         const int s = atom_st[i];
-        atomicAdd(energy + s, e_acc);
         for (int a = 0; a < 3; ++a) atomicAdd(forces + 3 * (size_t)i + a, fi_acc[a]);
         for (int a = 0; a < 6; ++a) atomicAdd(stress + 6 * (size_t)s + a, s_acc[a]);
     }
@@ -279,63 +302,104 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
 
 // ---------------------------------------------------------------------------
 // Half-pair loop, per-lane form: one lane per half pair (i, j) of the whole
-// list, the radial functions in registers (NB bounds their number) and Y_lm
-// with its gradient generated column by column (LB bounds max l), each key
-// used at once on its heads (the heads of a type pair are ordered by key). A
-// lane finds its atom i from the half-list offsets; the forces on i and j go
-// out as atomics per lane, the energy and stress with one atomic per wave
-// when the wave's pairs belong to one structure.
+// list (bd carries the half list), Y_lm with its gradient generated column by
+// column (LB bounds max l), each key used at once on its heads. The heads of a
+// type pair are laid out by key, then by radial function, in the head sums of
+// both atoms, so the heads of a key are two runs of cnt values, S_n = P_i[n] +
+// (-1)^l P_j[n], and the force needs only A = sum_n f'_n S_n and B = sum_n f_n S_n:
+//   f = -w (Re(Y A) d / r + Re(dY B)),  w = 1/2 where m = 0.
+// f_n and f'_n sit in LDS, a column per lane (an array in registers, indexed
+// by n, cost 48 KB of scratch a wave or a wave per SIMD). The forces on j go
+// out as atomics per lane, those on i per run of lanes with the same i. A wave
+// whose pairs belong to one structure writes its part of the stress to
+// part[wave] (eval_sum_kernel adds the waves up): as atomics on the structure's
+// six values the waves' sums took 13 ns each, one after the other, which was
+// the kernel's whole time on one large cell (FP64, 32,000 atoms: 1.97 -> 0.40 ms;
+// 160 alloys of 128 atoms, FP32: 5.4 -> 1.5 ms). blockIdx.y: the keys of m = y, y +
+// gridDim.y, .. only (few pairs: more waves, each with part of the keys).
 // ---------------------------------------------------------------------------
-template <class T, int LB, int NB>
-__global__ void __launch_bounds__(256) pair_lane_kernel(ModelDev md, EvalDev ed, BatchDev bd,
+template <class T, int LB>
+__global__ void __launch_bounds__(64) pair_lane_kernel(ModelDev md, EvalDev ed, BatchDev bd,
                                                    const int* __restrict__ atom_st,
-                                                   const int* __restrict__ hb_off,
-                                                   const int* __restrict__ hb_j,
-                                                   const double* __restrict__ hb_d, int n_half,
-                                                   const Cpx<T>* __restrict__ ps_e,
+                                                   int n_pairs,
                                                    const Cpx<T>* __restrict__ ps_f, int ps_stride,
-                                                   double* __restrict__ energy,
                                                    double* __restrict__ forces,
-                                                   double* __restrict__ stress, int pair_model) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    double eij = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+                                                   double* __restrict__ stress,
+                                                   double* __restrict__ part, int pair_model) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    using V2 = typename Vec2Of<T>::type;
+    V2* rad = reinterpret_cast<V2*>(smem_raw);  // [n][lane]: f_n, f'_n
+    const int lane = threadIdx.x;
+    const int k = blockIdx.x * 64 + lane;
+    double fx = 0.0, fy = 0.0, fz = 0.0;
     double dx = 0.0, dy = 0.0, dz = 0.0;
-    int st = -1;
-    if (k < n_half) {
-        // atom i of pair k: hb_off[i] <= k < hb_off[i + 1]
+    int st = -1, i = -1, j = -1;
+    if (k < n_pairs) {
+        // atom i of pair k: nb_off[i] <= k < nb_off[i + 1]
         int lo = 0, hi = bd.n_atoms_total;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
-            if (hb_off[mid] <= k) lo = mid;
+            if (bd.nb_off[mid] <= k) lo = mid;
             else hi = mid;
         }
-        const int i = lo;
+        i = lo;
         st = atom_st[i];
         const int t1 = bd.types[i];
-        const EvalTypeDev& E = ed.t[t1];
-        const Cpx<T>* Pi_e = ps_e + (size_t)i * ps_stride;
-        const Cpx<T>* Pi_f = ps_f + (size_t)i * ps_stride;
-        const int j = hb_j[k];
+        const int jj = bd.nb_j[k];
+        const int t2 = bd.types[jj];
         // diff_ij: r_i - r_j - T
-        dx = -hb_d[3 * (size_t)k], dy = -hb_d[3 * (size_t)k + 1], dz = -hb_d[3 * (size_t)k + 2];
+        dx = -bd.nb_d[3 * (size_t)k], dy = -bd.nb_d[3 * (size_t)k + 1], dz = -bd.nb_d[3 * (size_t)k + 2];
         const double dis = sqrt(dx * dx + dy * dy + dz * dz);
         if (dis < md.cutoff) {
-            const int tp = md.tp_of[t1 * md.n_type + bd.types[j]];
-            T fn[NB], fd[NB];
-            radial<T>(T(dis), T(md.cutoff), md.rad + (size_t)tp * md.n_fn * 2, md.rad_count[tp], fn, fd);
-            const Cpx<T>* Pj_e = ps_e + (size_t)j * ps_stride;
-            const Cpx<T>* Pj_f = ps_f + (size_t)j * ps_stride;
-            const int h0 = E.hd_off[tp], h1 = E.hd_off[tp + 1];
-            if (pair_model) {
-                T ef = T(0), ff = T(0);
-                for (int h = h0; h < h1; ++h) {
-                    const int4 hr = E.hd_rec[h];
-                    const int nid = hr.x, hi = hr.z, hj = hr.w & 0x0fffffff;
-                    ef += fn[nid] * (Pi_e[hi].re + Pj_e[hj].re);
-                    ff += fd[nid] * (Pi_f[hi].re + Pj_f[hj].re);
+            j = jj;
+            const int tp = md.tp_of[t1 * md.n_type + t2];
+            const int cnt = md.rad_count[tp];
+            // terms of f_n < 1e-20 are dropped (polymlp_eval.cpp:235)
+            {
+                const double* par = md.rad + (size_t)tp * md.n_fn * 2;
+                const T r = T(dis), kc = MathConst<T>::pi / T(md.cutoff);
+                T s, c;
+                dsincos(kc * r, &s, &c);
+                const T fc = T(0.5) * (c + T(1)), fcd = T(-0.5) * kc * s;
+                for (int n = 0; n < (cnt + 3) / 4 * 4; ++n) {
+                    const int nn = min(n, cnt - 1);
+                    const T beta = T(par[2 * nn]), mu = T(par[2 * nn + 1]);
+                    const T q = r - mu;
+                    const T g = dexp(-beta * q * q);
+                    const T gd = T(-2) * beta * q * g;
+                    const T fv = g * fc;
+                    const bool on = n < cnt && (pair_model || !(fv < T(1e-20)));
+                    V2 v;
+                    v.x = on ? fv : T(0), v.y = on ? gd * fc + g * fcd : T(0);
+                    rad[64 * n + lane] = v;
                 }
-                eij = double(ef);
-                const double fij = -double(ff) / dis;
+            }
+            const V2* Pi = reinterpret_cast<const V2*>(ps_f + (size_t)i * ps_stride) + ed.t[t1].hd_off[tp];
+            const V2* Pj = reinterpret_cast<const V2*>(ps_f + (size_t)j * ps_stride) + ed.t[t2].hd_off[tp];
+            // A and B of the heads of key (rows of four radial functions, whose
+            // last ones repeat the run's last value at zero weight)
+            auto run = [&](int key, T sj, Cpx<T>& A, Cpx<T>& B) {
+                const V2* pi = Pi + key * cnt;
+                const V2* pj = Pj + key * cnt;
+                A = {T(0), T(0)}, B = {T(0), T(0)};
+                for (int n = 0; n < cnt; n += 4) {
+                    V2 u[4], v[4], f[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) u[q] = pi[min(n + q, cnt - 1)], v[q] = pj[min(n + q, cnt - 1)];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) f[q] = rad[64 * (n + q) + lane];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const T sr = u[q].x + sj * v[q].x, si = u[q].y + sj * v[q].y;
+                        A.re += f[q].y * sr, A.im += f[q].y * si;
+                        B.re += f[q].x * sr, B.im += f[q].x * si;
+                    }
+                }
+            };
+            if (pair_model) {
+                Cpx<T> A, B;
+                run(0, T(1), A, B);
+                const double fij = -double(A.re) / dis;
                 fx = fij * dx, fy = fij * dy, fz = fij * dz;
             } else {
                 // Y_l^{-m} and its gradient generated column by column, m = max_l
@@ -365,31 +429,15 @@ __global__ void __launch_bounds__(256) pair_lane_kernel(ModelDev md, EvalDev ed,
                     }
                 }
                 const int lmax = md.max_l;
-                const int* ko = E.hd_koff + (size_t)tp * (md.n_lmh + 1);
-                T ea = T(0), fxa = T(0), fya = T(0), fza = T(0);
-                auto heads = [&](int key, Cpx<T> y, Cpx<T> gx, Cpx<T> gy, Cpx<T> gz) {
-                    for (int h = ko[key]; h < ko[key + 1]; ++h) {
-                        const int4 hr = E.hd_rec[h];
-                        const int nid = hr.x;
-                        const T fv = fn[nid];
-                        if (fv < T(1e-20)) continue;
-                        const int hi = hr.z, hj = hr.w & 0x0fffffff;
-                        const T sj = (hr.w >> 28) & 1 ? T(-1) : T(1);
-                        const T w = (hr.w >> 29) & 1 ? T(0.5) : T(1);
-                        const Cpx<T> se = {(Pi_e[hi].re + Pj_e[hj].re * sj) * w,
-                                           (Pi_e[hi].im + Pj_e[hj].im * sj) * w};
-                        const Cpx<T> sf = {(Pi_f[hi].re + Pj_f[hj].re * sj) * w,
-                                           (Pi_f[hi].im + Pj_f[hj].im * sj) * w};
-                        ea += fv * (y.re * se.re - y.im * se.im);
-                        const T d1r = fd[nid] * y.re * ir, d1i = fd[nid] * y.im * ir;
-                        // val_a = -(d1 * d_a + fn * dY_a)
-                        const Cpx<T> vx = {-(d1r * x + fv * gx.re), -(d1i * x + fv * gx.im)};
-                        const Cpx<T> vy = {-(d1r * yy + fv * gy.re), -(d1i * yy + fv * gy.im)};
-                        const Cpx<T> vz = {-(d1r * z + fv * gz.re), -(d1i * z + fv * gz.im)};
-                        fxa += re_mul(vx, sf);
-                        fya += re_mul(vy, sf);
-                        fza += re_mul(vz, sf);
-                    }
+                T fxa = T(0), fya = T(0), fza = T(0);
+                // l even or odd: the sign of the component seen from atom j
+                auto heads = [&](int key, bool odd, T w, Cpx<T> y, Cpx<T> gx, Cpx<T> gy, Cpx<T> gz) {
+                    Cpx<T> A, B;
+                    run(key, odd ? T(-1) : T(1), A, B);
+                    const T ra = re_mul(y, A) * ir;
+                    fxa -= w * (ra * x + re_mul(gx, B));
+                    fya -= w * (ra * yy + re_mul(gy, B));
+                    fza -= w * (ra * z + re_mul(gz, B));
                 };
                 T qn[LB + 1];  // Q(l, m + 1)
 #pragma unroll
@@ -434,11 +482,11 @@ __global__ void __launch_bounds__(256) pair_lane_kernel(ModelDev md, EvalDev ed,
                     }
 #pragma unroll
                     for (int l = m; l <= LB; ++l) {
-                        if (l > lmax) break;
+                        if (l > lmax || m % (int)gridDim.y != (int)blockIdx.y) break;
                         if (m == 0) {
                             const T common =
                                 (l >= 1) ? qn[l] * st * invr * dsqrt(T(0.5) * T(l) * T(l + 1)) : T(0);
-                            heads(lm2i(l, 0) + l, Cpx<T>{pc[l] * C::half_sqrt2, T(0)},
+                            heads(lm2i(l, 0) + l, l & 1, T(0.5), Cpx<T>{pc[l] * C::half_sqrt2, T(0)},
                                   Cpx<T>{common * ct * cp, T(0)}, Cpx<T>{common * ct * sp, T(0)},
                                   Cpx<T>{-common * st, T(0)});
                         } else {
@@ -452,7 +500,7 @@ __global__ void __launch_bounds__(256) pair_lane_kernel(ModelDev md, EvalDev ed,
                             const T ure = dth * ct * cp, uim = -dph * sp;
                             const T vre = dth * ct * sp, vim = dph * cp;
                             const T wre = -dth * st;
-                            heads(lm2i(l, -m) + l, Cpx<T>{tmp * c, -tmp * sv},
+                            heads(lm2i(l, -m) + l, l & 1, T(1), Cpx<T>{tmp * c, -tmp * sv},
                                   Cpx<T>{sign * (cre * ure - cim * uim), -sign * (cre * uim + cim * ure)},
                                   Cpx<T>{sign * (cre * vre - cim * vim), -sign * (cre * vim + cim * vre)},
                                   Cpx<T>{sign * (cre * wre), -sign * (cim * wre)});
@@ -461,140 +509,198 @@ __global__ void __launch_bounds__(256) pair_lane_kernel(ModelDev md, EvalDev ed,
 #pragma unroll
                     for (int l = 0; l <= LB; ++l) qn[l] = qc[l];
                 }
-                eij = double(ea), fx = double(fxa), fy = double(fya), fz = double(fza);
+                fx = double(fxa), fy = double(fya), fz = double(fza);
             }
-            atomicAdd(forces + 3 * (size_t)i, fx);
-            atomicAdd(forces + 3 * (size_t)i + 1, fy);
-            atomicAdd(forces + 3 * (size_t)i + 2, fz);
-            atomicAdd(forces + 3 * (size_t)j, -fx);
-            atomicAdd(forces + 3 * (size_t)j + 1, -fy);
-            atomicAdd(forces + 3 * (size_t)j + 2, -fz);
         }
     }
-    double sv[7] = {eij, dx * fx, dy * fy, dz * fz, dx * fy, dy * fz, dz * fx};
+    if (j >= 0) {
+        atomicAdd(forces + 3 * (size_t)j, -fx);
+        atomicAdd(forces + 3 * (size_t)j + 1, -fy);
+        atomicAdd(forces + 3 * (size_t)j + 2, -fz);
+    }
+    // the lanes of one i are neighbours: the first of them gets their sum
+    double si[3] = {fx, fy, fz};
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int io = __shfl_down(i, off);
+        const bool same = lane + off < 64 && io == i;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const double v = __shfl_down(si[a], off);
+            if (same) si[a] += v;
+        }
+    }
+    const int ip = __shfl_up(i, 1);
+    if (i >= 0 && (lane == 0 || ip != i))
+        for (int a = 0; a < 3; ++a) atomicAdd(forces + 3 * (size_t)i + a, si[a]);
+    double sv[6] = {dx * fx, dy * fy, dz * fz, dx * fy, dy * fz, dz * fx};
     const int s0 = __builtin_amdgcn_readfirstlane(st);
-    if (s0 < 0) return;  // lane 0 past the end: so is the whole wave
     if (__all(st == s0 || st < 0)) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
-            for (int a = 0; a < 7; ++a) sv[a] += __shfl_down(sv[a], off);
-        if ((threadIdx.x & 63) == 0) {
-            atomicAdd(energy + s0, sv[0]);
-            for (int a = 0; a < 6; ++a) atomicAdd(stress + 6 * (size_t)s0 + a, sv[1 + a]);
-        }
+            for (int a = 0; a < 6; ++a) sv[a] += __shfl_down(sv[a], off);
+        if (lane == 0)
+            for (int a = 0; a < 6; ++a)
+                part[6 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x) + a] = sv[a];
     } else if (st >= 0) {
-        atomicAdd(energy + st, sv[0]);
-        for (int a = 0; a < 6; ++a) atomicAdd(stress + 6 * (size_t)st + a, sv[1 + a]);
+        for (int a = 0; a < 6; ++a) atomicAdd(stress + 6 * (size_t)st + a, sv[a]);
     }
 }
 
-template <class T, int NL>
+// Per structure: its atoms' energies, and the stress parts of the pair loop's
+// waves that lie whole in its pairs (parts rows of n_waves; null: none).
+__global__ void __launch_bounds__(256) eval_sum_kernel(BatchDev bd, int n_pairs, int n_waves,
+                                                       int parts, const double* __restrict__ part,
+                                                       const double* __restrict__ e_at,
+                                                       double* __restrict__ energy,
+                                                       double* __restrict__ stress) {
+    __shared__ double sum[7][4];
+    const int s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int a0 = bd.st_atom_off[s], a1 = bd.st_atom_off[s + 1];
+    const int step = 256 * gridDim.y, first = 256 * blockIdx.y + threadIdx.x;
+    double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int i = a0 + first; i < a1; i += step) v[6] += e_at[i];
+    if (part) {
+        const int h0 = bd.nb_off[a0], h1 = bd.nb_off[a1];
+        const int w0 = (h0 + 63) / 64, w1 = h1 == n_pairs ? n_waves : h1 / 64;
+        for (int y = 0; y < parts; ++y) {
+            const double* p = part + 6 * (size_t)y * n_waves;
+#pragma unroll 2
+            for (int w = w0 + first; w < w1; w += step)
+#pragma unroll
+                for (int a = 0; a < 6; ++a) v[a] += p[6 * (size_t)w + a];
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 7; ++a) {
+        for (int off = 32; off > 0; off >>= 1) v[a] += __shfl_down(v[a], off);
+        if (lane == 0) sum[a][wave] = v[a];
+    }
+    __syncthreads();
+    if (threadIdx.x < 7) {
+        const int a = threadIdx.x;
+        const double t = (sum[a][0] + sum[a][1]) + (sum[a][2] + sum[a][3]);
+        double* o = a < 6 ? stress + 6 * (size_t)s + a : energy + s;
+        if (gridDim.y == 1) *o += t;
+        else atomicAdd(o, t);
+    }
+}
+
+template <class T, int NL, bool HEADS_E>
 void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
                       const void* a_full, int a_stride, void* ps_e, void* ps_f, int ps_stride,
-                      int max_lin, int pair_model) {
+                      double* e_at, int max_lin, int pair_model) {
     const size_t sm = 2 * NL * (4 * sizeof(double) + sizeof(int)) +
                       (size_t)a_stride * 2 * sizeof(T) + (size_t)std::max(1, max_lin) * sizeof(T);
     if (sm > 160 * 1024) throw std::invalid_argument("per-atom evaluation data exceed LDS");
-    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL>),
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL, HEADS_E>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
               "prodsum shared memory");
-    prodsum_kernel<T, NL><<<bd.n_atoms_total, NL, sm, st>>>(
+    prodsum_kernel<T, NL, HEADS_E><<<bd.n_atoms_total, NL, sm, st>>>(
         md, ed, bd, reinterpret_cast<const Cpx<T>*>(a_full), a_stride,
-        reinterpret_cast<Cpx<T>*>(ps_e), reinterpret_cast<Cpx<T>*>(ps_f), ps_stride, pair_model);
+        reinterpret_cast<Cpx<T>*>(ps_e), reinterpret_cast<Cpx<T>*>(ps_f), ps_stride, e_at,
+        pair_model);
 }
 
-template <class T>
+template <class T, bool HEADS_E>
 void launch_prodsum_lanes(hipStream_t st, const ModelDev& md, const EvalDev& ed,
                           const BatchDev& bd, const void* a_full, int a_stride, void* ps_e,
-                          void* ps_f, int ps_stride, int max_lin, int pair_model) {
+                          void* ps_f, int ps_stride, double* e_at, int max_lin, int pair_model) {
     // the term tables were laid out for ed.pq_lanes lanes
     if (ed.pq_lanes == 256)
-        launch_prodsum_t<T, 256>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride, max_lin,
-                                 pair_model);
+        launch_prodsum_t<T, 256, HEADS_E>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
+                                          e_at, max_lin, pair_model);
     else if (ed.pq_lanes == 64)
-        launch_prodsum_t<T, 64>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride, max_lin,
-                                pair_model);
+        launch_prodsum_t<T, 64, HEADS_E>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
+                                         e_at, max_lin, pair_model);
     else
         throw std::invalid_argument("contraction lanes must be 64 or 256");
 }
 
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
                     const BatchDev& bd, const void* a_full, int a_stride, void* ps_e, void* ps_f,
-                    int ps_stride, int max_lin, int pair_model) {
-    if (fp64)
-        launch_prodsum_lanes<double>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                     max_lin, pair_model);
+                    int ps_stride, double* e_at, int max_lin, int pair_model) {
+    if (fp64 && ps_e)
+        launch_prodsum_lanes<double, true>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
+                                           e_at, max_lin, pair_model);
+    else if (ps_e)
+        launch_prodsum_lanes<float, true>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
+                                          e_at, max_lin, pair_model);
+    else if (fp64)
+        launch_prodsum_lanes<double, false>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f,
+                                            ps_stride, e_at, max_lin, pair_model);
     else
-        launch_prodsum_lanes<float>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                    max_lin, pair_model);
+        launch_prodsum_lanes<float, false>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
+                                           e_at, max_lin, pair_model);
 }
 
 template <class T>
 void launch_pair_rec_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
-                   const int* atom_st, const int* hb_off, const int* hb_j, const double* hb_d,
-                   const void* ps_e, const void* ps_f, int ps_stride, double* energy,
-                   double* forces, double* stress, int pair_model) {
+                   const int* atom_st, const void* ps_f, int ps_stride, double* forces,
+                   double* stress, int pair_model) {
     const size_t sm = (size_t)kEvPairs * PairLayout<T>(md.n_fn, md.n_lmh).stride * sizeof(T);
     if (sm > 160 * 1024) throw std::invalid_argument("evaluation pair records exceed LDS");
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&pair_rec_kernel<T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
               "pair shared memory");
     pair_rec_kernel<T><<<bd.n_atoms_total, 64, sm, st>>>(
-        md, ed, bd, atom_st, hb_off, hb_j, hb_d, reinterpret_cast<const Cpx<T>*>(ps_e),
-        reinterpret_cast<const Cpx<T>*>(ps_f), ps_stride, energy, forces, stress, pair_model);
+        md, ed, bd, atom_st, bd.nb_off, bd.nb_j, bd.nb_d, reinterpret_cast<const Cpx<T>*>(ps_f),
+        ps_stride, forces, stress, pair_model);
 }
 
-template <class T, int LB, int NB>
+// Waves of the per-lane form and the parts its keys are split into: with fewer
+// waves than two a SIMD, the keys of a pair are dealt by m to several (54 atoms:
+// 21 waves; 138 us with all keys in one lane, 44 us so).
+static int pair_parts(const ModelDev& md, int waves, int pair_model) {
+    return pair_model ? 1 : std::max(1, std::min(md.max_l + 1, (2048 + waves - 1) / waves));
+}
+
+template <class T, int LB>
 void launch_pair_lb(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
-                    const int* atom_st, const int* hb_off, const int* hb_j, const double* hb_d,
-                    int n_half, const void* ps_e, const void* ps_f, int ps_stride, double* energy,
-                    double* forces, double* stress, int pair_model) {
-    if (n_half <= 0) return;
-    pair_lane_kernel<T, LB, NB><<<(n_half + 255) / 256, 256, 0, st>>>(
-        md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, reinterpret_cast<const Cpx<T>*>(ps_e),
-        reinterpret_cast<const Cpx<T>*>(ps_f), ps_stride, energy, forces, stress, pair_model);
+                    const int* atom_st, int n_half, const void* ps_f, int ps_stride,
+                    double* forces, double* stress, double* part, int pair_model) {
+    const int waves = (n_half + 63) / 64;
+    const size_t sm = (size_t)((md.n_fn + 3) / 4 * 4) * 64 * 2 * sizeof(T);
+    pair_lane_kernel<T, LB><<<dim3(waves, pair_parts(md, waves, pair_model)), 64, sm, st>>>(
+        md, ed, bd, atom_st, n_half, reinterpret_cast<const Cpx<T>*>(ps_f), ps_stride, forces,
+        stress, part, pair_model);
 }
 
 template <class T>
 void launch_pair_lane_t(hipStream_t st, const ModelDev& md, const EvalDev& ed,
-                        const BatchDev& bd, const int* atom_st, const int* hb_off,
-                        const int* hb_j, const double* hb_d, int n_half, const void* ps_e,
-                        const void* ps_f, int ps_stride, double* energy, double* forces,
-                        double* stress, int pair_model) {
+                        const BatchDev& bd, const int* atom_st, int n_half, const void* ps_f,
+                        int ps_stride, double* forces, double* stress, double* part,
+                        int pair_model) {
     const int L = md.max_l;
-    // radial arrays of 16 entries where the model has at most 16 radial
-    // functions and max_l <= 4: in FP64 they stay in registers (32 spill 528
-    // bytes per lane to scratch; 2.26 against 2.53 ms per 32,000 atoms), in
-    // FP32 the lower register count holds 4 waves per SIMD instead of 3 (1.60
-    // against 1.66 ms); at max_l 8 the 16-entry form's registers cost more than
-    // the spill (4.40 against 3.90 ms), so it keeps 32
-    if (L <= 4 && md.n_fn <= 16) {
-        launch_pair_lb<T, 4, 16>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f,
-                                 ps_stride, energy, forces, stress, pair_model);
-        return;
-    }
     if (md.n_fn > 32)
         throw std::invalid_argument("the per-lane pair loop supports at most 32 radial functions");
     if (L <= 4)
-        launch_pair_lb<T, 4, 32>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f, ps_stride,
-                                 energy, forces, stress, pair_model);
+        launch_pair_lb<T, 4>(st, md, ed, bd, atom_st, n_half, ps_f, ps_stride, forces, stress,
+                             part, pair_model);
     else if (L <= 8)
-        launch_pair_lb<T, 8, 32>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f, ps_stride,
-                                 energy, forces, stress, pair_model);
+        launch_pair_lb<T, 8>(st, md, ed, bd, atom_st, n_half, ps_f, ps_stride, forces, stress,
+                             part, pair_model);
     else if (L <= 12)
-        launch_pair_lb<T, 12, 32>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f, ps_stride,
-                                  energy, forces, stress, pair_model);
+        launch_pair_lb<T, 12>(st, md, ed, bd, atom_st, n_half, ps_f, ps_stride, forces, stress,
+                              part, pair_model);
     else
         throw std::invalid_argument("the per-lane pair loop supports max_l <= 12");
 }
 
+size_t pair_part_bytes(const ModelDev& md, int n_half, int pair_model) {
+    const int waves = (std::max(n_half, 1) + 63) / 64;
+    return (size_t)waves * pair_parts(md, waves, pair_model) * 48;
+}
+
 // The per-lane form where it applies (max_l <= 12, at most 32 radial
 // functions), the record form beyond; PLM_EVAL_PAIR=lane / records forces one.
+// e_at: the atoms' energies (launch_prodsum), added up per structure here.
 void launch_pair(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
-                 const BatchDev& bd, const int* atom_st, const int* hb_off, const int* hb_j,
-                 const double* hb_d, int n_half, const void* ps_e, const void* ps_f, int ps_stride,
-                 double* energy, double* forces, double* stress, int pair_model) {
+                 const BatchDev& bd, const int* atom_st, int n_half, const double* e_at,
+                 const void* ps_f, int ps_stride, double* part, double* energy, double* forces,
+                 double* stress, int pair_model) {
     if (n_half <= 0) return;
     bool lane = md.max_l <= 12 && md.n_fn <= 32;
     if (const char* e = getenv("PLM_EVAL_PAIR")) {
@@ -603,17 +709,23 @@ void launch_pair(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& e
         else throw std::invalid_argument("PLM_EVAL_PAIR: lane or records");
     }
     if (lane && fp64)
-        launch_pair_lane_t<double>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f,
-                                   ps_stride, energy, forces, stress, pair_model);
+        launch_pair_lane_t<double>(st, md, ed, bd, atom_st, n_half, ps_f, ps_stride, forces,
+                                   stress, part, pair_model);
     else if (lane)
-        launch_pair_lane_t<float>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, n_half, ps_e, ps_f,
-                                  ps_stride, energy, forces, stress, pair_model);
+        launch_pair_lane_t<float>(st, md, ed, bd, atom_st, n_half, ps_f, ps_stride, forces, stress,
+                                  part, pair_model);
     else if (fp64)
-        launch_pair_rec_t<double>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, ps_e, ps_f,
-                                  ps_stride, energy, forces, stress, pair_model);
+        launch_pair_rec_t<double>(st, md, ed, bd, atom_st, ps_f, ps_stride, forces, stress,
+                                  pair_model);
     else
-        launch_pair_rec_t<float>(st, md, ed, bd, atom_st, hb_off, hb_j, hb_d, ps_e, ps_f,
-                                 ps_stride, energy, forces, stress, pair_model);
+        launch_pair_rec_t<float>(st, md, ed, bd, atom_st, ps_f, ps_stride, forces, stress,
+                                 pair_model);
+    // a workgroup per structure, several for structures of more than 4,096 waves
+    const int waves = (n_half + 63) / 64, parts = pair_parts(md, waves, pair_model);
+    const int split = std::max(1, std::min(16, waves * parts / bd.n_st / 2048));
+    eval_sum_kernel<<<dim3(bd.n_st, split), 256, 0, st>>>(bd, n_half, waves, parts,
+                                                          lane ? part : nullptr, e_at, energy,
+                                                          stress);
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(double* __restrict__ x, size_t n) {

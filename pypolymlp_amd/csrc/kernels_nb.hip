@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(256) half_list_kernel(
         if (keep) {
             const int o = out + __popcll(vote & ((1ull << lane) - 1ull));
             hb_j[o] = j;
-            hb_t[o] = nb_t[p];
+            if (hb_t) hb_t[o] = nb_t[p];
             for (int a = 0; a < 3; ++a) hb_d[3 * (size_t)o + a] = d[a];
         }
         out += __popcll(vote);
