@@ -4,6 +4,7 @@
 #include <array>
 #include <cstdlib>
 #include <cstring>
+#include <numeric>
 #include <stdexcept>
 #include <vector>
 
@@ -19,22 +20,8 @@ void upload_potential(ModelHandle& m) {
     const int nt = M.n_type(), ntp = M.n_tp();
     const bool gt = M.input().gtinv;
     m.max_heads = 0, m.max_lin = 0;
-    // the contraction deals each atom's terms to one wave, or to four waves
-    // (sharing the atom's LDS data) when a wave would hold more than 128 terms
-    // per lane; PLM_PRODSUM_LANES=64|256 forces one
-    long max_terms = 0;
-    for (int t = 0; t < nt; ++t) {
-        long n = 0;
-        for (const auto& h : M.type(t).pot) n += (long)h.size();
-        max_terms = std::max(max_terms, n);
-    }
-    int lanes = max_terms > 128L * 64 ? 256 : 64;
-    if (const char* e = std::getenv("PLM_PRODSUM_LANES")) {
-        if (!std::strcmp(e, "64")) lanes = 64;
-        else if (!std::strcmp(e, "256")) lanes = 256;
-        else throw std::invalid_argument("PLM_PRODSUM_LANES must be 64 or 256");
-    }
-    m.ed.pq_lanes = lanes;
+    m.ed.value_max = std::max(1, m.v_maxf), m.ed.term_max = 1;
+    m.ed.poly_max = 0, m.ed.rows_max = 0;
     // The heads of each type in the order of the half-pair loop: grouped by type
     // pair, within one ordered by Y key (the per-lane pair loop generates Y_lm
     // key by key). The contraction writes head k of an atom at its position
@@ -59,7 +46,7 @@ void upload_potential(ModelHandle& m) {
             for (size_t k = 0; k < T.ntp.size(); ++k)
                 by_tp[T.ntp[k][2]].push_back({T.ntp[k][1], -1, (int)k, T.ntp[k][3], 1, 0});
         }
-        const int n_heads = (int)T.pot.size();
+        const int n_heads = (int)(gt ? T.noconj.size() : T.ntp.size());
         auto& rank = m.head_rank[t];
         rank.assign(n_heads, -1);
         for (int tp = 0; tp < ntp; ++tp) {
@@ -94,23 +81,9 @@ void upload_potential(ModelHandle& m) {
     for (int t = 0; t < nt; ++t) {
         const auto& T = M.type(t);
         EvalTypeDev& E = m.ed.t[t];
-        E.n_heads = (int)T.pot.size();
+        E.n_heads = (int)order[t].size();
         m.max_heads = std::max(m.max_heads, E.n_heads);
         m.max_lin = std::max(m.max_lin, (int)T.features.size());
-        // the terms by head position
-        std::vector<int> off(E.n_heads + 1, 0), pd, pf;
-        std::vector<double> ce, cf;
-        for (int r = 0; r < E.n_heads; ++r) {
-            for (const auto& pt : T.pot[order[t][r]]) {
-                const auto& k3 = T.prod_deriv[pt.prod];
-                const auto& k2 = T.prod_features[pt.prod_features];
-                if (k3.size() > 3 || k2.size() > 2) throw std::invalid_argument("term order too high");
-                for (int a = 0; a < 3; ++a) pd.push_back(a < (int)k3.size() ? k3[a] : -1);
-                for (int a = 0; a < 2; ++a) pf.push_back(a < (int)k2.size() ? k2[a] : -1);
-                ce.push_back(pt.coeff_e), cf.push_back(pt.coeff_f);
-            }
-            off[r + 1] = (int)ce.size();
-        }
         // per type pair its heads; hi and hj are head positions of atoms i and j
         const int nkey = m.md.n_lmh;
         std::vector<int> hoff(ntp + 1, 0), nid, ylm, hi, hj;
@@ -139,37 +112,194 @@ void upload_potential(ModelHandle& m) {
                     hj[hoff[tp]] != tp_first[t2][tp])
                     throw std::invalid_argument("evaluation head order");
         }
+        auto upv = [&](const auto& v) {
+            using V = typename std::decay_t<decltype(v)>::value_type;
+            return m.pot_store.upload(v.data(), v.size() * sizeof(V));
+        };
+        auto k16 = [](int v) -> unsigned {
+            if (v < 0 || v >= 0xffff) throw std::invalid_argument("evaluation table index exceeds 16 bits");
+            return (unsigned)v;
+        };
+        const std::vector<double>& coef = M.coeffs();
+        const int n_lin = (int)T.features.size();
+        const unsigned none = k16(m.md.t[t].n_nlm);
+        std::vector<double> lin(std::max(1, n_lin), 0.0);
+        std::vector<int> factor(std::max(1, n_lin), -1), pf_feat;
+        for (const auto& p : T.poly) {
+            if (p.local_ids.size() == 1) {
+                lin[p.local_ids[0]] += coef[p.global_id];
+                continue;
+            }
+            if (p.local_ids.size() > 3) throw std::invalid_argument("polynomial order above 3");
+            for (int f : p.local_ids)
+                if (factor[f] < 0) factor[f] = (int)pf_feat.size(), pf_feat.push_back(f);
+        }
+        E.n_poly = (int)pf_feat.size();
+        m.ed.poly_max = std::max(m.ed.poly_max, E.n_poly);
+        struct PolyRec {
+            unsigned rec;
+            double2 c;
+        };
+        auto order_of = [&](int f) { return (int)T.features[f][0].ids.size(); };
+        std::vector<std::vector<PolyRec>> by_factor(E.n_poly);
+        for (const auto& p : T.poly) {
+            const auto& id = p.local_ids;
+            if (id.size() == 1) continue;
+            int n_prods = 0;
+            for (int f : id) n_prods += order_of(f);
+            // each distinct factor once, with its power as a coefficient
+            for (size_t q = 0; q < id.size(); ++q) {
+                if (std::find(id.begin(), id.begin() + q, id[q]) != id.begin() + q) continue;
+                const int power = (int)std::count(id.begin(), id.end(), id[q]);
+                std::vector<int> o;
+                for (size_t r = 0; r < id.size(); ++r)
+                    if (r != q) o.push_back(factor[id[r]]);
+                const double c = power * coef[p.global_id];
+                by_factor[factor[id[q]]].push_back(
+                    {k16(o[0]) | k16(o.size() > 1 ? o[1] : E.n_poly) << 16, double2{c, c / n_prods}});
+            }
+        }
+        // pieces of at most `len` columns: the smallest that leaves 256 of them (a
+        // block for each of four waves), or whole multiples for more factors
+        size_t len = 8;
+        const size_t most = (size_t)std::max(1, (E.n_poly + 255) / 256) * 256;
+        for (;; ++len) {
+            size_t n = 0;
+            for (const auto& v : by_factor) n += (v.size() + len - 1) / len;
+            if (n <= most) break;
+        }
+        std::vector<std::pair<int, size_t>> pieces;  // factor, first column
+        std::vector<double2> pf_lin;
+        for (int q = 0; q < E.n_poly; ++q) {
+            for (size_t r = 0; r < by_factor[q].size(); r += len) pieces.push_back({q, r});
+            const int f = pf_feat[q];
+            pf_lin.push_back(double2{lin[f], lin[f] / order_of(f)});
+        }
+        E.pf_nblk = (int)(pieces.size() + 63) / 64;
+        std::vector<int> pf_piece((size_t)E.pf_nblk * 64, -1);
+        for (size_t p = 0; p < pieces.size(); ++p) pf_piece[p] = pieces[p].first;
+        std::vector<int> pf_boff(E.pf_nblk + 1, 0), pf_rec;
+        std::vector<double2> pf_c;
+        for (int bk = 0; bk < E.pf_nblk; ++bk) {
+            auto size_of = [&](size_t p) {
+                return std::min(len, by_factor[pieces[p].first].size() - pieces[p].second);
+            };
+            const size_t p1 = std::min(pieces.size(), (size_t)(bk + 1) * 64);
+            size_t rows = 0;
+            for (size_t p = (size_t)bk * 64; p < p1; ++p) rows = std::max(rows, size_of(p));
+            pf_boff[bk + 1] = pf_boff[bk] + (int)rows * 64;
+            pf_rec.resize(pf_boff[bk + 1], (int)(k16(E.n_poly) | k16(E.n_poly) << 16));
+            pf_c.resize(pf_boff[bk + 1], double2{0.0, 0.0});
+            for (size_t p = (size_t)bk * 64; p < p1; ++p)
+                for (size_t j = 0; j < size_of(p); ++j) {
+                    const PolyRec& v = by_factor[pieces[p].first][pieces[p].second + j];
+                    const size_t r = (size_t)pf_boff[bk] + j * 64 + (p - (size_t)bk * 64);
+                    pf_rec[r] = (int)v.rec, pf_c[r] = v.c;
+                }
+        }
+        // the factors' value terms
+        auto value_key = [&](int prod) {
+            const auto& k = T.prod[prod];
+            if (k.size() > 4) throw std::invalid_argument("invariant order above 4");
+            unsigned p[4] = {none, none, none, none};
+            for (size_t q = 0; q < k.size(); ++q) p[q] = k16(k[q]);
+            return int2{(int)(p[0] | p[1] << 16), (int)(p[2] | p[3] << 16)};
+        };
+        std::vector<int> vq(E.n_poly);
+        std::iota(vq.begin(), vq.end(), 0);
+        std::stable_sort(vq.begin(), vq.end(), [&](int x, int y) {
+            return T.feat_val[pf_feat[x]].size() > T.feat_val[pf_feat[y]].size();
+        });
+        E.vq_nblk = (E.n_poly + 63) / 64;
+        std::vector<int> vboff(E.vq_nblk + 1, 0), vitem((size_t)E.vq_nblk * 64, -1);
+        std::vector<int2> vkey;
+        std::vector<double> vc;
+        for (int bk = 0; bk < E.vq_nblk; ++bk) {
+            vboff[bk + 1] = vboff[bk] + (int)T.feat_val[pf_feat[vq[bk * 64]]].size() * 64;
+            vkey.resize(vboff[bk + 1], int2{(int)(none | none << 16), (int)(none | none << 16)});
+            vc.resize(vboff[bk + 1], 0.0);
+            for (int l = 0; l < 64 && bk * 64 + l < E.n_poly; ++l) {
+                const int q = vq[bk * 64 + l];
+                vitem[(size_t)bk * 64 + l] = q;
+                size_t r = (size_t)vboff[bk] + l;
+                for (const auto& pc : T.feat_val[pf_feat[q]])
+                    vkey[r] = value_key(pc.first), vc[r] = pc.second, r += 64;
+            }
+        }
+        // derivative terms by head position; terms of one product and factor are
+        // one (features outside the polynomial share the constant factor)
+        struct Term {
+            int prod, factor;
+            double c;
+        };
+        std::vector<std::vector<Term>> terms(E.n_heads);
+        for (int f = 0; f < n_lin; ++f)
+            for (const auto& d : T.feat_deriv[f]) {
+                if (gt && T.nlm[d.head].conj) continue;
+                const int k = gt ? T.local_to_noconj[d.head] : d.head;
+                const bool poly = factor[f] >= 0;
+                const int n_pd = (int)T.prod_deriv[d.prod].size();
+                if (n_pd > 3) throw std::invalid_argument("term order too high");
+                terms[m.head_rank[t][k]].push_back(
+                    {d.prod, poly ? factor[f] : E.n_poly + n_pd, poly ? d.coeff : d.coeff * lin[f]});
+            }
+        for (auto& v : terms) {
+            std::stable_sort(v.begin(), v.end(), [](const Term& x, const Term& y) {
+                return x.prod != y.prod ? x.prod < y.prod : x.factor < y.factor;
+            });
+            size_t n = 0;
+            for (size_t q = 0; q < v.size(); ++q)
+                if (n > 0 && v[n - 1].prod == v[q].prod && v[n - 1].factor == v[q].factor)
+                    v[n - 1].c += v[q].c;
+                else
+                    v[n++] = v[q];
+            v.resize(n);
+        }
+        std::vector<int> by_count(E.n_heads);
+        std::iota(by_count.begin(), by_count.end(), 0);
+        std::stable_sort(by_count.begin(), by_count.end(),
+                         [&](int x, int y) { return terms[x].size() > terms[y].size(); });
+        E.tq_nblk = (E.n_heads + 63) / 64;
+        const unsigned pad_y = none | k16(E.n_poly) << 16;
+        std::vector<int> boff(E.tq_nblk + 1, 0), item((size_t)E.tq_nblk * 64, -1);
+        std::vector<int2> key;
+        std::vector<double> tc;
+        for (int bk = 0; bk < E.tq_nblk; ++bk) {
+            const int rows = (int)terms[by_count[bk * 64]].size();
+            boff[bk + 1] = boff[bk] + rows * 64;
+            key.resize(boff[bk + 1], int2{(int)(none | none << 16), (int)pad_y});
+            tc.resize(boff[bk + 1], 0.0);
+            for (int l = 0; l < 64 && bk * 64 + l < E.n_heads; ++l) {
+                const int h = by_count[bk * 64 + l];
+                item[(size_t)bk * 64 + l] = h;
+                for (size_t j = 0; j < terms[h].size(); ++j) {
+                    const auto& pd = T.prod_deriv[terms[h][j].prod];
+                    m.ed.term_max = std::max(m.ed.term_max, (int)pd.size());
+                    unsigned p[3] = {none, none, none};
+                    for (size_t q = 0; q < pd.size(); ++q) p[q] = k16(pd[q]);
+                    const size_t r = (size_t)boff[bk] + j * 64 + l;
+                    key[r] = int2{(int)(p[0] | p[1] << 16), (int)(p[2] | k16(terms[h][j].factor) << 16)};
+                    tc[r] = terms[h][j].c;
+                }
+            }
+        }
+        m.ed.rows_max = std::max<int>(m.ed.rows_max, (boff[E.tq_nblk] + vboff[E.vq_nblk] +
+                                                      (int)pf_rec.size()) / 64);
+        const std::vector<float> tcf(tc.begin(), tc.end()), vcf(vc.begin(), vc.end());
+        std::vector<float2> pf_cf;
+        for (const double2& c : pf_c) pf_cf.push_back(float2{(float)c.x, (float)c.y});
         std::vector<int> ha(std::max(1, E.n_heads), 0);
         for (int r = 0; r < E.n_heads; ++r) {
             const int k = order[t][r];
             ha[r] = gt ? T.noconj[k] | (T.nlm[T.noconj[k]].m == 0 ? 1 << 30 : 0) : k;
         }
-        auto upv = [&](const auto& v) {
-            using V = typename std::decay_t<decltype(v)>::value_type;
-            return m.pot_store.upload(v.data(), v.size() * sizeof(V));
-        };
-        E.pot_off = upv(off);
-        // interleaved lane chunks of the contraction (keys and heads fit 16 bits:
-        // the order parameters and features they index are held in LDS)
-        const long n_terms = (long)ce.size();
-        const long iters = (n_terms + lanes - 1) / lanes;
-        std::vector<int4> pq_key((size_t)std::max(1L, iters) * lanes, int4{-1, -1, -1, 0});
-        std::vector<double2> pq_c(pq_key.size(), double2{0.0, 0.0});
-        auto k16 = [](int v) -> unsigned {
-            if (v >= 0xffff) throw std::invalid_argument("evaluation table index exceeds 16 bits");
-            return v < 0 ? 0xffffu : (unsigned)v;
-        };
-        for (int h = 0; h < E.n_heads; ++h)
-            for (int e = off[h]; e < off[h + 1]; ++e) {
-                const size_t r = (size_t)(e % iters) * lanes + e / iters;
-                pq_key[r] = int4{(int)(k16(pd[3 * e]) | k16(pd[3 * e + 1]) << 16),
-                                 (int)(k16(pd[3 * e + 2]) | k16(h) << 16),
-                                 (int)(k16(pf[2 * e]) | k16(pf[2 * e + 1]) << 16), 0};
-                pq_c[r] = double2{ce[e], cf[e]};
-            }
-        E.pq_iters = (int)iters;
-        E.pq_key = static_cast<const int4*>(upv(pq_key));
-        E.pq_c = static_cast<const double2*>(upv(pq_c));
+        E.hd_a = upv(ha);
+        E.vq_boff = upv(vboff), E.vq_item = upv(vitem), E.vq_key = upv(vkey);
+        E.vq_c = upv(vc), E.vq_cf = upv(vcf);
+        E.pf_boff = upv(pf_boff), E.pf_piece = upv(pf_piece), E.pf_rec = upv(pf_rec), E.pf_lin = upv(pf_lin);
+        E.pf_c = upv(pf_c), E.pf_cf = upv(pf_cf);
+        E.tq_boff = upv(boff), E.tq_item = upv(item), E.tq_key = upv(key);
+        E.tq_c = upv(tc), E.tq_cf = upv(tcf);
         std::vector<int4> rec(std::max<size_t>(1, nid.size()), int4{0, 0, 0, 0});
         for (size_t h = 0; h < nid.size(); ++h) {
             if (hj[h] < 0 || hj[h] >= (1 << 28)) throw std::invalid_argument("head index range");
@@ -177,7 +307,6 @@ void upload_potential(ModelHandle& m) {
                           hj[h] | (sj[h] < 0.f ? 1 << 28 : 0) | (m0[h] ? 1 << 29 : 0)};
         }
         E.hd_off = upv(hoff);
-        E.hd_a = upv(ha);
         E.hd_rec = static_cast<const int4*>(upv(rec));
     }
     m.pot_uploaded = true;
@@ -216,8 +345,8 @@ void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, con
     check_hip(hipGetLastError(), "eval anlm launch");
     {
         ProfScope ps("eval_prodsum", st);
-        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, nullptr, psf,
-                       std::max(1, m.max_heads), e_at, m.max_lin, pair_model);
+        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, psf,
+                       std::max(1, m.max_heads), e_at, pair_model);
     }
     check_hip(hipGetLastError(), "prodsum launch");
     {

@@ -140,11 +140,16 @@ void launch_xrows(hipStream_t st, bool fp64, const ModelDev& md, const ColumnsDe
                   const PairRec& R, void* X, const double* roww, double* xe_sum, double* xe_sq);
 
 struct EvalDev;
-// prod_sum_f per atom and head into ps_f, and either prod_sum_e into ps_e or,
-// with ps_e null, the atoms' energies into e_at
+// prod_sum_f per atom and head into ps_f, the atoms' energies into e_at
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
-                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_e, void* ps_f,
-                    int ps_stride, double* e_at, int max_lin, int pair_model);
+                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,
+                    int ps_stride, double* e_at, int pair_model);
+// prod_sum_e and prod_sum_f of one atom from the folded potential's terms of each
+// head (off [n_heads + 1]; keys (pd0 | pd1 << 16, pd2, pf0 | pf1 << 16, 0), 0xffff:
+// none; coefficients (e, f))
+void launch_head_terms(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd,
+                       const void* a, int n_heads, const int* off, const int4* key,
+                       const double2* coeff, int max_lin, void* ps_e, void* ps_f);
 // x[0, n) = 0 by a kernel (a graph of it replays correctly; a memset node is avoided)
 void launch_fill_zero(hipStream_t st, double* x, size_t n);
 // half-pair loop over the n_half pairs of the half list, which bd carries as its

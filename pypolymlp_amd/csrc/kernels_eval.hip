@@ -3,6 +3,7 @@
 // Reference loop nests:
 //   PolymlpEval::compute_sum_of_prod_anlmtp   src/cxx/src/compute/polymlp_eval.cpp:337-404
 //   Potential::compute_sum_of_prod_anlmtp     src/cxx/src/polymlp/polymlp_potential.cpp:235-321
+//                                             (here as a gradient by features, then by heads)
 //   PolymlpEval::eval_gtinv (half-pair loop)  polymlp_eval.cpp:182-291
 //   PolymlpEval::eval_pair / compute_sum_of_prod_antp  polymlp_eval.cpp:46-180,
 //                                             polymlp_potential.cpp:203-233
@@ -24,48 +25,181 @@ namespace plm {
 
 void check_hip(hipError_t e, const char* what);
 
+template <class T> struct EvalTab;  // the tables' coefficients by precision
+template <> struct EvalTab<double> {
+    __device__ static const double* value(const EvalTypeDev& e) { return e.vq_c; }
+    __device__ static const double2* poly(const EvalTypeDev& e) { return e.pf_c; }
+    __device__ static const double* term(const EvalTypeDev& e) { return e.tq_c; }
+};
+template <> struct EvalTab<float> {
+    __device__ static const float* value(const EvalTypeDev& e) { return e.vq_cf; }
+    __device__ static const float2* poly(const EvalTypeDev& e) { return e.pf_cf; }
+    __device__ static const float* term(const EvalTypeDev& e) { return e.tq_cf; }
+};
+
+// product of the order parameters of a value term (16-bit keys, absent ones
+// point at the constant 1)
+template <class T>
+__device__ __forceinline__ Cpx<T> value_prod(const Cpx<T>* a, int2 k, int n) {
+    Cpx<T> p = a[k.x & 0xffff];
+    if (n > 1) p = cmul(p, a[(unsigned)k.x >> 16]);
+    if (n > 2) p = cmul(p, a[k.y & 0xffff]);
+    if (n > 3) p = cmul(p, a[(unsigned)k.y >> 16]);
+    return p;
+}
+
 // ---------------------------------------------------------------------------
-// Per atom: features, products of features, and
-//   prod_sum_{e,f}[h] = sum_terms coeff_{e,f} * prod_features * prod_anlm
-// One workgroup of NL lanes (one wave, or four for models with many terms)
-// per atom; the atom's order parameters and features staged in LDS (the term
-// products gather from them at random keys). The terms of all heads are dealt
-// to the lanes in equal contiguous chunks (every lane does the same number of
-// terms, whatever the heads' lengths), read as one 16-byte key record and one
-// coefficient pair per term, one coalesced load per wave and iteration. A
-// lane writes the heads that begin and end in its chunk; the heads that cross
-// a chunk boundary are summed from the lanes' boundary slots in LDS.
-//
-// The pair loop needs prod_sum_f only. The energy is a sum over pairs of
-// f_n Re(Y (prod_sum_e(i) + (-1)^l prod_sum_e(j))), and the sum of f_n Y over an
-// atom's neighbours is its order parameter, so it is formed here per atom,
-//   e_i = sum_h w_h Re(a_h prod_sum_e[h])  (w_h = 1/2 where m = 0),
-// and no prod_sum_e is stored, which halves what the pair loop reads. HEADS_E:
-// prod_sum_e is written as well and the energy is not (plm_api_sum_of_prod).
+// Per atom: the derivatives of its energy E_i = sum_c c Pi x by the order parameters,
+//   prod_sum_f[h] = 2 sum_f (dE_i / dx_f) (dx_f / da_h),
+// and the energy from the same terms: with each column's coefficient divided by
+// the number n_c of its order parameters (prod_sum_e),
+//   E_i = sum_h w_h Re(a_h prod_sum_e[h]), w_h = 1/2 where m = 0. (The reference sums
+// f_n Re(Y prod_sum_e) over pairs; an atom's sum of f_n Y is its a_h.)
+// One workgroup of NL lanes (one wave, or four where there are few atoms or
+// much work) per atom, the atom's order parameters, the features that the
+// polynomial uses (its factors) and the columns' derivatives by them in LDS.
+//   1. values of the factors;
+//   2. dE/dx over the columns that hold a factor, each a coefficient times one
+//      or two other factors (also with c / n_c), in pieces of equal length, a
+//      lane each, added up in LDS;
+//   3. per head, a lane: its terms, a coefficient (for features outside the
+//      polynomial with dE/dx, a constant, folded in and merged), dE/dx and up
+//      to three order parameters; heads in order of decreasing term count in
+//      blocks of 64, so that a wave's lanes end together and no lane ends
+//      inside another's head.
+// Taking the gradient by the features first leaves about 600 terms instead of
+// 11,792 for the one-type order-2 model (every column's derivative by every
+// head before), and records of 12 or 16 bytes instead of 32: the tables come
+// from L2 for every atom, which held the kernel at 8 TB/s on the 1,350-head
+// model. FP64, 32,000 atoms of the one-type model: 0.71 -> 0.18 ms; 1,024-atom
+// alloy: 0.40 -> 0.09 ms; FP32, 20,480 atoms of the alloy: 5.8 -> 0.88 ms.
 // ---------------------------------------------------------------------------
-template <class T, int NL, bool HEADS_E>
+template <class T, int NL>
 __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, BatchDev bd,
                                                      const Cpx<T>* __restrict__ a_full,
-                                                     int a_stride, Cpx<T>* __restrict__ ps_e,
-                                                     Cpx<T>* __restrict__ ps_f, int ps_stride,
-                                                     double* __restrict__ e_at, int pair_model) {
+                                                     int a_stride, Cpx<T>* __restrict__ ps_f,
+                                                     int ps_stride, double* __restrict__ e_at,
+                                                     int pair_model) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    // two slots per lane of head sums (4 values each) and their heads, the
-    // atom's order parameters (a_stride complex values), then its features
-    constexpr int NS = 2 * NL;
-    double* sv = reinterpret_cast<double*>(smem_raw);
-    int* sh = reinterpret_cast<int*>(sv + 4 * NS);
-    Cpx<T>* a = reinterpret_cast<Cpx<T>*>(sh + NS);
-    T* xs = reinterpret_cast<T*>(a + a_stride);
+    __shared__ double e_part[NL / 64];
     const int i = blockIdx.x;
-    if (i >= bd.n_atoms_total) return;
     const int t1 = bd.types[i];
     const TypeDev& TT = md.t[t1];
     const EvalTypeDev& E = ed.t[t1];
-    const Cpx<T>* ag = a_full + (size_t)i * a_stride;
-    stage_cpx(a, ag, TT.n_nlm);
+    // sums of the derivatives by the factors; order parameters and the constant
+    // 1; (derivatives, the same with c / n_c) by the factors, then the constants of features outside the polynomial with
+    // 0 to 3 other order parameters; factors and 1
+    using V2 = typename Vec2Of<T>::type;
+    double2* sum = reinterpret_cast<double2*>(smem_raw);
+    Cpx<T>* a = reinterpret_cast<Cpx<T>*>(sum + E.n_poly);
+    V2* g = reinterpret_cast<V2*>(a + a_stride + 1);
+    T* xs = reinterpret_cast<T*>(g + E.n_poly + 4);
+    const int one = TT.n_nlm, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NW = NL / 64;
+    stage_cpx(a, a_full + (size_t)i * a_stride, TT.n_nlm);
+    if (threadIdx.x == 0) a[one] = {T(1), T(0)}, xs[E.n_poly] = T(1);
+    for (int q = threadIdx.x; q < E.n_poly; q += NL) sum[q] = E.pf_lin[q];
+    if (threadIdx.x < 4) {
+        V2 v;
+        v.x = T(1), v.y = T(1) / T(int(threadIdx.x) + 1);
+        g[E.n_poly + threadIdx.x] = v;
+    }
     __syncthreads();
-    for (int f = threadIdx.x; f < TT.n_lin; f += blockDim.x) {
+    {
+        // products with |Re| <= 1e-20 are dropped where the reference drops them
+        const T least = TT.fv_skip ? T(1e-20) : T(-1);
+        const T* c = EvalTab<T>::value(E);
+        for (int bk = wave; bk < E.vq_nblk; bk += NW) {
+            const int f = E.vq_item[bk * 64 + lane];
+            T v = T(0);
+            const int r1 = E.vq_boff[bk + 1];
+#pragma unroll 2
+            for (int r = E.vq_boff[bk] + lane; r < r1; r += 64) {
+                const T p = value_prod<T>(a, E.vq_key[r], ed.value_max).re;
+                v += fabs(p) > least ? c[r] * p : T(0);
+            }
+            if (f >= 0) xs[f] = v;
+        }
+    }
+    __syncthreads();
+    {
+        const auto* c = EvalTab<T>::poly(E);
+        for (int bk = wave; bk < E.pf_nblk; bk += NW) {
+            const int r1 = E.pf_boff[bk + 1];
+            double2 v = {0.0, 0.0};
+#pragma unroll 4
+            for (int r = E.pf_boff[bk] + lane; r < r1; r += 64) {
+                const unsigned k = (unsigned)E.pf_rec[r];
+                const double x = double(xs[k & 0xffff]) * double(xs[k >> 16]);
+                const auto cr = c[r];
+                v.x += double(cr.x) * x, v.y += double(cr.y) * x;
+            }
+            const int q = E.pf_piece[bk * 64 + lane];
+            if (q >= 0) atomicAdd(&sum[q].x, v.x), atomicAdd(&sum[q].y, v.y);
+        }
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < E.n_poly; q += NL) {
+        V2 w;
+        w.x = T(sum[q].x), w.y = T(sum[q].y);
+        g[q] = w;
+    }
+    __syncthreads();
+    const T scale = pair_model ? T(1) : T(2);
+    double e_sum = 0.0;
+    Cpx<T>* o = ps_f + (size_t)i * ps_stride;
+    const T* c = EvalTab<T>::term(E);
+    for (int bk = wave; bk < E.tq_nblk; bk += NW) {
+        const int h = E.tq_item[bk * 64 + lane];
+        T vr = T(0), vi = T(0), er = T(0), ei = T(0);
+        const int r1 = E.tq_boff[bk + 1];
+#pragma unroll 2
+        for (int r = E.tq_boff[bk] + lane; r < r1; r += 64) {
+            const int2 k = E.tq_key[r];
+            const V2 w = g[(unsigned)k.y >> 16];
+            const T cf = c[r] * w.x, ce = c[r] * w.y;
+            Cpx<T> p = a[k.x & 0xffff];
+            if (ed.term_max > 1) p = cmul(p, a[(unsigned)k.x >> 16]);
+            if (ed.term_max > 2) p = cmul(p, a[k.y & 0xffff]);
+            vr += cf * p.re, vi += cf * p.im;
+            er += ce * p.re, ei += ce * p.im;
+        }
+        if (h >= 0) {
+            o[h] = {scale * vr, scale * vi};
+            const int ha = E.hd_a[h];  // the head's order parameter, bit 30: m = 0
+            const Cpx<T> ac = a[ha & 0x3fffffff];
+            const double v = double(er) * double(ac.re) - double(ei) * double(ac.im);
+            e_sum += (ha >> 30) & 1 ? 0.5 * v : v;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) e_sum += __shfl_xor(e_sum, off);
+    if (lane == 0) e_part[wave] = e_sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < NW; ++w) e_sum += e_part[w];
+        e_at[i] = double(scale) * e_sum;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// prod_sum_e and prod_sum_f of one atom's heads from the folded potential's
+// terms, coeff_{e,f} * prod_features * prod_anlm (plm_api_sum_of_prod).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int key16(unsigned k) { return k == 0xffffu ? -1 : (int)k; }
+
+template <class T>
+__global__ void __launch_bounds__(64) head_terms_kernel(ModelDev md, BatchDev bd,
+                                                        const Cpx<T>* __restrict__ a, int n_heads,
+                                                        const int* __restrict__ off,
+                                                        const int4* __restrict__ key,
+                                                        const double2* __restrict__ coeff,
+                                                        Cpx<T>* __restrict__ ps_e,
+                                                        Cpx<T>* __restrict__ ps_f) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    T* xs = reinterpret_cast<T*>(smem_raw);
+    const TypeDev& TT = md.t[bd.types[0]];
+    for (int f = threadIdx.x; f < TT.n_lin; f += 64) {
         T v = T(0);
         for (int e = TT.fv_off[f]; e < TT.fv_off[f + 1]; ++e) {
             Cpx<T> pr = {T(1), T(0)};
@@ -77,101 +211,24 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
         xs[f] = v;
     }
     __syncthreads();
-    const int lane = threadIdx.x;
-    Cpx<T>* oe = HEADS_E ? ps_e + (size_t)i * ps_stride : nullptr;
-    Cpx<T>* of = ps_f + (size_t)i * ps_stride;
-    const double scale = pair_model ? 0.5 : 1.0;
-    // a head that begins and ends inside the lane's chunk is written at once;
-    // the chunk's first and last heads (which may continue in the neighbouring
-    // chunks) go to the lane's two slots, summed over lanes afterwards
-    int cur = -1, first = -1;
-    T er = T(0), ei = T(0), fr = T(0), fi = T(0);
-    double e_sum = 0.0;
-    auto add_energy = [&] {
-        if constexpr (!HEADS_E) {
-            const int ha = E.hd_a[cur];  // its order parameter, bit 30: m = 0
-            const Cpx<T> ac = a[ha & 0x3fffffff];
-            const double v = double(er) * double(ac.re) - double(ei) * double(ac.im);
-            e_sum += (ha >> 30) & 1 ? 0.5 * v : v;
+    for (int h = threadIdx.x; h < n_heads; h += 64) {
+        T er = T(0), ei = T(0), fr = T(0), fi = T(0);
+        for (int e = off[h]; e < off[h + 1]; ++e) {
+            const int4 k = key[e];
+            const int pd[3] = {key16(k.x & 0xffff), key16((unsigned)k.x >> 16), key16(k.y & 0xffff)};
+            const int pf[2] = {key16(k.z & 0xffff), key16((unsigned)k.z >> 16)};
+            T fval = T(1);
+            for (int q = 0; q < 2; ++q)
+                if (pf[q] >= 0) fval *= xs[pf[q]];
+            Cpx<T> pr = {T(1), T(0)};
+            for (int q = 0; q < 3; ++q)
+                if (pd[q] >= 0) pr = cmul(pr, a[pd[q]]);
+            const T se = fval * T(coeff[e].x), sf = fval * T(coeff[e].y);
+            er += pr.re * se, ei += pr.im * se;
+            fr += pr.re * sf, fi += pr.im * sf;
         }
-    };
-    auto to_slot = [&](int sl) {
-        sh[sl] = cur;
-        if constexpr (HEADS_E) sv[4 * sl] = double(er), sv[4 * sl + 1] = double(ei);
-        sv[4 * sl + 2] = double(fr), sv[4 * sl + 3] = double(fi);
-    };
-    sh[2 * lane] = sh[2 * lane + 1] = -1;
-    for (int h = lane; h < E.n_heads; h += blockDim.x)
-        if (E.pot_off[h + 1] == E.pot_off[h]) {
-            if constexpr (HEADS_E) oe[h] = {T(0), T(0)};
-            of[h] = {T(0), T(0)};
-        }
-    for (int it = 0; it < E.pq_iters; ++it) {
-        const int4 k = E.pq_key[(size_t)it * NL + lane];
-        const double2 c = E.pq_c[(size_t)it * NL + lane];
-        const int head = (unsigned)k.y >> 16;
-        if (head == 0xffff) break;  // the rest of this lane's chunk is padding
-        if (head != cur) {
-            if (cur >= 0) {
-                add_energy();
-                if (cur == first) {
-                    to_slot(2 * lane);
-                } else {
-                    if constexpr (HEADS_E) oe[cur] = {T(scale * er), T(scale * ei)};
-                    of[cur] = {T(scale * fr), T(scale * fi)};
-                }
-            }
-            if (first < 0) first = head;
-            cur = head, er = ei = fr = fi = T(0);
-        }
-        const int pd0 = k.x & 0xffff, pd1 = (unsigned)k.x >> 16, pd2 = k.y & 0xffff;
-        const int pf0 = k.z & 0xffff, pf1 = (unsigned)k.z >> 16;
-        T fval = T(1);
-        if (pf0 != 0xffff) fval *= xs[pf0];
-        if (pf1 != 0xffff) fval *= xs[pf1];
-        Cpx<T> pr = {T(1), T(0)};
-        if (pd0 != 0xffff) {
-            pr = a[pd0];
-            if (pd1 != 0xffff) {
-                pr = cmul(pr, a[pd1]);
-                if (pd2 != 0xffff) pr = cmul(pr, a[pd2]);
-            }
-        }
-        const T se = fval * T(c.x), sf = fval * T(c.y);
-        er += pr.re * se, ei += pr.im * se;
-        fr += pr.re * sf, fi += pr.im * sf;
-    }
-    if (cur >= 0) {
-        add_energy();
-        to_slot(cur == first ? 2 * lane : 2 * lane + 1);
-    }
-    __syncthreads();
-    // slots in term order, empty ones skipped: the first slot of each head sums
-    // the slots of that head and writes it
-    for (int sl = 2 * lane; sl < 2 * lane + 2; ++sl) {
-        const int h = sh[sl];
-        if (h < 0) continue;
-        int p = sl - 1;
-        while (p >= 0 && sh[p] < 0) --p;
-        if (p >= 0 && sh[p] == h) continue;
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-        for (int q = sl; q < NS && (sh[q] == h || sh[q] < 0); ++q) {
-            if (sh[q] < 0) continue;
-            if constexpr (HEADS_E) s0 += sv[4 * q], s1 += sv[4 * q + 1];
-            s2 += sv[4 * q + 2], s3 += sv[4 * q + 3];
-        }
-        if constexpr (HEADS_E) oe[h] = {T(scale * s0), T(scale * s1)};
-        of[h] = {T(scale * s2), T(scale * s3)};
-    }
-    if constexpr (!HEADS_E) {
-        for (int off = 32; off > 0; off >>= 1) e_sum += __shfl_down(e_sum, off);
-        __syncthreads();  // the slots are read
-        if ((lane & 63) == 0) sv[lane >> 6] = e_sum;
-        __syncthreads();
-        if (lane == 0) {
-            for (int w = 1; w < NL / 64; ++w) e_sum += sv[w];
-            e_at[i] = scale * e_sum;
-        }
+        ps_e[h] = {er, ei};
+        ps_f[h] = {fr, fi};
     }
 }
 
@@ -588,52 +645,72 @@ __global__ void __launch_bounds__(256) eval_sum_kernel(BatchDev bd, int n_pairs,
     }
 }
 
-template <class T, int NL, bool HEADS_E>
+template <class T, int NL>
 void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
-                      const void* a_full, int a_stride, void* ps_e, void* ps_f, int ps_stride,
-                      double* e_at, int max_lin, int pair_model) {
-    const size_t sm = 2 * NL * (4 * sizeof(double) + sizeof(int)) +
-                      (size_t)a_stride * 2 * sizeof(T) + (size_t)std::max(1, max_lin) * sizeof(T);
+                      const void* a_full, int a_stride, void* ps_f, int ps_stride, double* e_at,
+                      int pair_model) {
+    const size_t sm = (size_t)ed.poly_max * sizeof(double2) +
+                      (size_t)(a_stride + 1) * 2 * sizeof(T) + (size_t)(ed.poly_max + 4) * 2 * sizeof(T) +
+                      (size_t)(ed.poly_max + 1) * sizeof(T);
     if (sm > 160 * 1024) throw std::invalid_argument("per-atom evaluation data exceed LDS");
-    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL, HEADS_E>),
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
               "prodsum shared memory");
-    prodsum_kernel<T, NL, HEADS_E><<<bd.n_atoms_total, NL, sm, st>>>(
+    prodsum_kernel<T, NL><<<bd.n_atoms_total, NL, sm, st>>>(
         md, ed, bd, reinterpret_cast<const Cpx<T>*>(a_full), a_stride,
-        reinterpret_cast<Cpx<T>*>(ps_e), reinterpret_cast<Cpx<T>*>(ps_f), ps_stride, e_at,
-        pair_model);
+        reinterpret_cast<Cpx<T>*>(ps_f), ps_stride, e_at, pair_model);
 }
 
-template <class T, bool HEADS_E>
-void launch_prodsum_lanes(hipStream_t st, const ModelDev& md, const EvalDev& ed,
-                          const BatchDev& bd, const void* a_full, int a_stride, void* ps_e,
-                          void* ps_f, int ps_stride, double* e_at, int max_lin, int pair_model) {
-    // the term tables were laid out for ed.pq_lanes lanes
-    if (ed.pq_lanes == 256)
-        launch_prodsum_t<T, 256, HEADS_E>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                          e_at, max_lin, pair_model);
-    else if (ed.pq_lanes == 64)
-        launch_prodsum_t<T, 64, HEADS_E>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                         e_at, max_lin, pair_model);
-    else
-        throw std::invalid_argument("contraction lanes must be 64 or 256");
-}
-
+// Four waves an atom where its table rows are more than 128 or the atoms do
+// not fill the chip with eight waves a SIMD, else one (20,480 atoms of the
+// 1,350-head model, FP32: 0.98 ms with four, 2.73 with one; 54 atoms of the
+// one-type model 22 and 54 us; 32,000 atoms of it 0.64 and 0.66 ms, equal);
+// PLM_PRODSUM_LANES=64|256 forces one form.
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
-                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_e, void* ps_f,
-                    int ps_stride, double* e_at, int max_lin, int pair_model) {
-    if (fp64 && ps_e)
-        launch_prodsum_lanes<double, true>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                           e_at, max_lin, pair_model);
-    else if (ps_e)
-        launch_prodsum_lanes<float, true>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                          e_at, max_lin, pair_model);
+                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,
+                    int ps_stride, double* e_at, int pair_model) {
+    bool four = ed.rows_max > 128 || bd.n_atoms_total < 8192;
+    if (const char* e = std::getenv("PLM_PRODSUM_LANES")) {
+        if (!std::strcmp(e, "64")) four = false;
+        else if (!std::strcmp(e, "256")) four = true;
+        else throw std::invalid_argument("PLM_PRODSUM_LANES must be 64 or 256");
+    }
+    if (fp64 && four)
+        launch_prodsum_t<double, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
+                                      pair_model);
     else if (fp64)
-        launch_prodsum_lanes<double, false>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f,
-                                            ps_stride, e_at, max_lin, pair_model);
+        launch_prodsum_t<double, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
+                                     pair_model);
+    else if (four)
+        launch_prodsum_t<float, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
+                                     pair_model);
     else
-        launch_prodsum_lanes<float, false>(st, md, ed, bd, a_full, a_stride, ps_e, ps_f, ps_stride,
-                                           e_at, max_lin, pair_model);
+        launch_prodsum_t<float, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
+                                    pair_model);
+}
+
+void launch_head_terms(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd,
+                       const void* a, int n_heads, const int* off, const int4* key,
+                       const double2* coeff, int max_lin, void* ps_e, void* ps_f) {
+    const size_t sm = (size_t)std::max(1, max_lin) * (fp64 ? 8 : 4);
+    if (sm > 160 * 1024) throw std::invalid_argument("per-atom evaluation data exceed LDS");
+    if (fp64) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&head_terms_kernel<double>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
+                  "head terms shared memory");
+        head_terms_kernel<double><<<1, 64, sm, st>>>(md, bd, static_cast<const Cpx<double>*>(a),
+                                                     n_heads, off, key, coeff,
+                                                     static_cast<Cpx<double>*>(ps_e),
+                                                     static_cast<Cpx<double>*>(ps_f));
+    } else {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&head_terms_kernel<float>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
+                  "head terms shared memory");
+        head_terms_kernel<float><<<1, 64, sm, st>>>(md, bd, static_cast<const Cpx<float>*>(a),
+                                                    n_heads, off, key, coeff,
+                                                    static_cast<Cpx<float>*>(ps_e),
+                                                    static_cast<Cpx<float>*>(ps_f));
+    }
 }
 
 template <class T>

@@ -88,7 +88,6 @@ struct TypeTables {
     std::vector<std::vector<DerivTerm>> feat_deriv;      // feature -> deriv terms (sorted)
     std::vector<PolyTerm> poly;                          // polynomial columns of this type
     std::vector<std::vector<int>> prod_features;         // products of features (poly)
-    std::vector<std::vector<PotTerm>> pot;               // per noconj head (eval)
 };
 
 class Model {
@@ -112,10 +111,13 @@ class Model {
     const std::vector<std::vector<std::vector<int>>>& tp_combs() const { return tp_combs_; }
     const std::vector<std::vector<int>>& type_pairs() const { return type_pairs_; }
 
-    // Fold fitted coefficients (as passed to PolymlpEval, i.e. coeffs/scales;
-    // the factor 2 of polymlp_eval.cpp:17 is applied here) into per-head terms.
+    // Fitted coefficients as passed to PolymlpEval, i.e. coeffs/scales (the
+    // factor 2 of polymlp_eval.cpp:17 is applied where they are used).
     void set_potential(const std::vector<double>& coeffs);
     bool has_potential() const { return has_pot_; }
+    const std::vector<double>& coeffs() const { return coeffs_; }
+    // the folded per-head terms of a type (plm_api_sum_of_prod)
+    std::vector<std::vector<PotTerm>> head_terms(int t) const;
 
   private:
     ModelInput in_;
@@ -135,6 +137,7 @@ class Model {
     int n_linear_ = 0, n_variables_ = 0;
     std::vector<TypeTables> types_;
     bool has_pot_ = false;
+    std::vector<double> coeffs_;
 
     void set_type_pairs();
     void set_nlm();
