@@ -1165,31 +1165,51 @@ int plm_features_x(plm_model* mp, plm_batch* bp, int precision, double* x_out) {
         hipStream_t st = dev.stream;
         DevBuf xb;
         XWork work;
-        std::vector<double> hx((size_t)F);
-        std::vector<long> order(R);
-        plm_batch_row_order(bp, order.data());
-        std::vector<long> inv(R);
-        for (long r = 0; r < R; ++r) inv[order[r]] = r;
+        DevBuf outb, srcb;
+        std::vector<int> src;
         // process structures in chunks bounded by ~1 GiB of X
         const size_t row_bytes = (size_t)F * elem;
+        // the rows leave in the reference's order (energies, stresses, forces),
+        // gathered on the device kOutBytes at a time: each gathered piece is
+        // one to three runs of the caller's rows
+        constexpr size_t kOutBytes = 128ull << 20;
+        const long piece = std::max<long>(1, (long)(kOutBytes / ((size_t)F * 8)));
         int s0 = 0;
-        std::vector<char> hbuf;
         while (s0 < b->n_st) {
             int s1 = s0 + 1;
             while (s1 < b->n_st && (size_t)(b->row_off[s1 + 1] - b->row_off[s0]) * row_bytes < (1ull << 30)) ++s1;
-            const long r0 = b->row_off[s0], r1 = b->row_off[s1];
-            xb.alloc((size_t)(r1 - r0) * row_bytes);
+            const long r0 = b->row_off[s0], rows = b->row_off[s1] - r0;
+            xb.alloc((size_t)rows * row_bytes);
             build_x_rows(*m, *b, s0, s1, fp64, xb.ptr, F, nullptr, nullptr, nullptr, work);
-            hbuf.resize((size_t)(r1 - r0) * row_bytes);
-            check_hip(hipMemcpyAsync(hbuf.data(), xb.ptr, hbuf.size(), hipMemcpyDeviceToHost, st), "copy");
-            check_hip(hipStreamSynchronize(st), "sync");
-            for (long r = r0; r < r1; ++r) {
-                double* dst = x_out + (size_t)inv[r] * F;
-                if (fp64) std::memcpy(dst, hbuf.data() + (size_t)(r - r0) * row_bytes, row_bytes);
-                else {
-                    const float* src = reinterpret_cast<const float*>(hbuf.data() + (size_t)(r - r0) * row_bytes);
-                    for (int c = 0; c < F; ++c) dst[c] = src[c];
+            src.clear();
+            for (int s = s0; s < s1; ++s) src.push_back((int)(b->row_off[s] - r0));
+            for (int s = s0; s < s1; ++s)
+                for (int k = 0; k < 6; ++k) src.push_back((int)(b->row_off[s] - r0) + 1 + k);
+            for (int s = s0; s < s1; ++s)
+                for (long r = b->row_off[s] + 7; r < b->row_off[s + 1]; ++r)
+                    src.push_back((int)(r - r0));
+            srcb.alloc(src.size() * sizeof(int));
+            check_hip(hipMemcpyAsync(srcb.ptr, src.data(), src.size() * sizeof(int),
+                                     hipMemcpyHostToDevice, st), "copy");
+            outb.alloc((size_t)std::min(piece, rows) * F * 8);
+            const long ns = s1 - s0;
+            // runs of the chunk's rows and where they start in the caller's
+            const long run0[4] = {0, ns, 7 * ns, rows};
+            const long dst0[3] = {s0, b->n_st + 6l * s0, 7l * b->n_st + 3l * b->atom_off[s0]};
+            for (long q0 = 0; q0 < rows; q0 += piece) {
+                const long q1 = std::min(rows, q0 + piece);
+                launch_gather_rows(st, fp64, xb.ptr, F, (const int*)srcb.ptr + q0, (int)(q1 - q0),
+                                   F, (double*)outb.ptr);
+                check_hip(hipGetLastError(), "gather rows launch");
+                for (int k = 0; k < 3; ++k) {
+                    const long u0 = std::max(q0, run0[k]), u1 = std::min(q1, run0[k + 1]);
+                    if (u0 >= u1) continue;
+                    check_hip(hipMemcpyAsync(x_out + (size_t)(dst0[k] + u0 - run0[k]) * F,
+                                             (const double*)outb.ptr + (size_t)(u0 - q0) * F,
+                                             (size_t)(u1 - u0) * F * 8, hipMemcpyDeviceToHost, st),
+                              "copy");
                 }
+                check_hip(hipStreamSynchronize(st), "sync");
             }
             s0 = s1;
         }
@@ -1235,19 +1255,31 @@ int plm_normal_result(plm_normal* ap, double* xtx, double* xty, double* xe_sum, 
         const int F = acc->F, Fp = acc->F_pad;
         check_hip(hipStreamSynchronize(st), "sync");
         // Gram of [X | y]: the upper element triangle is valid (the tiles cover
-        // the upper block triangle), so mirror element-wise; column F holds
-        // X^T y and element (F, F) y^T y
+        // the upper block triangle), column F holds X^T y and element (F, F)
+        // y^T y; the rows leave mirrored and unpadded, kOutBytes at a time
         if (xtx || xty) {
-            std::vector<double> full((size_t)Fp * Fp);
-            check_hip(hipMemcpy(full.data(), acc->xtx.ptr, full.size() * 8, hipMemcpyDeviceToHost),
-                      "copy");
-            if (xtx)
-                for (int i = 0; i < F; ++i)
-                    for (int j = 0; j < F; ++j)
-                        xtx[(size_t)i * F + j] =
-                            i <= j ? full[(size_t)i * Fp + j] : full[(size_t)j * Fp + i];
-            if (xty)
-                for (int i = 0; i < F; ++i) xty[i] = full[(size_t)i * Fp + F];
+            constexpr size_t kOutBytes = 128ull << 20;
+            const int piece =
+                std::min<long>((F + 31) / 32, std::max<long>(1, (long)(kOutBytes / (256ull * F)))) * 32;
+            DevBuf rows, col;
+            rows.alloc((size_t)std::min(piece, F) * F * 8);
+            col.alloc((size_t)F * 8);
+            for (int i0 = 0; i0 < F; i0 += piece) {
+                const int n = std::min(piece, F - i0);
+                launch_gram_mirror(st, (const double*)acc->xtx.ptr, Fp, F, i0, n,
+                                   (double*)rows.ptr, (double*)col.ptr);
+                check_hip(hipGetLastError(), "gram mirror launch");
+                if (xtx) {
+                    check_hip(hipMemcpyAsync(xtx + (size_t)i0 * F, rows.ptr, (size_t)n * F * 8,
+                                             hipMemcpyDeviceToHost, st), "copy");
+                    check_hip(hipStreamSynchronize(st), "sync");
+                }
+            }
+            if (xty) {
+                check_hip(hipMemcpyAsync(xty, col.ptr, (size_t)F * 8, hipMemcpyDeviceToHost, st),
+                          "copy");
+                check_hip(hipStreamSynchronize(st), "sync");
+            }
         }
         if (y_sq)
             check_hip(hipMemcpy(y_sq, (const double*)acc->xtx.ptr + (size_t)F * Fp + F, 8,
