@@ -224,6 +224,15 @@ void ModelHandle::build_device() {
         }
         max_nlm = std::max(max_nlm, D.n_nlm);
         max_noconj = std::max(max_noconj, D.n_noconj);
+        {
+            std::vector<int> at_nc(D.n_noconj, 0), at;
+            const int ncol = 2 * std::max(1, md.n_lmh);
+            for (int g = 0; g < nt; ++g)
+                for (const auto& e : by_tp[md.tp_of[t * nt + g]])
+                    at_nc[e[0]] = (g * md.n_fn + e[1]) * ncol + 2 * std::max(0, e[2]);
+            for (int k : src) at.push_back(at_nc[k]);
+            D.nlm_at = up(*this, at);
+        }
         D.nlm_src = up(*this, src);
         D.nlm_sign = up(*this, sign);
         D.nlm_conj = up(*this, conj);

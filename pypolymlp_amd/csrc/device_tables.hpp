@@ -19,6 +19,9 @@ struct TypeDev {
     const int* nlm_src;        // [n_nlm] noconj index of the source
     const float* nlm_sign;     // [n_nlm] +1 plain, cc for conjugates (sign of imag flips)
     const unsigned char* nlm_conj;  // [n_nlm]
+    // where component k's source sits in the atom's sums by (neighbour type,
+    // radial function, Y key, re/im): [n_type][n_fn][2 max(1, n_lmh)]
+    const int* nlm_at;         // [n_nlm]
     // anlm accumulation grouped by type pair: heads with tp == p
     const int* nc_tp_off;      // [n_tp+1]
     const int* nc_tp_head;     // noconj index

@@ -4,6 +4,7 @@
 //   Local::compute_anlmtp_d (values, conjugate fill)  src/cxx/src/compute/local.cpp:116-217
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <stdexcept>
@@ -168,6 +169,234 @@ __global__ void __launch_bounds__(NT) anlm_reg_kernel(ModelDev md, BatchDev bd,
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same sums as a matrix product per atom, one workgroup of four waves:
+//   a[(type, n)][key] = sum_p F[n][p] Y[key][p],
+// F the radial functions (a row of another type's pairs masked to zero), Y the
+// spherical harmonics, re and im in columns of their own, p the atom's
+// neighbours, 64 at a time. A lane takes a pair; one or two waves take the
+// columns m of Y (recurrences unrolled to LB, so their square roots are
+// constants; the form above takes them, and a division each, per pair), the
+// others the radial functions; both go to LDS as [row][pair] (pitch 66 doubles or
+// 68 floats: the 16 rows x 4 pairs of an MFMA operand are then on banks of
+// their own), and 16 x 16 x 4 MFMA tiles, dealt to the waves, Q at most each,
+// add them up in registers. Bound by the FP64 functions of each pair (distance,
+// angles, cos, exp: the matrix units take a fifth of the time), hence by waves
+// in flight: four a SIMD (128 registers; with the 144 the compiler took 0.24 ms)
+// and the angles and the cutoff function not in every wave (0.32 ms).
+// Register sums -> this: FP64, 32,000 atoms of 55 neighbours, 165 heads 0.77 ->
+// 0.20 ms; 1,024 alloy atoms, 1,350 heads 0.17 -> 0.056 ms; 54 atoms 41 -> 7 us;
+// 8,000 atoms, pair model 0.15 -> 0.05 ms; FP32, 20,480 alloy atoms 1.85 -> 0.39 ms.
+// ---------------------------------------------------------------------------
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+template <class T> struct AnlmTile;
+template <> struct AnlmTile<float> {
+    using acc = floatx4;
+    static constexpr int pitch = 68;
+    static __device__ acc mfma(float a, float b, acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
+};
+template <> struct AnlmTile<double> {
+    using acc = doublex4;
+    static constexpr int pitch = 66;
+    static __device__ acc mfma(double a, double b, acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
+};
+
+// cos(pi r / rc) and (cos phi, sin phi): FP32 by the expressions of the forms
+// above, whose rounding is most of the error of its energies; FP64 (1e-16 apart)
+// without the reduction of large arguments, the scaling of hypot and one division
+__device__ __forceinline__ float cutoff_cos(float r, float rc) {
+    return cos(MathConst<float>::pi / rc * r);
+}
+__device__ __forceinline__ double cutoff_cos(double r, double rc) { return cospi(r / rc); }
+__device__ __forceinline__ void phi_unit(float x, float y, float& cp, float& sp) {
+    const float rho = dhypot(x, y);
+    if (rho > 0.f) cp = x / rho, sp = y / rho;
+}
+__device__ __forceinline__ void phi_unit(double x, double y, double& cp, double& sp) {
+    const double rho = sqrt(x * x + y * y);
+    if (rho > 0.0) {
+        const double inv = 1.0 / rho;
+        cp = x * inv, sp = y * inv;
+    }
+}
+
+template <class T, int LB, int Q>
+__global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev md, BatchDev bd,
+                                                        Cpx<T>* __restrict__ a_full, int a_stride,
+                                                        int atom0, int negate) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    using M = AnlmTile<T>;
+    using C = MathConst<T>;
+    constexpr int P = M::pitch;
+    const int nfn = md.n_fn, ncol = 2 * max(1, md.n_lmh);
+    T* F = reinterpret_cast<T*>(smem_raw);  // [n_fn][P]
+    T* Y = F + (size_t)nfn * P;             // [ncol][P]
+    __shared__ int group[64];
+    const int ia = blockIdx.x;
+    const int i = atom0 + ia;
+    const int t1 = bd.types[i];
+    const TypeDev& TT = md.t[t1];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rt = (nfn + 15) / 16, ct = (ncol + 15) / 16;
+    const int tiles = md.n_type * rt * ct;
+    const int lmax = md.max_l;
+    // waves on Y's columns, the others take the radial functions
+    constexpr int NA = LB <= 4 ? 1 : 2;
+    const int na = lmax < 0 ? 0 : NA;
+    typename M::acc acc[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] = typename M::acc{T(0), T(0), T(0), T(0)};
+    const int p0 = bd.nb_off[i], p1 = bd.nb_off[i + 1];
+    for (int c0 = p0; c0 < p1; c0 += 64) {
+        const int np = min(64, p1 - c0);
+        if (c0 > p0) __syncthreads();  // the tiles have read the last chunk
+        double dx = 0.0, dy = 0.0, dz = 0.0, dis = 0.0;
+        int t2 = 0;
+        if (lane < np) {
+            const double* dk = bd.nb_d + 3 * (size_t)(c0 + lane);
+            t2 = bd.types[bd.nb_j[c0 + lane]];
+            // evaluation: the reversed vector r_i - r_j - T (polymlp_eval.cpp:376-379)
+            const double sg = negate ? -1.0 : 1.0;
+            dx = sg * dk[0], dy = sg * dk[1], dz = sg * dk[2];
+            dis = sqrt(dx * dx + dy * dy + dz * dz);
+        }
+        const bool on = lane < np && dis < md.cutoff;
+        if (w == 0) group[lane] = t2;
+        if (w >= na) {
+            const int tp = md.tp_of[t1 * md.n_type + t2];
+            const int cnt = on ? md.rad_count[tp] : 0;
+            const double* rp = md.rad + (size_t)tp * nfn * 2;
+            const T fc = T(0.5) * (cutoff_cos(T(dis), T(md.cutoff)) + T(1));
+            for (int n = w - na; n < nfn; n += 4 - na) {
+                const T beta = T(rp[2 * n]), x = T(dis) - T(rp[2 * n + 1]);
+                const T f = dexp(-beta * x * x) * fc;
+                F[n * P + lane] = n < cnt && !(f < T(1e-20)) ? f : T(0);
+            }
+            if (lmax < 0 && w < 2) Y[w * P + lane] = w == 0 ? T(1) : T(0);
+        } else {
+            const T x = T(dx), y = T(dy), z = T(dz), r = T(dis);
+            const T ct_ = on ? z / r : T(1);
+            T cp = T(1), sp = T(0);
+            phi_unit(x, y, cp, sp);
+            const T st = dsqrt(T(1) - ct_ * ct_);
+            T c = T(1), s = T(0);  // cos, sin (m phi) by the Chebyshev recurrence
+            T c1 = T(1), c2 = cp, s1 = T(0), s2 = -sp, pmm = C::sqrt_inv_2pi;
+            const T tc = T(2) * c2;
+#pragma unroll
+            for (int m = 0; m <= LB; ++m) {
+                if (m > lmax) break;
+                if (m >= 1) {
+                    s = tc * s1 - s2;
+                    c = tc * c1 - c2;
+                    c2 = c1, c1 = c, s2 = s1, s1 = s;
+                    pmm *= m == 1 ? -st * C::sqrt3div2
+                                  : -dsqrt(T(1) + T(0.5) / T(m)) * st;
+                }
+                if (m % NA != w) continue;
+                const T sign = (m % 2 == 1) ? T(-1) : T(1);
+                T pa = T(0), pb = pmm;
+#pragma unroll
+                for (int l = m; l <= LB; ++l) {
+                    if (l > lmax) break;
+                    if (l == m + 1) {
+                        const T pn = m == 0 ? ct_ * C::sqrt3 * C::sqrt_inv_2pi
+                                            : dsqrt(T(2) * T(m) + T(3)) * ct_ * pb;
+                        pa = pb, pb = pn;
+                    } else if (l > m) {
+                        const T ls = T(l * l), lm1s = T((l - 1) * (l - 1)), msq = T(m * m);
+                        const T alm = dsqrt((T(4) * ls - T(1)) / (ls - msq));
+                        const T blm = -dsqrt((lm1s - msq) / (T(4) * lm1s - T(1)));
+                        const T pn = alm * (ct_ * pb + blm * pa);
+                        pa = pb, pb = pn;
+                    }
+                    const int key = lm2i(l, -m) + l;
+                    const T tmp = sign * pb * C::half_sqrt2;
+                    Y[(2 * key) * P + lane] = on ? (m == 0 ? tmp : tmp * c) : T(0);
+                    Y[(2 * key + 1) * P + lane] = on && m > 0 ? -tmp * s : T(0);
+                }
+            }
+        }
+        __syncthreads();
+        const int rl = lane & 15, kl = lane >> 4;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int t = w + 4 * q;
+            if (t >= tiles) break;
+            const int g = t / (rt * ct), tr = t % (rt * ct) / ct, tcol = t % ct;
+            // rows and columns past the end: any values, not read back
+            const T* a = F + (size_t)min(16 * tr + rl, nfn - 1) * P + kl;
+            const T* b = Y + (size_t)min(16 * tcol + rl, ncol - 1) * P + kl;
+            for (int k = 0; k < np; k += 16) {
+                T fa[4], fb[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int gu = group[k + 4 * u + kl];
+                    fa[u] = a[k + 4 * u], fb[u] = b[k + 4 * u];
+                    fa[u] = gu == g ? fa[u] : T(0);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[q] = M::mfma(fa[u], fb[u], acc[q]);
+            }
+        }
+    }
+    __syncthreads();
+    T* sums = F;  // [n_type][n_fn][ncol]
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int t = w + 4 * q;
+        if (t >= tiles) break;
+        const int g = t / (rt * ct), tr = t % (rt * ct) / ct, tcol = t % ct;
+        const int col = 16 * tcol + (lane & 15);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int n = 16 * tr + M::row(lane, v);
+            if (n < nfn && col < ncol) sums[((size_t)g * nfn + n) * ncol + col] = acc[q][v];
+        }
+    }
+    __syncthreads();
+    Cpx<T>* out = a_full + (size_t)ia * a_stride;
+    for (int k = threadIdx.x; k < TT.n_nlm; k += 256) {
+        const int at = TT.nlm_at[k];
+        const T re = sums[at], im = sums[at + 1];
+        const T cc = T(TT.nlm_sign[k]);
+        out[k] = TT.nlm_conj[k] ? Cpx<T>{cc * re, -cc * im} : Cpx<T>{re, im};
+    }
+}
+
+// true: launched; false: the model has Y columns past the unrolled ones, more
+// tiles than four waves hold in registers (16 each) or rows past a CU's LDS, and
+// the forms with sums per head below take it. Where it fits it is the faster
+// one at every size tried (54 to 32,000 atoms, above).
+template <class T>
+bool launch_anlm_mfma(hipStream_t st, const ModelDev& md, const BatchDev& bd, void* a_full,
+                      int a_stride, int atom0, int n_atoms, int negate) {
+    const int ncol = 2 * std::max(1, md.n_lmh);
+    const int tiles = md.n_type * ((md.n_fn + 15) / 16) * ((ncol + 15) / 16);
+    const size_t sm = std::max((size_t)(md.n_fn + ncol) * AnlmTile<T>::pitch,
+                               (size_t)md.n_type * md.n_fn * ncol) * sizeof(T);
+    if (md.max_l > 12 || tiles > 4 * 16 || sm > 156 * 1024) return false;
+    auto go = [&](auto kernel) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
+                  "anlm shared memory");
+        kernel<<<n_atoms, 256, sm, st>>>(md, bd, reinterpret_cast<Cpx<T>*>(a_full), a_stride,
+                                         atom0, negate);
+    };
+    const int q = (tiles + 3) / 4;
+    if (md.max_l <= 4 && q <= 4) go(&anlm_mfma_kernel<T, 4, 4>);
+    else if (md.max_l <= 8 && q <= 4) go(&anlm_mfma_kernel<T, 8, 4>);
+    else go(&anlm_mfma_kernel<T, 12, 16>);
+    return true;
+}
+
 size_t anlm_smem(const ModelDev& md, int elem, int nthreads, int max_noconj) {
     const PairLayout<double> L(md.n_fn, md.n_lmh, false);
     return (size_t)nthreads * L.stride * elem + (size_t)max_noconj * 2 * elem;
@@ -183,7 +412,8 @@ void launch_anlm_reg(hipStream_t st, const ModelDev& md, const BatchDev& bd, voi
                                                        a_stride, atom0, n_atoms, negate);
 }
 
-// register sums with 2-4 entries per thread (measured: 128 x 2 for 165 heads
+// The product form above where the model fits it; else register sums with 2-4
+// entries per thread (measured: 128 x 2 for 165 heads
 // 0.96 ms per 32,000 atoms against 1.37 ms for 64 x 4 and 1.06 ms for 256 x 1;
 // 512 x 3 for 1,350 heads 2.20 ms per 8,192 atoms against 2.73 ms for 256 x 8),
 // up to 2,048 heads per type; LDS sums beyond
@@ -192,6 +422,9 @@ void launch_anlm_reg(hipStream_t st, const ModelDev& md, const BatchDev& bd, voi
 template <class T>
 void launch_anlm_t(hipStream_t st, const ModelDev& md, const BatchDev& bd, void* a_full,
                    int a_stride, int atom0, int n_atoms, int max_noconj, int negate) {
+    if (!getenv("PLM_ANLM_SHAPE") &&
+        launch_anlm_mfma<T>(st, md, bd, a_full, a_stride, atom0, n_atoms, negate))
+        return;
     const int B = 64;
     const size_t sm = anlm_smem(md, sizeof(T), kAnlmPairs, max_noconj);
     if (const char* e = getenv("PLM_ANLM_SHAPE")) {

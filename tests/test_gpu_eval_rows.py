@@ -2,7 +2,8 @@
 stresses are the energy, force and stress rows times c, and the rows come from
 kernels of their own. FP64, 1e-11 of the largest value per structure (sums of
 up to some thousand terms); at radial functions that do not fill the pair loop's
-rows of four, at each of its bounds on max_l, with few pairs (keys split over
+rows of four, at each of its bounds on max_l, with neighbours around and past
+the 64 of an order-parameter chunk and more tiles than that form holds, with few pairs (keys split over
 workgroups) and many, with type pairs of unequal and no radial functions."""
 
 import numpy as np
@@ -38,6 +39,7 @@ def spec(n_type=1, max_l=(4,), n_gauss=4, max_p=2, model_type=4, cond=None, **kw
 SMALL = [(1, 3.1), (2, 4.0), (9, 6.2)]
 LARGE = SMALL + [(64, 11.0), (200, 17.0)]
 MANY = [(1500, 32.0)]
+DENSE = [(8, 4.2), (27, 6.0), (64, 6.5), (125, 9.0)]  # 55, 65, 120, 90 neighbours
 COND = {(0, 0): [0, 1, 2, 3, 4], (0, 1): [0, 2, 3], (1, 1): [1]}
 NONE = {(0, 0): [0, 1, 2], (0, 1): [], (1, 1): [0, 1, 2, 4]}
 
@@ -52,6 +54,10 @@ CASES = {
     "l12_n17": (spec(max_l=(12,), n_gauss=16, model_type=3), SMALL),
     "cond": (spec(n_type=2, max_l=(4, 2), model_type=3, cond=COND), LARGE),
     "cond_none": (spec(n_type=2, max_l=(2,), cond=NONE), LARGE),
+    "dense": (spec(max_l=(4,), n_gauss=6), DENSE),
+    "dense_alloy": (spec(n_type=3, max_l=(6,), n_gauss=3, model_type=3), DENSE),
+    "dense_pair": (spec(n_type=2, max_l=(), n_gauss=5), DENSE),
+    "tiles_beyond": (spec(n_type=4, max_l=(10,), n_gauss=19, max_p=1, model_type=3), SMALL),
     "order3_p3": (spec(n_type=3, max_l=(4, 2), n_gauss=1, max_p=3, model_type=3), SMALL),
     "pair": (spec(n_type=2, max_l=(), n_gauss=6), LARGE),
     "pair_many": (spec(n_type=2, max_l=(), n_gauss=5, cond=COND), MANY),
