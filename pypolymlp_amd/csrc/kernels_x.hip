@@ -184,9 +184,9 @@ __global__ void __launch_bounds__(NT) anlm_reg_kernel(ModelDev md, BatchDev bd,
 // angles, cos, exp: the matrix units take a fifth of the time), hence by waves
 // in flight: four a SIMD (128 registers; with the 144 the compiler took 0.24 ms)
 // and the angles and the cutoff function not in every wave (0.32 ms).
-// Register sums -> this: FP64, 32,000 atoms of 55 neighbours, 165 heads 0.77 ->
+// Register sums -> this: FP64, 32,000 atoms of 50 neighbours, 165 heads 0.77 ->
 // 0.20 ms; 1,024 alloy atoms, 1,350 heads 0.17 -> 0.056 ms; 54 atoms 41 -> 7 us;
-// 8,000 atoms, pair model 0.15 -> 0.05 ms; FP32, 20,480 alloy atoms 1.85 -> 0.39 ms.
+// 2,744 atoms of 232 neighbours, pair model 0.15 -> 0.05 ms; FP32, 20,480 alloy atoms 1.85 -> 0.39 ms.
 // ---------------------------------------------------------------------------
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef double doublex4 __attribute__((ext_vector_type(4)));

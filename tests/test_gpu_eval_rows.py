@@ -89,3 +89,20 @@ def test_eval_matches_rows(name, form, monkeypatch):
         assert np.abs(S[k] - y[rows]).max() <= 1e-11 * size[rows].max() + 1e-13
         assert np.abs(F[k].reshape(-1) - y[at:at + n]).max() <= 1e-11 * size[at:at + n].max() + 1e-13
         at += n
+
+
+@pytest.mark.parametrize("max_p,model_type", [(2, 4), (3, 3)])
+def test_fp32_energy_rows(max_p, model_type):
+    """Energy rows summed by quarters of the atoms, four at a time: atom counts
+    around those, two and three factors. FP32 features within 1e-5 of the sum
+    of their magnitudes (some 1e-6 per factor, three factors)."""
+    sp = spec(max_l=(2,), n_gauss=3, max_p=max_p, model_type=model_type)
+    sts = [structure(n, 3.1 * n ** (1 / 3), 1, n) for n in (1, 3, 4, 5, 15, 16, 17, 33, 64, 65)]
+    m = capi.Model(sp.as_dict())
+    b = capi.Batch(m, [s.axis for s in sts], [s.positions_cartesian for s in sts],
+                   [s.types for s in sts])
+    x64 = capi.features_x(m, b)[:len(sts)]
+    x32 = capi.features_x(m, b, capi.PLM_MIXED)[:len(sts)]
+    per_atom = np.abs(x64) / np.array([s.n_total for s in sts])[:, None]
+    size = per_atom.max(axis=0) * np.array([s.n_total for s in sts])[:, None]
+    assert np.all(np.abs(x32 - x64) <= 1e-5 * size)
