@@ -147,8 +147,9 @@ def eval_leg(steps: int, graph_steps: int, cpu: bool):
 
     Roofline of the dominant evaluation kernel, the half-pair loop
     (pair_lane_kernel): algorithmic
-    flops = 40 n_fn n_lm_half per half pair (radial functions, Y_lm and their
-    gradients, and the contraction with both atoms' prod_sum), against the
+    flops = 12 n_fn n_lm_half (the sums of f'_n S_n and f_n S_n over both atoms'
+    head sums) + 60 n_lm_half (Y_lm, its gradient and the force) + 40 n_fn
+    (radial functions) per half pair, against the
     vector peak of the precision it computes in (FP64 78.6, FP32 157.3 TFLOP/s)."""
     import tempfile
 
@@ -196,13 +197,14 @@ def eval_leg(steps: int, graph_steps: int, cpu: bool):
             f"{st.n_total / dt:.4g} atoms/s")
         ms_p, n_p = kern["eval_pair"]
         peak = FP64_PEAK_TFLOPS if name == "fp64" else FP32_PEAK_TFLOPS
-        ach = 40.0 * n_fn * n_lmh * n_half / (ms_p / n_p * 1e-3) / 1e12
+        flops = 12 * n_fn * n_lmh + 60 * n_lmh + 40 * n_fn
+        ach = float(flops) * n_half / (ms_p / n_p * 1e-3) / 1e12
         form = os.environ.get("PLM_EVAL_PAIR") or "lane"
         out[f"eval_roofline_{name}"] = {
             "bound": "valu", "unit": "TFLOP/s",
             "kernel": "pair_lane_kernel" if form == "lane" else "pair_rec_kernel",
             "achieved": ach, "peak": peak, "frac": ach / peak,
-            "work": f"40 n_fn n_lm_half = {40 * n_fn * n_lmh} flops per half pair x {n_half} "
+            "work": f"12 n_fn n_lm_half + 60 n_lm_half + 40 n_fn = {flops} flops per half pair x {n_half} "
                     "half pairs per launch"}
         del graph, batch
     e64, f64, s64 = res["fp64"]
