@@ -118,10 +118,15 @@ size_t poly_bytes(ModelHandle& m, const BatchHandle& b, int s0, int s1, bool fp6
     return n * (fp64 ? 8 : 4);
 }
 
-// LDS per workgroup of the factor-derivative kernel. Every pass walks all of
-// an atom's pairs with one thread per factor of the chunk, so the factors are
-// split into as few passes as the LDS holds, in chunks of equal size.
-constexpr size_t kDerivLds = 150 * 1024;
+// LDS per workgroup of the factor-derivative kernel: its loops wait for gathers,
+// so four workgroups a CU (kDerivLds each) walk an atom's pairs once per chunk of
+// factors rather than one workgroup once for all (66 factors, 54 atoms, FP64,
+// 89 KB: 4.55 ms per 10,800 atoms; in three chunks 2.31 ms; 128 alloy atoms, FP32
+// 2.42 -> 1.86 ms). Not below 16 factors, whose passes over the pairs are 16 threads
+// wide each, as long as the rows fit (kDerivLdsMax).
+constexpr size_t kDerivLdsMax = 150 * 1024;
+constexpr int kDerivFactors = 16;
+constexpr size_t kDerivLds = 38 * 1024;
 
 std::vector<long> poly_d_offsets(ModelHandle& m, const BatchHandle& b, int s0, int s1) {
     const PolyDev& pd = m.poly().dev;
@@ -164,11 +169,12 @@ void build_poly_rows(ModelHandle& m, BatchHandle& b, int s0, int s1, bool fp64, 
         ProfScope ps("poly_deriv", st);
         launch_poly_factor(st, fp64, m.md, pd, bd, a0, na, work.x.ptr, x_stride, work.xf.ptr,
                            work.m.ptr);
-        // factor chunks whose per-atom rows fit kDerivLds bytes of LDS
-        // (at most 128, so that the 256-thread workgroup has at least two
-        // threads per factor)
+        // factor chunks whose per-atom rows fit that LDS (at most 128, so that the
+        // 256-thread workgroup has at least two threads per factor), of equal size
+        const size_t row = (size_t)rd_max * elem;
         const int kc_max = std::max(
-            1, std::min({pd.K, 128, (int)(kDerivLds / ((size_t)rd_max * elem))}));
+            1, std::min({pd.K, 128, (int)(kDerivLdsMax / row),
+                         std::max(kDerivFactors, (int)(kDerivLds / row))}));
         const int passes = (pd.K + kc_max - 1) / kc_max;
         const int kc = (pd.K + passes - 1) / passes;
         if ((size_t)kc * rd_max * elem > 160 * 1024)
