@@ -216,44 +216,46 @@ __global__ void __launch_bounds__(kRowThreads) poly_rows_kernel(PolyDev pd, Batc
 }
 
 // Energy rows of the polynomial columns: X[row][c0 + c] = w sum_i prod_s x_{f_s}(i),
-// the raw sums into the scale sums.
-// Bound by the latency of its gathers: a wave per column run of 64 and quarter of
-// the atoms, four atoms' factors in flight. One thread per column over all atoms,
-// one after another, took 43 us per structure of 8-216 atoms and 2,178 columns
-// (FP32), this 6.6 us.
+// the raw sums into the scale sums. One lane per column. The atoms are added one
+// after another, each product rounded before its addition: the column scales
+// come from the variance of these sums, which magnifies a change of rounding by
+// the ratio of their mean to their spread, so another order of the FP32 sums
+// would give the mixed form other scales. Bound by the latency of the gathers:
+// kEnergyAtoms atoms' factors are in flight (ternary cells of 8-216 atoms, 2,178
+// columns, FP32: 44 us a launch with the factors fetched one by one, 8.5 us so).
+constexpr int kEnergyAtoms = 16;
+
 template <class T>
-__global__ void __launch_bounds__(256) poly_energy_kernel(PolyDev pd, BatchDev bd, int s_first,
-                                                          int atom_base, const T* __restrict__ XF,
-                                                          T* __restrict__ X, int ld, int row_base,
-                                                          const double* __restrict__ roww,
-                                                          double* __restrict__ xe_sum,
-                                                          double* __restrict__ xe_sq) {
-    __shared__ T part[4][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + lane;
+__global__ void __launch_bounds__(64) poly_energy_kernel(PolyDev pd, BatchDev bd, int s_first,
+                                                         int atom_base, const T* __restrict__ XF,
+                                                         T* __restrict__ X, int ld, int row_base,
+                                                         const double* __restrict__ roww,
+                                                         double* __restrict__ xe_sum,
+                                                         double* __restrict__ xe_sq) {
+#pragma clang fp contract(off)
+    const int c = blockIdx.x * 64 + threadIdx.x;
     const int s = s_first + blockIdx.y;
+    if (c >= pd.n_cols) return;
     const int a0 = bd.st_atom_off[s], nat = bd.st_atom_off[s + 1] - a0;
+    const int* ph = pd.col_phi + 3 * (size_t)c;
+    const int f0 = ph[0], f1 = ph[1], f2 = ph[2];
+    const T* xf = XF + (size_t)(a0 - atom_base) * pd.K;
     T e = T(0);
-    if (c < pd.n_cols) {
-        const int* ph = pd.col_phi + 3 * (size_t)c;
-        const int f0 = ph[0], f1 = ph[1], f2 = ph[2];
-        const T* xf = XF + (size_t)(a0 - atom_base) * pd.K;
-        for (int i = w; i < nat; i += 16) {
-            T u[4], v[4], t[4];
+    for (int i = 0; i < nat; i += kEnergyAtoms) {
+        // past the last atom: its factors again, not added
+        T u[kEnergyAtoms], v[kEnergyAtoms], t[kEnergyAtoms];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const T* x = xf + (size_t)min(i + 4 * q, nat - 1) * pd.K;
-                u[q] = x[f0], v[q] = x[f1], t[q] = x[max(f2, 0)];
-            }
+        for (int q = 0; q < kEnergyAtoms; ++q) {
+            const T* x = xf + (size_t)min(i + q, nat - 1) * pd.K;
+            u[q] = x[f0], v[q] = x[f1], t[q] = x[max(f2, 0)];
+        }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (i + 4 * q < nat) e += f2 >= 0 ? u[q] * v[q] * t[q] : u[q] * v[q];
+        for (int q = 0; q < kEnergyAtoms; ++q) {
+            T p = u[q] * v[q];
+            if (f2 >= 0) p = p * t[q];
+            if (i + q < nat) e = e + p;
         }
     }
-    part[w][lane] = e;
-    __syncthreads();
-    if (w != 0 || c >= pd.n_cols) return;
-    e = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     const int rb = bd.st_row_off[s] - row_base;
     const double wt = roww ? roww[rb] : 1.0;
     X[(size_t)rb * ld + pd.c0 + c] = T(wt * double(e));
@@ -287,7 +289,7 @@ static void poly_rows_t(hipStream_t st, const PolyDev& pd, const BatchDev& bd, i
                                                          reinterpret_cast<const T*>(Z), z_stride,
                                                          reinterpret_cast<T*>(X), ld, row_base,
                                                          roww);
-    poly_energy_kernel<T><<<dim3((pd.n_cols + 63) / 64, n_st), 256, 0, st>>>(
+    poly_energy_kernel<T><<<dim3((pd.n_cols + 63) / 64, n_st), 64, 0, st>>>(
         pd, bd, s_first, atom_base, reinterpret_cast<const T*>(XF), reinterpret_cast<T*>(X), ld,
         row_base, roww, xe_sum, xe_sq);
 }

@@ -93,8 +93,8 @@ def test_eval_matches_rows(name, form, monkeypatch):
 
 @pytest.mark.parametrize("max_p,model_type", [(2, 4), (3, 3)])
 def test_fp32_energy_rows(max_p, model_type):
-    """Energy rows summed by quarters of the atoms, four at a time: atom counts
-    around those, two and three factors. FP32 features within 1e-5 of the sum
+    """Energy rows with 16 atoms' factors in flight: atom counts around that,
+    two and three factors. FP32 features within 1e-5 of the sum
     of their magnitudes (some 1e-6 per factor, three factors)."""
     sp = spec(max_l=(2,), n_gauss=3, max_p=max_p, model_type=model_type)
     sts = [structure(n, 3.1 * n ** (1 / 3), 1, n) for n in (1, 3, 4, 5, 15, 16, 17, 33, 64, 65)]

@@ -1,0 +1,63 @@
+"""Energy rows of the mixed form are FP32 sums over the atoms in their order, each
+product rounded before it is added. Structures of separate dimers of several
+lengths: both atoms of a dimer have its FP32 pair features, half of what the
+linear columns of the dimer alone hold (a sum of two equal numbers, exact), so
+numpy adds the same products in the same order and every bit is known."""
+
+import numpy as np
+import pytest
+
+from pypolymlp_amd import capi
+from pypolymlp_amd.params import ModelSpec
+
+pytestmark = pytest.mark.gpu
+
+
+def dimers(n, seed):
+    """n displacements, as multiples of 2^-12 (differences of positions are exact)."""
+    d = np.random.default_rng(seed).normal(size=(n, 3))
+    length = np.linspace(1.7, 3.9, n)
+    return np.round(d / np.linalg.norm(d, axis=1)[:, None] * length[:, None] * 4096) / 4096
+
+
+def cell(d):
+    """Dimers on a grid of 16, none within the cutoff of another."""
+    side = int(np.ceil(len(d) ** (1 / 3)))
+    at = 16.0 * np.mgrid[0:side, 0:side, 0:side].reshape(3, -1).T[:len(d)] + 6.0
+    pos = np.stack([at, at + d], axis=1).reshape(-1, 3)
+    return np.diag(np.full(3, 16.0 * side)), np.ascontiguousarray(pos.T)
+
+
+# dimers a structure: one batch of the kernel's 16 atoms in flight and around it,
+# several batches, and a remainder of each size class
+@pytest.mark.parametrize("max_p", [2, 3])
+@pytest.mark.parametrize("sizes", [(1, 2, 7, 8, 9), (15, 16, 17, 33), (64, 65, 100)])
+def test_energy_rows_add_atoms_in_order(sizes, max_p):
+    spec = ModelSpec(n_type=1, cutoff=5.0, feature_type="pair", model_type=2, max_p=max_p,
+                     gtinv_order=0, gtinv_maxl=(), gaussian_params1=(1.0, 1.0, 1),
+                     gaussian_params2=(0.0, 4.0, 6))
+    m = capi.Model(spec.as_dict())
+    d = dimers(max(sizes), 3)
+
+    def rows(sets):
+        cells = [cell(v) for v in sets]
+        b = capi.Batch(m, [c[0] for c in cells], [c[1] for c in cells],
+                       [np.zeros(2 * len(v), dtype=int) for v in sets])
+        return capi.features_x(m, b, capi.PLM_MIXED)[:len(sets)]
+
+    alone = rows([d[k:k + 1] for k in range(len(d))])
+    n = 7
+    x = (alone[:, :n] / 2).astype(np.float32)
+    assert np.array_equal(2 * x.astype(np.float64), alone[:, :n])
+    cols = [(b, a) for a in range(n) for b in range(a + 1)]
+    if max_p == 3:
+        cols += [(c, b, a) for a in range(n) for b in range(a + 1) for c in range(b + 1)]
+    p = np.stack([x[:, c[0]] * x[:, c[1]] * (x[:, c[2]] if len(c) == 3 else np.float32(1))
+                  for c in cols], axis=1)
+    got = rows([d[:k] for k in sizes])[:, n:]
+    for g, k in zip(got, sizes):
+        want = np.zeros(len(cols), dtype=np.float32)
+        for q in range(k):
+            want = want + p[q]
+            want = want + p[q]
+        assert np.array_equal(g, want.astype(np.float64))
