@@ -134,7 +134,6 @@ def eval_cpu_baseline(model_yaml, st, steps=1):
     return out
 
 
-FP32_PEAK_TFLOPS = 157.3
 
 
 def eval_leg(steps: int, graph_steps: int, cpu: bool):
@@ -149,8 +148,8 @@ def eval_leg(steps: int, graph_steps: int, cpu: bool):
     (pair_lane_kernel): algorithmic
     flops = 12 n_fn n_lm_half (the sums of f'_n S_n and f_n S_n over both atoms'
     head sums) + 60 n_lm_half (Y_lm, its gradient and the force) + 40 n_fn
-    (radial functions) per half pair, against the
-    vector peak of the precision it computes in (FP64 78.6, FP32 157.3 TFLOP/s)."""
+    (radial functions) per half pair, against the FP64 vector peak (78.6
+    TFLOP/s): evaluations in the mixed form compute in FP64, too."""
     import tempfile
 
     from pypolymlp_amd import capi, datasets, mlp_dev
@@ -196,14 +195,13 @@ def eval_leg(steps: int, graph_steps: int, cpu: bool):
         log(f"eval graph {name}: {dt * 1e3:.2f} ms/step over {graph_steps} replays, "
             f"{st.n_total / dt:.4g} atoms/s")
         ms_p, n_p = kern["eval_pair"]
-        peak = FP64_PEAK_TFLOPS if name == "fp64" else FP32_PEAK_TFLOPS
         flops = 12 * n_fn * n_lmh + 60 * n_lmh + 40 * n_fn
         ach = float(flops) * n_half / (ms_p / n_p * 1e-3) / 1e12
         form = os.environ.get("PLM_EVAL_PAIR") or "lane"
         out[f"eval_roofline_{name}"] = {
             "bound": "valu", "unit": "TFLOP/s",
             "kernel": "pair_lane_kernel" if form == "lane" else "pair_rec_kernel",
-            "achieved": ach, "peak": peak, "frac": ach / peak,
+            "achieved": ach, "peak": FP64_PEAK_TFLOPS, "frac": ach / FP64_PEAK_TFLOPS,
             "work": f"12 n_fn n_lm_half + 60 n_lm_half + 40 n_fn = {flops} flops per half pair x {n_half} "
                     "half pairs per launch"}
         del graph, batch

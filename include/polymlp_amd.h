@@ -31,7 +31,9 @@ extern "C" {
 #define PLM_FP64 0  /* plain FP64 features, FP64 MFMA X^T X (the drop-in form) */
 #define PLM_MIXED 1 /* FP32 features; X^T X as the exact Gram of X quantised per
                      * (row chunk, column) to a shared exponent and three signed
-                     * 7-bit slices, on int8 MFMA with int32 sums combined in FP64 */
+                     * 7-bit slices, on int8 MFMA with int32 sums combined in FP64.
+                     * Evaluations compute in FP64 (in FP32 only for models whose
+                     * per-atom data fit a CU's LDS in FP32 and not in FP64) */
 #define PLM_MIXED64 2 /* FP64 features with the quantised int8 Gram of PLM_MIXED
                        * (X^T X accumulation; elsewhere the same as PLM_FP64) */
 
@@ -263,10 +265,11 @@ int plm_eval(plm_model* m, const double* axis, const double* pos_c, const int* t
  * harnesses that forbid hipMalloc): the same kernels and results as plm_eval,
  * with every device buffer (staged inputs, full and half neighbour lists,
  * order parameters, per-atom contractions, outputs) carved out of one
- * file-scope device array of 64 MiB per GPU, held until the process ends. It
+ * file-scope device array of 128 MiB per GPU, held until the process ends. It
  * calls no hipMalloc / hipFree. The model must already hold its coefficients
- * (plm_model_set_coeffs). A structure whose buffers exceed 64 MiB is refused
- * with PLM_ERR_ARG (about 6,000 atoms of a 1-type order-2 max_l 4 model).
+ * (plm_model_set_coeffs). A structure whose buffers exceed 64 MiB in the
+ * requested precision is refused with PLM_ERR_ARG (about 6,000 atoms of a
+ * 1-type order-2 max_l 4 model).
  * Calls on one GPU share the array: overlapping calls on the same GPU race. */
 int plm_eval_noalloc(plm_model* m, const double* axis, const double* pos_c, const int* types,
                      int n, int precision, double* energy, double* forces, double* stress);

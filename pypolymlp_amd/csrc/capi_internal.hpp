@@ -325,6 +325,12 @@ struct EvalGraph {
     EvalGraph& operator=(const EvalGraph&) = delete;
     ~EvalGraph();
 };
+// Whether an evaluation with this feature precision computes in FP64. The mixed
+// form does, too: its pair functions, sums and head sums in FP32 left energies
+// and stresses 1e-7 to 3e-5 off, and any other order of its sums moved them by
+// up to as much, while FP64 costs 1.0-1.4 times the time. FP32 remains for
+// models whose per-atom data fit the LDS in FP32 only.
+bool eval_in_fp64(const ModelHandle& m, bool fp64);
 void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, const int* hb_j,
                       const double* hb_d, int n_half, bool fp64, void* a_buf, double* e_at,
                       void* psf, double* part, double* out, size_t n_out, hipStream_t st);

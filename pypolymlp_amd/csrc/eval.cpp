@@ -313,6 +313,10 @@ void upload_potential(ModelHandle& m) {
     ++m.pot_version;
 }
 
+bool eval_in_fp64(const ModelHandle& m, bool fp64) {
+    return fp64 || (anlm_fits(m.md, true, m.max_noconj) && prodsum_fits(m.ed, true, m.max_nlm));
+}
+
 // Work buffers of one evaluation; out = [energies | forces (3 per atom) | stresses (6)].
 static void alloc_eval(const ModelHandle& m, const BatchHandle& b, bool fp64, DevBuf& a_buf,
                        DevBuf& e_at, DevBuf& psf, DevBuf& part, DevBuf& out, size_t& n_out) {
@@ -387,6 +391,7 @@ static void prepare_eval(ModelHandle& m, BatchHandle& b) {
 void eval_batch(ModelHandle& m, BatchHandle& b, bool fp64, double* energies, double* forces,
                 double* stresses) {
     prepare_eval(m, b);
+    fp64 = eval_in_fp64(m, fp64);
     hipStream_t st = device().stream;
     std::lock_guard<std::mutex> lock(m.eval_mutex);
     size_t n_out = 0;
@@ -405,6 +410,7 @@ void eval_graph_capture(EvalGraph& g) {
     ModelHandle& m = *g.m;
     BatchHandle& b = *g.b;
     prepare_eval(m, b);
+    g.fp64 = eval_in_fp64(m, g.fp64);
     hipStream_t st = device().stream;
     alloc_eval(m, b, g.fp64, g.a_buf, g.e_at, g.psf, g.part, g.out, g.n_out);
     // one eager pass first: kernel attributes are set and every buffer exists

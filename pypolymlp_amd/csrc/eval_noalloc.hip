@@ -23,7 +23,12 @@
 
 namespace plm {
 
-constexpr size_t kNoallocScratchBytes = size_t(64) << 20;  // 64 MiB per GPU
+// A structure is refused when its buffers in the requested precision (with two
+// head sums an atom and translation indices in both lists) exceed 64 MiB per
+// GPU. The array is twice that: the mixed form's order parameters and head sums
+// are FP64 (eval_in_fp64), at most twice what counts for them.
+constexpr size_t kNoallocLimit = size_t(64) << 20;
+constexpr size_t kNoallocScratchBytes = 2 * kNoallocLimit;
 constexpr int kNoallocMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kNoallocScratchBytes];
@@ -49,16 +54,17 @@ unsigned char* scratch_base() {
     return static_cast<unsigned char*>(g_scratch_dev[dev]);
 }
 
-// Bump allocator over the scratch array: offsets only, checked against the size.
+// Bump allocator over the scratch array: offsets only, checked against the limit.
 struct Arena {
     unsigned char* base;
+    size_t limit = kNoallocScratchBytes;
     size_t off = 0;
     void* take(size_t bytes) {
         off = (off + 255) & ~size_t(255);
-        if (bytes > kNoallocScratchBytes || off > kNoallocScratchBytes - bytes)
+        if (bytes > limit || off > limit - bytes)
             throw std::invalid_argument(
                 "structure too large for plm_eval_noalloc: needs more than " +
-                std::to_string(kNoallocScratchBytes >> 20) + " MiB of scratch");
+                std::to_string(kNoallocLimit >> 20) + " MiB of scratch");
         void* p = base + off;
         off += bytes;
         return p;
@@ -80,7 +86,9 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     hipStream_t st = device().stream;
     const double cutoff = m.host.input().cutoff;
     const double cut2 = cutoff * cutoff, tol = 1e-10, tol2 = tol * tol;
-    const int elem = fp64 ? 8 : 4;
+    const size_t elem_asked = fp64 ? 8 : 4;
+    fp64 = eval_in_fp64(m, fp64);
+    const size_t elem = fp64 ? 8 : 4;
 
     // host side: translations and search positions (NeighborCell)
     std::vector<double> trans, prev;
@@ -92,8 +100,28 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     const int tr_off[2] = {0, n_tr}, atom_off[2] = {0, n}, row_off[2] = {0, 7 + 3 * n};
     std::vector<int> zeros(n, 0);
 
+    // whether the structure is one to refuse: its buffers without the lists
+    // (before the GPU is touched), then with lists of mf and mh pairs
+    const size_t heads = (size_t)std::max(1, m.max_heads);
+    const size_t n_out = 1 + 3 * (size_t)n + 6;
+    unsigned char* const base = scratch_base();
+    auto check_limit = [&](bool lists, size_t mf, size_t mh) {
+        const size_t N = n, off = (N + 1) * 4, head_sums = N * heads * 2 * elem_asked;
+        Arena c{base, kNoallocLimit};
+        for (size_t bytes : {N * 4, N * 24, std::max<size_t>(trans.size(), 3) * 8, size_t(8), N * 4,
+                             size_t(8), size_t(8), N * 8})
+            c.take(bytes);
+        if (lists)
+            for (size_t bytes : {off, mf * 4, mf * 4, mf * 24, off, mh * 4, mh * 4, mh * 24})
+                c.take(bytes);
+        for (size_t bytes : {N * m.max_nlm * 2 * elem_asked, head_sums, head_sums, n_out * 8})
+            c.take(bytes);
+        if (!lists) c.take(2 * off);
+    };
+    check_limit(false, 0, 0);
+
     // fixed part: inputs and the two count arrays
-    Arena ar{scratch_base()};
+    Arena ar{base};
     int* d_types = (int*)ar.take((size_t)n * 4);
     double* d_pos = (double*)ar.take((size_t)n * 24);
     double* d_trans = (double*)ar.take(std::max<size_t>(trans.size(), 3) * 8);
@@ -102,19 +130,7 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
     int* d_atom_off = (int*)ar.take(8);
     int* d_row_off = (int*)ar.take(8);
     int* d_cnt = (int*)ar.take((size_t)n * 8);  // full counts, then half counts
-    // the per-atom work buffers are sized before any neighbour is counted, so
-    // that an oversized structure is refused before the GPU is touched
-    const size_t heads = (size_t)std::max(1, m.max_heads);
-    const size_t n_out = 1 + 3 * (size_t)n + 6;
     const size_t fixed_end = ar.off;
-    {
-        Arena probe = ar;
-        probe.take((size_t)n * m.max_nlm * 2 * elem);
-        probe.take((size_t)n * 8);
-        probe.take((size_t)n * heads * 2 * elem);
-        probe.take(n_out * 8);
-        probe.take((size_t)(n + 1) * 8);
-    }
     auto up = [&](void* dst, const void* src, size_t bytes) {
         check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st), "copy");
     };
@@ -137,6 +153,7 @@ void eval_single_noalloc(ModelHandle& m, const double* axis, const double* pos_c
         off_h[i + 1] = off_h[i] + c[n + i];
     }
     const size_t Mf = std::max(off_f[n], 1), Mh = std::max(off_h[n], 1);
+    check_limit(true, Mf, Mh);
 
     ar.off = fixed_end;
     int* d_nb_off = (int*)ar.take((size_t)(n + 1) * 4);

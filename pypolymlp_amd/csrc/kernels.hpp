@@ -48,6 +48,8 @@ void launch_half_list(hipStream_t st, int n, double tol, const int* nb_off, cons
                       double* hb_d);
 
 size_t anlm_smem(const ModelDev& md, int elem, int nthreads, int max_noconj);
+// whether an atom's order parameters fit the LDS of a form of launch_anlm
+bool anlm_fits(const ModelDev& md, bool fp64, int max_noconj);
 void launch_anlm(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd, void* a_full,
                  int a_stride, int atom0, int n_atoms, int max_noconj, int negate = 0);
 
@@ -140,6 +142,8 @@ void launch_xrows(hipStream_t st, bool fp64, const ModelDev& md, const ColumnsDe
                   const PairRec& R, void* X, const double* roww, double* xe_sum, double* xe_sq);
 
 struct EvalDev;
+// whether an atom's data fit the LDS of launch_prodsum
+bool prodsum_fits(const EvalDev& ed, bool fp64, int a_stride);
 // prod_sum_f per atom and head into ps_f, the atoms' energies into e_at
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
                     const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,

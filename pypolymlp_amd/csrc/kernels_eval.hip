@@ -645,14 +645,24 @@ __global__ void __launch_bounds__(256) eval_sum_kernel(BatchDev bd, int n_pairs,
     }
 }
 
+static size_t prodsum_smem(const EvalDev& ed, int a_stride, size_t elem) {
+    return (size_t)ed.poly_max * sizeof(double2) + (size_t)(a_stride + 1) * 2 * elem +
+           (size_t)(ed.poly_max + 4) * 2 * elem + (size_t)(ed.poly_max + 1) * elem;
+}
+
+// dynamic LDS of a workgroup, next to the waves' energies
+static constexpr size_t kProdsumLds = 160 * 1024 - 64;
+
+bool prodsum_fits(const EvalDev& ed, bool fp64, int a_stride) {
+    return prodsum_smem(ed, a_stride, fp64 ? 8 : 4) <= kProdsumLds;
+}
+
 template <class T, int NL>
 void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
                       const void* a_full, int a_stride, void* ps_f, int ps_stride, double* e_at,
                       int pair_model) {
-    const size_t sm = (size_t)ed.poly_max * sizeof(double2) +
-                      (size_t)(a_stride + 1) * 2 * sizeof(T) + (size_t)(ed.poly_max + 4) * 2 * sizeof(T) +
-                      (size_t)(ed.poly_max + 1) * sizeof(T);
-    if (sm > 160 * 1024) throw std::invalid_argument("per-atom evaluation data exceed LDS");
+    const size_t sm = prodsum_smem(ed, a_stride, sizeof(T));
+    if (sm > kProdsumLds) throw std::invalid_argument("per-atom evaluation data exceed LDS");
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
               "prodsum shared memory");

@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <stdexcept>
+#include <type_traits>
 
 #include "device_math.hpp"
 #include "device_tables.hpp"
@@ -177,64 +178,32 @@ __global__ void __launch_bounds__(NT) anlm_reg_kernel(ModelDev md, BatchDev bd,
 // neighbours, 64 at a time. A lane takes a pair; one or two waves take the
 // columns m of Y (recurrences unrolled to LB, so their square roots are
 // constants; the form above takes them, and a division each, per pair), the
-// others the radial functions; both go to LDS as [row][pair] (pitch 66 doubles or
-// 68 floats: the 16 rows x 4 pairs of an MFMA operand are then on banks of
-// their own), and 16 x 16 x 4 MFMA tiles, dealt to the waves, Q at most each,
-// add them up in registers. Bound by the FP64 functions of each pair (distance,
+// others the radial functions; both go to LDS as [row][pair] (pitch 66: the 16
+// rows x 4 pairs of an MFMA operand are then on banks of their own), and 16 x 16
+// x 4 MFMA tiles, dealt to the waves, Q at most each, add them up in registers.
+// Bound by the functions of each pair (distance,
 // angles, cos, exp: the matrix units take a fifth of the time), hence by waves
 // in flight: four a SIMD (128 registers; with the 144 the compiler took 0.24 ms)
 // and the angles and the cutoff function not in every wave (0.32 ms).
-// Register sums -> this: FP64, 32,000 atoms of 50 neighbours, 165 heads 0.77 ->
-// 0.20 ms; 1,024 alloy atoms, 1,350 heads 0.17 -> 0.056 ms; 54 atoms 41 -> 7 us;
-// 2,744 atoms of 232 neighbours, pair model 0.15 -> 0.05 ms; FP32, 20,480 alloy atoms 1.85 -> 0.39 ms.
+// Register sums -> this: 32,000 atoms of 50 neighbours, 165 heads 0.77 -> 0.20
+// ms; 1,024 alloy atoms, 1,350 heads 0.17 -> 0.056 ms; 54 atoms 41 -> 7 us; 2,744
+// atoms of 232 neighbours, pair model 0.15 -> 0.05 ms. FP64 only: an evaluation
+// in FP32 (models past the LDS of the FP64 one) takes the forms above.
 // ---------------------------------------------------------------------------
-typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kAnlmPitch = 66;
 typedef double doublex4 __attribute__((ext_vector_type(4)));
-template <class T> struct AnlmTile;
-template <> struct AnlmTile<float> {
-    using acc = floatx4;
-    static constexpr int pitch = 68;
-    static __device__ acc mfma(float a, float b, acc c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
-};
-template <> struct AnlmTile<double> {
-    using acc = doublex4;
-    static constexpr int pitch = 66;
-    static __device__ acc mfma(double a, double b, acc c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
-};
 
-// cos(pi r / rc) and (cos phi, sin phi): FP32 by the expressions of the forms
-// above, whose rounding is most of the error of its energies; FP64 (1e-16 apart)
-// without the reduction of large arguments, the scaling of hypot and one division
-__device__ __forceinline__ float cutoff_cos(float r, float rc) {
-    return cos(MathConst<float>::pi / rc * r);
-}
-__device__ __forceinline__ double cutoff_cos(double r, double rc) { return cospi(r / rc); }
-__device__ __forceinline__ void phi_unit(float x, float y, float& cp, float& sp) {
-    const float rho = dhypot(x, y);
-    if (rho > 0.f) cp = x / rho, sp = y / rho;
-}
-__device__ __forceinline__ void phi_unit(double x, double y, double& cp, double& sp) {
-    const double rho = sqrt(x * x + y * y);
-    if (rho > 0.0) {
-        const double inv = 1.0 / rho;
-        cp = x * inv, sp = y * inv;
-    }
-}
+// row of a lane's output element v of a 16 x 16 tile
+__device__ __forceinline__ int anlm_row(int lane, int v) { return (lane >> 4) + 4 * v; }
 
-template <class T, int LB, int Q>
+template <int LB, int Q>
 __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev md, BatchDev bd,
-                                                        Cpx<T>* __restrict__ a_full, int a_stride,
-                                                        int atom0, int negate) {
+                                                        Cpx<double>* __restrict__ a_full,
+                                                        int a_stride, int atom0, int negate) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    using M = AnlmTile<T>;
+    using T = double;
     using C = MathConst<T>;
-    constexpr int P = M::pitch;
+    constexpr int P = kAnlmPitch;
     const int nfn = md.n_fn, ncol = 2 * max(1, md.n_lmh);
     T* F = reinterpret_cast<T*>(smem_raw);  // [n_fn][P]
     T* Y = F + (size_t)nfn * P;             // [ncol][P]
@@ -251,9 +220,9 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
     // waves on Y's columns, the others take the radial functions
     constexpr int NA = LB <= 4 ? 1 : 2;
     const int na = lmax < 0 ? 0 : NA;
-    typename M::acc acc[Q];
+    doublex4 acc[Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q] = typename M::acc{T(0), T(0), T(0), T(0)};
+    for (int q = 0; q < Q; ++q) acc[q] = doublex4{0.0, 0.0, 0.0, 0.0};
     const int p0 = bd.nb_off[i], p1 = bd.nb_off[i + 1];
     for (int c0 = p0; c0 < p1; c0 += 64) {
         const int np = min(64, p1 - c0);
@@ -274,7 +243,7 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
             const int tp = md.tp_of[t1 * md.n_type + t2];
             const int cnt = on ? md.rad_count[tp] : 0;
             const double* rp = md.rad + (size_t)tp * nfn * 2;
-            const T fc = T(0.5) * (cutoff_cos(T(dis), T(md.cutoff)) + T(1));
+            const T fc = T(0.5) * (cospi(dis / md.cutoff) + T(1));
             for (int n = w - na; n < nfn; n += 4 - na) {
                 const T beta = T(rp[2 * n]), x = T(dis) - T(rp[2 * n + 1]);
                 const T f = dexp(-beta * x * x) * fc;
@@ -285,7 +254,11 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
             const T x = T(dx), y = T(dy), z = T(dz), r = T(dis);
             const T ct_ = on ? z / r : T(1);
             T cp = T(1), sp = T(0);
-            phi_unit(x, y, cp, sp);
+            const T rho = sqrt(x * x + y * y);
+            if (rho > T(0)) {
+                const T inv = T(1) / rho;
+                cp = x * inv, sp = y * inv;
+            }
             const T st = dsqrt(T(1) - ct_ * ct_);
             T c = T(1), s = T(0);  // cos, sin (m phi) by the Chebyshev recurrence
             T c1 = T(1), c2 = cp, s1 = T(0), s2 = -sp, pmm = C::sqrt_inv_2pi;
@@ -343,7 +316,8 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
                     fa[u] = gu == g ? fa[u] : T(0);
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) acc[q] = M::mfma(fa[u], fb[u], acc[q]);
+                for (int u = 0; u < 4; ++u)
+                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u], fb[u], acc[q], 0, 0, 0);
             }
         }
     }
@@ -357,7 +331,7 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
         const int col = 16 * tcol + (lane & 15);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int n = 16 * tr + M::row(lane, v);
+            const int n = 16 * tr + anlm_row(lane, v);
             if (n < nfn && col < ncol) sums[((size_t)g * nfn + n) * ncol + col] = acc[q][v];
         }
     }
@@ -371,35 +345,49 @@ __global__ void __launch_bounds__(256, Q <= 4 ? 4 : 1) anlm_mfma_kernel(ModelDev
     }
 }
 
-// true: launched; false: the model has Y columns past the unrolled ones, more
-// tiles than four waves hold in registers (16 each) or rows past a CU's LDS, and
-// the forms with sums per head below take it. Where it fits it is the faster
-// one at every size tried (54 to 32,000 atoms, above).
-template <class T>
-bool launch_anlm_mfma(hipStream_t st, const ModelDev& md, const BatchDev& bd, void* a_full,
-                      int a_stride, int atom0, int n_atoms, int negate) {
+static size_t anlm_mfma_smem(const ModelDev& md) {
     const int ncol = 2 * std::max(1, md.n_lmh);
-    const int tiles = md.n_type * ((md.n_fn + 15) / 16) * ((ncol + 15) / 16);
-    const size_t sm = std::max((size_t)(md.n_fn + ncol) * AnlmTile<T>::pitch,
-                               (size_t)md.n_type * md.n_fn * ncol) * sizeof(T);
-    if (md.max_l > 12 || tiles > 4 * 16 || sm > 156 * 1024) return false;
+    return std::max((size_t)(md.n_fn + ncol) * kAnlmPitch, (size_t)md.n_type * md.n_fn * ncol) *
+           sizeof(double);
+}
+
+static int anlm_mfma_tiles(const ModelDev& md) {
+    return md.n_type * ((md.n_fn + 15) / 16) * ((2 * std::max(1, md.n_lmh) + 15) / 16);
+}
+
+// false: the model has Y columns past the unrolled ones, more tiles than four
+// waves hold in registers (16 each) or rows past a CU's LDS, and the forms with
+// sums per head below take it. Where it fits it is the faster one at every size
+// tried (54 to 32,000 atoms, above).
+static bool anlm_mfma_fits(const ModelDev& md) {
+    return !getenv("PLM_ANLM_SHAPE") && md.max_l <= 12 && anlm_mfma_tiles(md) <= 4 * 16 &&
+           anlm_mfma_smem(md) <= 156 * 1024;
+}
+
+static void launch_anlm_mfma(hipStream_t st, const ModelDev& md, const BatchDev& bd, void* a_full,
+                      int a_stride, int atom0, int n_atoms, int negate) {
+    const size_t sm = anlm_mfma_smem(md);
     auto go = [&](auto kernel) {
         check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
                   "anlm shared memory");
-        kernel<<<n_atoms, 256, sm, st>>>(md, bd, reinterpret_cast<Cpx<T>*>(a_full), a_stride,
+        kernel<<<n_atoms, 256, sm, st>>>(md, bd, reinterpret_cast<Cpx<double>*>(a_full), a_stride,
                                          atom0, negate);
     };
-    const int q = (tiles + 3) / 4;
-    if (md.max_l <= 4 && q <= 4) go(&anlm_mfma_kernel<T, 4, 4>);
-    else if (md.max_l <= 8 && q <= 4) go(&anlm_mfma_kernel<T, 8, 4>);
-    else go(&anlm_mfma_kernel<T, 12, 16>);
-    return true;
+    const int q = (anlm_mfma_tiles(md) + 3) / 4;
+    if (md.max_l <= 4 && q <= 4) go(&anlm_mfma_kernel<4, 4>);
+    else if (md.max_l <= 8 && q <= 4) go(&anlm_mfma_kernel<8, 4>);
+    else go(&anlm_mfma_kernel<12, 16>);
 }
 
 size_t anlm_smem(const ModelDev& md, int elem, int nthreads, int max_noconj) {
     const PairLayout<double> L(md.n_fn, md.n_lmh, false);
     return (size_t)nthreads * L.stride * elem + (size_t)max_noconj * 2 * elem;
+}
+
+bool anlm_fits(const ModelDev& md, bool fp64, int max_noconj) {
+    return (fp64 && anlm_mfma_fits(md)) ||
+           anlm_smem(md, fp64 ? 8 : 4, kAnlmPairs, max_noconj) <= 160 * 1024;
 }
 
 template <class T, int Q, int NT>
@@ -422,9 +410,10 @@ void launch_anlm_reg(hipStream_t st, const ModelDev& md, const BatchDev& bd, voi
 template <class T>
 void launch_anlm_t(hipStream_t st, const ModelDev& md, const BatchDev& bd, void* a_full,
                    int a_stride, int atom0, int n_atoms, int max_noconj, int negate) {
-    if (!getenv("PLM_ANLM_SHAPE") &&
-        launch_anlm_mfma<T>(st, md, bd, a_full, a_stride, atom0, n_atoms, negate))
+    if (std::is_same<T, double>::value && anlm_mfma_fits(md)) {
+        launch_anlm_mfma(st, md, bd, a_full, a_stride, atom0, n_atoms, negate);
         return;
+    }
     const int B = 64;
     const size_t sm = anlm_smem(md, sizeof(T), kAnlmPairs, max_noconj);
     if (const char* e = getenv("PLM_ANLM_SHAPE")) {
