@@ -192,43 +192,23 @@ int plm_api_sum_of_prod(plm_model* mp, int type, const double* anlm_re, const do
         OneAtom one(m, type, anlm_re, anlm_im, fp64, st);
         const int elem = fp64 ? 8 : 4;
         const int ps = std::max(1, m.max_heads);
-        DevBuf pe, pf;
+        DevBuf pe, pf, e;
         pe.alloc((size_t)ps * 2 * elem);
         pf.alloc((size_t)ps * 2 * elem);
-        // the folded terms of each head, in the potential's order
-        const auto pot = m.host.head_terms(type);
-        const int nh = (int)pot.size();
-        const auto& T = m.host.type(type);
-        std::vector<int> off(nh + 1, 0);
-        std::vector<int4> key;
-        std::vector<double2> coeff;
-        auto k16 = [](const std::vector<int>& v, size_t q) -> unsigned {
-            if (q >= v.size()) return 0xffffu;
-            if (v[q] >= 0xffff) throw std::invalid_argument("evaluation table index exceeds 16 bits");
-            return (unsigned)v[q];
-        };
-        for (int h = 0; h < nh; ++h) {
-            for (const auto& p : pot[h]) {
-                const auto& d = T.prod_deriv[p.prod];
-                const auto& x = T.prod_features[p.prod_features];
-                if (d.size() > 3 || x.size() > 2) throw std::invalid_argument("term order too high");
-                key.push_back(int4{(int)(k16(d, 0) | k16(d, 1) << 16), (int)k16(d, 2),
-                                   (int)(k16(x, 0) | k16(x, 1) << 16), 0});
-                coeff.push_back(double2{p.coeff_e, p.coeff_f});
-            }
-            off[h + 1] = (int)key.size();
-        }
-        DevBuf d_off, d_key, d_c;
-        upload(d_off, off.data(), off.size() * 4, st);
-        upload(d_key, key.data(), key.size() * sizeof(int4), st);
-        upload(d_c, coeff.data(), coeff.size() * sizeof(double2), st);
-        launch_head_terms(st, fp64, m.md, one.bd, one.a.ptr, nh, (const int*)d_off.ptr,
-                          (const int4*)d_key.ptr, (const double2*)d_c.ptr, m.max_lin, pe.ptr,
-                          pf.ptr);
+        e.alloc(8);
+        launch_prodsum(st, fp64, m.md, m.ed, one.bd, one.a.ptr, m.max_nlm, pf.ptr, pe.ptr, ps,
+                       (double*)e.ptr, 0);
         check_hip(hipGetLastError(), "prodsum launch");
-        for (auto [dst, buf] : {std::pair<double*, const DevBuf*>{prod_e, &pe}, {prod_f, &pf}})
-            if (dst) download_cpx(dst, *buf, (size_t)nh, fp64, st);
-        check_hip(hipStreamSynchronize(st), "sync");  // the host tables go out of scope
+        // the sums are stored by head position; returned in the potential's order
+        const int nh = m.ed.t[type].n_heads;
+        const std::vector<int>& rank = m.head_rank.at(type);
+        std::vector<double> tmp(2 * (size_t)nh);
+        for (auto [dst, buf] : {std::pair<double*, const DevBuf*>{prod_e, &pe}, {prod_f, &pf}}) {
+            if (!dst) continue;
+            download_cpx(tmp.data(), *buf, (size_t)nh, fp64, st);
+            for (int k = 0; k < nh; ++k)
+                dst[2 * k] = tmp[2 * (size_t)rank[k]], dst[2 * k + 1] = tmp[2 * (size_t)rank[k] + 1];
+        }
     });
 }
 

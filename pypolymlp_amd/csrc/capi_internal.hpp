@@ -101,7 +101,7 @@ struct ModelHandle {
     bool pot_uploaded = false;
     unsigned pot_version = 0;  // counts uploads of the potential tables
     EvalDev ed{};
-    int max_heads = 0, max_lin = 0;
+    int max_heads = 0;
     // per type, the position of each head (in the potential's order) in the
     // per-atom head sums, which follow the half-pair loop's order
     std::vector<std::vector<int>> head_rank;

@@ -1,5 +1,7 @@
-// Evaluation (PolymlpEval) orchestration: potential tables, half neighbour
-// list, order parameters, per-atom prod_sum and the half-pair loop.
+// Evaluation (PolymlpEval) orchestration: potential tables (Potential,
+// polymlp_potential.cpp:25-156; the factor 2 of polymlp_eval.cpp:12-20 is in the
+// contraction), half neighbour list, order parameters, per-atom prod_sum and the
+// half-pair loop.
 #include <algorithm>
 #include <array>
 #include <cstdlib>
@@ -19,7 +21,7 @@ void upload_potential(ModelHandle& m) {
     m.pot_store.bufs.clear();
     const int nt = M.n_type(), ntp = M.n_tp();
     const bool gt = M.input().gtinv;
-    m.max_heads = 0, m.max_lin = 0;
+    m.max_heads = 0;
     m.ed.value_max = std::max(1, m.v_maxf), m.ed.term_max = 1;
     m.ed.poly_max = 0, m.ed.rows_max = 0;
     // The heads of each type in the order of the half-pair loop: grouped by type
@@ -83,7 +85,6 @@ void upload_potential(ModelHandle& m) {
         EvalTypeDev& E = m.ed.t[t];
         E.n_heads = (int)order[t].size();
         m.max_heads = std::max(m.max_heads, E.n_heads);
-        m.max_lin = std::max(m.max_lin, (int)T.features.size());
         // per type pair its heads; hi and hj are head positions of atoms i and j
         const int nkey = m.md.n_lmh;
         std::vector<int> hoff(ntp + 1, 0), nid, ylm, hi, hj;
@@ -349,7 +350,7 @@ void enqueue_eval_dev(ModelHandle& m, const BatchDev& bd, const int* hb_off, con
     check_hip(hipGetLastError(), "eval anlm launch");
     {
         ProfScope ps("eval_prodsum", st);
-        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, psf,
+        launch_prodsum(st, fp64, m.md, m.ed, bd, a_buf, m.max_nlm, psf, nullptr,
                        std::max(1, m.max_heads), e_at, pair_model);
     }
     check_hip(hipGetLastError(), "prodsum launch");

@@ -144,16 +144,11 @@ void launch_xrows(hipStream_t st, bool fp64, const ModelDev& md, const ColumnsDe
 struct EvalDev;
 // whether an atom's data fit the LDS of launch_prodsum
 bool prodsum_fits(const EvalDev& ed, bool fp64, int a_stride);
-// prod_sum_f per atom and head into ps_f, the atoms' energies into e_at
+// prod_sum_f per atom and head (by position) into ps_f, prod_sum_e into ps_e
+// unless it is null, the atoms' energies into e_at
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
-                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,
+                    const BatchDev& bd, const void* a_full, int a_stride, void* ps_f, void* ps_e,
                     int ps_stride, double* e_at, int pair_model);
-// prod_sum_e and prod_sum_f of one atom from the folded potential's terms of each
-// head (off [n_heads + 1]; keys (pd0 | pd1 << 16, pd2, pf0 | pf1 << 16, 0), 0xffff:
-// none; coefficients (e, f))
-void launch_head_terms(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd,
-                       const void* a, int n_heads, const int* off, const int4* key,
-                       const double2* coeff, int max_lin, void* ps_e, void* ps_f);
 // x[0, n) = 0 by a kernel (a graph of it replays correctly; a memset node is avoided)
 void launch_fill_zero(hipStream_t st, double* x, size_t n);
 // half-pair loop over the n_half pairs of the half list, which bd carries as its

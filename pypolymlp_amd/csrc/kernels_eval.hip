@@ -78,8 +78,8 @@ template <class T, int NL>
 __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, BatchDev bd,
                                                      const Cpx<T>* __restrict__ a_full,
                                                      int a_stride, Cpx<T>* __restrict__ ps_f,
-                                                     int ps_stride, double* __restrict__ e_at,
-                                                     int pair_model) {
+                                                     Cpx<T>* __restrict__ ps_e, int ps_stride,
+                                                     double* __restrict__ e_at, int pair_model) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ double e_part[NL / 64];
     const int i = blockIdx.x;
@@ -167,6 +167,7 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
         }
         if (h >= 0) {
             o[h] = {scale * vr, scale * vi};
+            if (ps_e) ps_e[(size_t)i * ps_stride + h] = {scale * er, scale * ei};
             const int ha = E.hd_a[h];  // the head's order parameter, bit 30: m = 0
             const Cpx<T> ac = a[ha & 0x3fffffff];
             const double v = double(er) * double(ac.re) - double(ei) * double(ac.im);
@@ -179,56 +180,6 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
     if (threadIdx.x == 0) {
         for (int w = 1; w < NW; ++w) e_sum += e_part[w];
         e_at[i] = double(scale) * e_sum;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// prod_sum_e and prod_sum_f of one atom's heads from the folded potential's
-// terms, coeff_{e,f} * prod_features * prod_anlm (plm_api_sum_of_prod).
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int key16(unsigned k) { return k == 0xffffu ? -1 : (int)k; }
-
-template <class T>
-__global__ void __launch_bounds__(64) head_terms_kernel(ModelDev md, BatchDev bd,
-                                                        const Cpx<T>* __restrict__ a, int n_heads,
-                                                        const int* __restrict__ off,
-                                                        const int4* __restrict__ key,
-                                                        const double2* __restrict__ coeff,
-                                                        Cpx<T>* __restrict__ ps_e,
-                                                        Cpx<T>* __restrict__ ps_f) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    T* xs = reinterpret_cast<T*>(smem_raw);
-    const TypeDev& TT = md.t[bd.types[0]];
-    for (int f = threadIdx.x; f < TT.n_lin; f += 64) {
-        T v = T(0);
-        for (int e = TT.fv_off[f]; e < TT.fv_off[f + 1]; ++e) {
-            Cpx<T> pr = {T(1), T(0)};
-            const int* keys = TT.fv_keys + 4 * (size_t)e;
-            for (int k = 0; k < 4 && keys[k] >= 0; ++k) pr = cmul(pr, a[keys[k]]);
-            if (TT.fv_skip && fabs(pr.re) <= T(1e-20)) continue;
-            v += T(TT.fv_coeff[e]) * pr.re;
-        }
-        xs[f] = v;
-    }
-    __syncthreads();
-    for (int h = threadIdx.x; h < n_heads; h += 64) {
-        T er = T(0), ei = T(0), fr = T(0), fi = T(0);
-        for (int e = off[h]; e < off[h + 1]; ++e) {
-            const int4 k = key[e];
-            const int pd[3] = {key16(k.x & 0xffff), key16((unsigned)k.x >> 16), key16(k.y & 0xffff)};
-            const int pf[2] = {key16(k.z & 0xffff), key16((unsigned)k.z >> 16)};
-            T fval = T(1);
-            for (int q = 0; q < 2; ++q)
-                if (pf[q] >= 0) fval *= xs[pf[q]];
-            Cpx<T> pr = {T(1), T(0)};
-            for (int q = 0; q < 3; ++q)
-                if (pd[q] >= 0) pr = cmul(pr, a[pd[q]]);
-            const T se = fval * T(coeff[e].x), sf = fval * T(coeff[e].y);
-            er += pr.re * se, ei += pr.im * se;
-            fr += pr.re * sf, fi += pr.im * sf;
-        }
-        ps_e[h] = {er, ei};
-        ps_f[h] = {fr, fi};
     }
 }
 
@@ -659,8 +610,8 @@ bool prodsum_fits(const EvalDev& ed, bool fp64, int a_stride) {
 
 template <class T, int NL>
 void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, const BatchDev& bd,
-                      const void* a_full, int a_stride, void* ps_f, int ps_stride, double* e_at,
-                      int pair_model) {
+                      const void* a_full, int a_stride, void* ps_f, void* ps_e, int ps_stride,
+                      double* e_at, int pair_model) {
     const size_t sm = prodsum_smem(ed, a_stride, sizeof(T));
     if (sm > kProdsumLds) throw std::invalid_argument("per-atom evaluation data exceed LDS");
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&prodsum_kernel<T, NL>),
@@ -668,7 +619,8 @@ void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, con
               "prodsum shared memory");
     prodsum_kernel<T, NL><<<bd.n_atoms_total, NL, sm, st>>>(
         md, ed, bd, reinterpret_cast<const Cpx<T>*>(a_full), a_stride,
-        reinterpret_cast<Cpx<T>*>(ps_f), ps_stride, e_at, pair_model);
+        reinterpret_cast<Cpx<T>*>(ps_f), reinterpret_cast<Cpx<T>*>(ps_e), ps_stride, e_at,
+        pair_model);
 }
 
 // Four waves an atom where its table rows are more than 128 or the atoms do
@@ -678,7 +630,7 @@ void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, con
 // PLM_PRODSUM_LANES=64|256 forces one form.
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
                     const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,
-                    int ps_stride, double* e_at, int pair_model) {
+                    void* ps_e, int ps_stride, double* e_at, int pair_model) {
     bool four = ed.rows_max > 128 || bd.n_atoms_total < 8192;
     if (const char* e = std::getenv("PLM_PRODSUM_LANES")) {
         if (!std::strcmp(e, "64")) four = false;
@@ -686,41 +638,17 @@ void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev
         else throw std::invalid_argument("PLM_PRODSUM_LANES must be 64 or 256");
     }
     if (fp64 && four)
-        launch_prodsum_t<double, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
-                                      pair_model);
+        launch_prodsum_t<double, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_e, ps_stride,
+                                      e_at, pair_model);
     else if (fp64)
-        launch_prodsum_t<double, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
-                                     pair_model);
+        launch_prodsum_t<double, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_e, ps_stride,
+                                     e_at, pair_model);
     else if (four)
-        launch_prodsum_t<float, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
-                                     pair_model);
+        launch_prodsum_t<float, 256>(st, md, ed, bd, a_full, a_stride, ps_f, ps_e, ps_stride,
+                                     e_at, pair_model);
     else
-        launch_prodsum_t<float, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_stride, e_at,
-                                    pair_model);
-}
-
-void launch_head_terms(hipStream_t st, bool fp64, const ModelDev& md, const BatchDev& bd,
-                       const void* a, int n_heads, const int* off, const int4* key,
-                       const double2* coeff, int max_lin, void* ps_e, void* ps_f) {
-    const size_t sm = (size_t)std::max(1, max_lin) * (fp64 ? 8 : 4);
-    if (sm > 160 * 1024) throw std::invalid_argument("per-atom evaluation data exceed LDS");
-    if (fp64) {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&head_terms_kernel<double>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
-                  "head terms shared memory");
-        head_terms_kernel<double><<<1, 64, sm, st>>>(md, bd, static_cast<const Cpx<double>*>(a),
-                                                     n_heads, off, key, coeff,
-                                                     static_cast<Cpx<double>*>(ps_e),
-                                                     static_cast<Cpx<double>*>(ps_f));
-    } else {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(&head_terms_kernel<float>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm),
-                  "head terms shared memory");
-        head_terms_kernel<float><<<1, 64, sm, st>>>(md, bd, static_cast<const Cpx<float>*>(a),
-                                                    n_heads, off, key, coeff,
-                                                    static_cast<Cpx<float>*>(ps_e),
-                                                    static_cast<Cpx<float>*>(ps_f));
-    }
+        launch_prodsum_t<float, 64>(st, md, ed, bd, a_full, a_stride, ps_f, ps_e, ps_stride,
+                                    e_at, pair_model);
 }
 
 template <class T>

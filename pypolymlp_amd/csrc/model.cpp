@@ -386,10 +386,6 @@ void Model::set_poly_tables() {
         for (int i : comb3_idx_[t])
             T.poly.push_back(
                 {b3 + i, {map1.at(comb3_[i][0]), map1.at(comb3_[i][1]), map1.at(comb3_[i][2])}});
-        std::set<std::vector<int>> uniq;
-        for (const auto& p : T.poly)
-            for (size_t i = 0; i < p.local_ids.size(); ++i) uniq.insert(erase_key(p.local_ids, i));
-        T.prod_features.assign(uniq.begin(), uniq.end());
     }
 }
 
@@ -398,48 +394,6 @@ void Model::set_potential(const std::vector<double>& coeffs) {
         throw std::invalid_argument("number of coefficients does not match the model");
     coeffs_ = coeffs;
     has_pot_ = true;
-}
-
-// polymlp_potential.cpp:25-156 with the factor 2 of polymlp_eval.cpp:12-20
-std::vector<std::vector<PotTerm>> Model::head_terms(int t) const {
-    const bool elim_conj = in_.gtinv;
-    const auto& T = types_[t];
-    const auto didx = index_of(T.prod_deriv);
-    const auto fidx = index_of(T.prod_features);
-    std::map<std::array<int, 3>, std::array<double, 2>> acc;
-    for (const auto& term : T.poly) {
-        int n_prods = 0;
-        for (int id : term.local_ids) n_prods += (int)T.features[id][0].ids.size();
-        const double c = 2.0 * coeffs_[term.global_id];
-        for (size_t i = 0; i < term.local_ids.size(); ++i) {
-            const int head_feature = term.local_ids[i];
-            const int pf = fidx.at(erase_key(term.local_ids, i));
-            for (const auto& s : T.features[head_feature]) {
-                const double cf = c * s.coeff;
-                const double ce = cf / double(n_prods);
-                for (size_t j = 0; j < s.ids.size(); ++j) {
-                    const int head = s.ids[j];
-                    if (elim_conj && T.nlm[head].conj) continue;
-                    const int pid = didx.at(erase_key(s.ids, j));
-                    auto& v = acc[{head, pid, pf}];
-                    v[0] += ce;
-                    v[1] += cf;
-                }
-            }
-        }
-    }
-    std::vector<std::vector<PotTerm>> pot(in_.gtinv ? T.noconj.size() : T.ntp.size());
-    for (const auto& kv : acc) {
-        const int head = kv.first[0];
-        const int slot = in_.gtinv ? T.local_to_noconj[head] : head;
-        pot[slot].push_back({kv.second[0], kv.second[1], kv.first[1], kv.first[2]});
-    }
-    for (auto& v : pot)
-        std::sort(v.begin(), v.end(), [](const PotTerm& a, const PotTerm& b) {
-            if (a.prod != b.prod) return a.prod < b.prod;
-            return a.prod_features < b.prod_features;
-        });
-    return pot;
 }
 
 }  // namespace plm

@@ -69,11 +69,6 @@ struct DerivTerm {
     int head, prod;  // local nlmtp id of the head, id of the product of the rest
 };
 
-struct PotTerm {
-    double coeff_e, coeff_f;
-    int prod, prod_features;
-};
-
 struct TypeTables {
     std::vector<NlmAttr> nlm;         // all local components (incl. conjugates)
     std::vector<int> noconj;          // local ids of non-conjugate components
@@ -87,7 +82,6 @@ struct TypeTables {
     std::vector<std::vector<int>> prod_deriv;            // products of all-but-head
     std::vector<std::vector<DerivTerm>> feat_deriv;      // feature -> deriv terms (sorted)
     std::vector<PolyTerm> poly;                          // polynomial columns of this type
-    std::vector<std::vector<int>> prod_features;         // products of features (poly)
 };
 
 class Model {
@@ -116,8 +110,6 @@ class Model {
     void set_potential(const std::vector<double>& coeffs);
     bool has_potential() const { return has_pot_; }
     const std::vector<double>& coeffs() const { return coeffs_; }
-    // the folded per-head terms of a type (plm_api_sum_of_prod)
-    std::vector<std::vector<PotTerm>> head_terms(int t) const;
 
   private:
     ModelInput in_;

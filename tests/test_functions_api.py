@@ -228,3 +228,22 @@ def test_device_polymlp_api(mgo_api, precision, tol):
             assert _close(f, rf, tol)
             pe, pf = capi.api_sum_of_prod(model, re, im, t, precision)
             assert _close(pe, rpe, 10 * tol) and _close(pf, rpf, 10 * tol)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,tol", [(capi.PLM_FP64, 1e-12), (capi.PLM_MIXED, 1e-5)])
+@pytest.mark.parametrize("lanes", ["64", "256"])
+def test_device_prod_sum_is_the_evaluations(mgo_api, lanes, precision, tol, monkeypatch):
+    """prod_sum comes from the evaluation's contraction kernel, in both of its
+    forms: the golden sums hold in each, and a form that it refuses is refused."""
+    spec, coeffs = mgo_api
+    model = capi.Model(spec.as_dict())
+    model.set_coeffs(coeffs)
+    n = 1899
+    monkeypatch.setenv("PLM_PRODSUM_LANES", lanes)
+    pe, pf = capi.api_sum_of_prod(model, np.arange(n), np.arange(n), 0, precision)
+    assert pe.sum() == pytest.approx(API_PROD_E_SUM, rel=max(tol, 1e-12))
+    assert pf.sum() == pytest.approx(API_PROD_F_SUM, rel=max(tol, 1e-12))
+    monkeypatch.setenv("PLM_PRODSUM_LANES", "7")
+    with pytest.raises(RuntimeError, match="PLM_PRODSUM_LANES"):
+        capi.api_sum_of_prod(model, np.arange(n), np.arange(n), 0, precision)
