@@ -108,6 +108,7 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
     __syncthreads();
     {
         // products with |Re| <= 1e-20 are dropped where the reference drops them
+        // (NaN is not one of them)
         const T least = TT.fv_skip ? T(1e-20) : T(-1);
         const T* c = EvalTab<T>::value(E);
         for (int bk = wave; bk < E.vq_nblk; bk += NW) {
@@ -117,7 +118,7 @@ __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, Ba
 #pragma unroll 2
             for (int r = E.vq_boff[bk] + lane; r < r1; r += 64) {
                 const T p = value_prod<T>(a, E.vq_key[r], ed.value_max).re;
-                v += fabs(p) > least ? c[r] * p : T(0);
+                v += fabs(p) <= least ? T(0) : c[r] * p;
             }
             if (f >= 0) xs[f] = v;
         }

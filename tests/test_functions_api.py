@@ -247,3 +247,24 @@ def test_device_prod_sum_is_the_evaluations(mgo_api, lanes, precision, tol, monk
     monkeypatch.setenv("PLM_PRODSUM_LANES", "7")
     with pytest.raises(RuntimeError, match="PLM_PRODSUM_LANES"):
         capi.api_sum_of_prod(model, np.arange(n), np.arange(n), 0, precision)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [capi.PLM_FP64, capi.PLM_MIXED])
+def test_device_prod_sum_keeps_nan(mgo_api, precision):
+    """A NaN order parameter reaches every head that depends on it, also through
+    the values of the polynomial's features."""
+    spec, coeffs = mgo_api
+    model = capi.Model(spec.as_dict())
+    model.set_coeffs(coeffs)
+    rng = np.random.default_rng(7)
+    re, im = rng.normal(size=270), rng.normal(size=270)
+    base = capi.api_sum_of_prod(model, re, im, 0, precision)
+    for k in (0, 15, 135):
+        moved, lost = re.copy(), re.copy()
+        moved[k] += 100.0
+        lost[k] = np.nan
+        for b, v, g in zip(base, capi.api_sum_of_prod(model, moved, im, 0, precision),
+                           capi.api_sum_of_prod(model, lost, im, 0, precision)):
+            depends = np.abs(v - b) > 1e-5 * np.abs(b).max()
+            assert depends.any() and np.isnan(g[depends]).all()
