@@ -1168,7 +1168,7 @@ int plm_features_x(plm_model* mp, plm_batch* bp, int precision, double* x_out) {
         if (!m->built) m->build_device();
         const bool fp64 = fp64_features(precision);
         const int F = m->host.n_features();
-        const long R = b->row_off.back();
+        if (F == 0) throw std::invalid_argument("model has no features");
         const int elem = fp64 ? 8 : 4;
         Device& dev = device();
         hipStream_t st = dev.stream;
@@ -1266,7 +1266,7 @@ int plm_normal_result(plm_normal* ap, double* xtx, double* xty, double* xe_sum, 
         // Gram of [X | y]: the upper element triangle is valid (the tiles cover
         // the upper block triangle), column F holds X^T y and element (F, F)
         // y^T y; the rows leave mirrored and unpadded, kOutBytes at a time
-        if (xtx || xty) {
+        if ((xtx || xty) && F > 0) {
             constexpr size_t kOutBytes = 128ull << 20;
             const int piece =
                 std::min<long>((F + 31) / 32, std::max<long>(1, (long)(kOutBytes / (256ull * F)))) * 32;

@@ -44,3 +44,19 @@ def test_rows_as_structure_by_structure(name):
         one = capi.features_x(m, batch([s]), precision)
         rows = np.concatenate([[k], len(sts) + 6 * k + np.arange(6), np.arange(off[k], off[k + 1])])
         assert np.all(np.abs(X[rows] - one) <= eps * scale)
+
+
+def test_model_without_features():
+    """No radial function in any type pair: rows are refused, as their kernels
+    have nothing to launch, and the normal equations are empty."""
+    spec = ModelSpec(n_type=1, cutoff=4.0, feature_type="pair", model_type=2, max_p=2,
+                     gtinv_order=0, gtinv_maxl=(), gaussian_params1=(1.0, 1.0, 1),
+                     gaussian_params2=(0.0, 3.0, 4), pair_params_conditional={(0, 0): []})
+    m = capi.Model(spec.as_dict())
+    assert m.n_features == 0
+    s = datasets.config4_structure(reps=(2, 2, 2))
+    b = capi.Batch(m, [s.axis], [s.positions_cartesian], [s.types])
+    with pytest.raises(RuntimeError):
+        capi.features_x(m, b)
+    xtx, xty, s1, s2, y_sq, n = capi.Normal(m).result()
+    assert xtx.shape == (0, 0) and xty.shape == (0,) and y_sq == 0.0 and n == 0
