@@ -1133,6 +1133,8 @@ int plm_batch_create(const plm_model* m, int n_st, const double* axes, const dou
         if (!mh->built) mh->build_device();
         auto b = std::make_unique<BatchHandle>(mh, mh->host.input().cutoff, n_st, axes, pos, types,
                                                n_atoms);
+        // the lists' fill is still queued; the caller's batch is complete
+        check_hip(hipStreamSynchronize(device().stream), "sync");
         *out = reinterpret_cast<plm_batch*>(b.release());
     });
 }

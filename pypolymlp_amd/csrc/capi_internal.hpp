@@ -29,7 +29,9 @@ void check_hip(hipError_t e, const char* what);
 
 // Device memory from the library's pool (capi.cpp): released blocks are kept
 // for later buffers of all handles. Everything the library enqueues goes
-// through one stream, so a block may be handed on while work on it is queued.
+// through one stream, so a block may be handed on while work on it is queued;
+// the synchronous copies (Store::upload, plm_normal_result) are on the null
+// stream and wait for it because it is created as a blocking stream.
 struct DevBuf {
     void* ptr = nullptr;
     size_t bytes = 0;
