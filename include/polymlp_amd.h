@@ -16,6 +16,8 @@
 #ifndef POLYMLP_AMD_H
 #define POLYMLP_AMD_H
 
+#include <stddef.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -70,6 +72,12 @@ typedef struct plm_model_desc {
 
 const char* plm_last_error(void);
 int plm_device_count(int* n);
+
+/* Device memory of finished calls is kept for later ones: up to an eighth of the
+ * card while any handle lives, at most 1 GiB when none does. This gives it back
+ * (for another allocator, which fails on it otherwise); bytes, which may be
+ * NULL, receives how much that was. No counterpart in the reference. */
+int plm_release_memory(size_t* bytes);
 
 /* Model setup: Mapping / ModelParams / Features / FeaturesPoly
  * (src/cxx/src/polymlp/polymlp_features.cpp:27-59). Uploads the tables. */

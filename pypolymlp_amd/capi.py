@@ -35,7 +35,7 @@ EXPORTS = [
     "plm_eval_graph_destroy", "plm_profile_enable", "plm_profile_reset", "plm_profile_get",
     "plm_surrogate_n_params", "plm_surrogate_train", "plm_surrogate_grad",
     "plm_surrogate_predict", "plm_get_fn", "plm_get_ylm", "plm_api_features",
-    "plm_api_sum_of_prod",
+    "plm_api_sum_of_prod", "plm_release_memory",
 ]
 
 _dp = ctypes.POINTER(ctypes.c_double)
@@ -116,6 +116,7 @@ def lib():
         L.plm_get_ylm.argtypes = [ctypes.c_int, _dp, ctypes.c_int, ctypes.c_int, _dp, _dp]
         L.plm_api_features.argtypes = [vp, ctypes.c_int, _dp, _dp, ctypes.c_int, _dp, _dp]
         L.plm_api_sum_of_prod.argtypes = [vp, ctypes.c_int, _dp, _dp, ctypes.c_int, _dp, _dp]
+        L.plm_release_memory.argtypes = [ctypes.POINTER(ctypes.c_size_t)]
         _lib = L
     return _lib
 
@@ -139,6 +140,14 @@ def _pd(a):
 
 def _pi(a):
     return a.ctypes.data_as(_ip) if a is not None else None
+
+
+def release_memory() -> int:
+    """Give the device memory kept for later calls back (plm_release_memory);
+    returns its bytes."""
+    n = ctypes.c_size_t()
+    _check(lib().plm_release_memory(ctypes.byref(n)))
+    return n.value
 
 
 class Model:

@@ -33,12 +33,15 @@ void check_hip(hipError_t e, const char* what) {
 }
 
 // ---------------------------------------------------------------------------
-// Device memory pool. A fit allocates and frees tens of GB; freed device memory
-// is not at once available again, so that repeated passes slowed down from 157
-// ms to 0.4-4 s each once they had gone through the card's memory. Released
-// blocks are kept up to an eighth of the device memory (the oldest given back
-// beyond that), all of them but 1 GiB are given back when no buffer is in use,
-// and all when an allocation fails.
+// Device memory pool. A fit allocates and frees tens of GB (a mixed fit of 200
+// alloys 30); freed device memory is not at once available again, so that
+// repeated passes slowed down from 157 ms to 0.4-4 s each once they had gone
+// through the card's memory, and do so again with a bound of 1 to 16 GiB.
+// Released blocks are kept up to an eighth of the device memory (the oldest
+// given back beyond that) for as long as any handle holds a buffer; all but
+// 1 GiB are given back with the last buffer, and all when an allocation of this
+// library fails or plm_release_memory asks for it (another allocator, of this
+// process or not, finds the idle blocks taken).
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -88,10 +91,15 @@ class DevPool {
             e = hipMalloc(&p, size);
         }
         check_hip(e, "hipMalloc");
-        in_use[p] = size;
+        try {
+            in_use[p] = size;
+        } catch (...) {
+            (void)hipFree(p);
+            throw;
+        }
         return p;
     }
-    void give(void* p) {
+    void give(void* p) noexcept {
         std::lock_guard<std::mutex> lock(mu);
         auto it = in_use.find(p);
         if (it == in_use.end()) return;
@@ -99,14 +107,24 @@ class DevPool {
             size_t f = 0, total = 0;
             bound = hipMemGetInfo(&f, &total) == hipSuccess ? total / 8 : (4ull << 30);
         }
-        idle.emplace(it->second, Block{p, ++tick});
-        cached += it->second;
+        try {
+            idle.emplace(it->second, Block{p, ++tick});
+            cached += it->second;
+        } catch (...) {  // no host memory to keep it by
+            (void)hipFree(p);
+        }
         in_use.erase(it);
         trim(in_use.empty() ? std::min<size_t>(bound, 1ull << 30) : bound);
     }
     size_t cached_bytes() {
         std::lock_guard<std::mutex> lock(mu);
         return cached;
+    }
+    size_t give_back() {
+        std::lock_guard<std::mutex> lock(mu);
+        const size_t n = cached;
+        trim(0);
+        return n;
     }
 };
 
@@ -1033,6 +1051,13 @@ int plm_device_count(int* n) {
         int c = 0;
         if (hipGetDeviceCount(&c) != hipSuccess) c = 0;
         *n = c;
+    });
+}
+
+int plm_release_memory(size_t* bytes) {
+    PLM_TRY({
+        const size_t n = pool().give_back();
+        if (bytes) *bytes = n;
     });
 }
 

@@ -64,3 +64,22 @@ def test_ridge_after_larger_buffers():
         c = mlp_dev.solver_ridge(A, A @ np.ones(F), np.array([1e-9, 1e-8]))
         res.append(np.abs(c - 1.0).max())
     assert max(res) < 1e-6
+
+
+def test_idle_memory_is_given_back_on_request():
+    """A model keeps the pool's idle blocks alive (a GiB and more of X here);
+    they are free for another allocator after release_memory, and results stay."""
+    import torch
+
+    spec = datasets.config1_model()
+    sts = [datasets.config4_structure(seed=k, reps=(4, 4, 4)) for k in range(120)]
+    run = job(spec, sts, 5)
+    first = run()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    given = capi.release_memory()
+    assert given >= 1 << 30
+    assert torch.cuda.mem_get_info()[0] - free >= given // 2
+    assert capi.release_memory() == 0
+    for a, b in zip(run(), first):
+        assert close(a, b)
