@@ -3,8 +3,11 @@ stresses are the energy, force and stress rows times c, and the rows come from
 kernels of their own. FP64, 1e-11 of the largest value per structure (sums of
 up to some thousand terms); at radial functions that do not fill the pair loop's
 rows of four, at each of its bounds on max_l, with neighbours around and past
-the 64 of an order-parameter chunk and more tiles than that form holds, with few pairs (keys split over
-workgroups) and many, with type pairs of unequal and no radial functions."""
+the 64 of an order-parameter chunk and more tiles than that form holds, with
+few pairs (keys split over workgroups), with type pairs of unequal and no radial
+functions. Cells of many atoms and pairs (a wave per atom in the contraction,
+unsplit keys, energies and stresses summed by several workgroups) are periodic
+replicas of a small cell whose rows are known."""
 
 import numpy as np
 import pytest
@@ -89,6 +92,39 @@ def test_eval_matches_rows(name, form, monkeypatch):
         assert np.abs(S[k] - y[rows]).max() <= 1e-11 * size[rows].max() + 1e-13
         assert np.abs(F[k].reshape(-1) - y[at:at + n]).max() <= 1e-11 * size[at:at + n].max() + 1e-13
         at += n
+
+
+# from 8,192 atoms on a wave per atom contracts, from 2,048 waves of half pairs on
+# a lane takes all keys, from 4,096 on several workgroups add a structure up
+REPLICAS = {
+    "metal": (spec(max_l=(2,), n_gauss=3), 7),
+    "pair": (spec(n_type=2, max_l=(), n_gauss=5), 7),
+    "alloy": (spec(n_type=2, max_l=(4, 2), n_gauss=3, model_type=3), 6),
+}
+
+
+@pytest.mark.parametrize("precision", [capi.PLM_FP64, capi.PLM_MIXED])
+@pytest.mark.parametrize("name", sorted(REPLICAS))
+def test_large_cell_matches_rows_of_its_unit(name, precision):
+    sp, reps = REPLICAS[name]
+    s = structure(54, 9.3, sp.n_type, 3)
+    pos, types = s.positions_cartesian, np.array(s.types)
+    m = capi.Model(sp.as_dict())
+    b = capi.Batch(m, [s.axis], [pos], [types])
+    X = capi.features_x(m, b)
+    scale = np.abs(X).max(axis=0)
+    c = np.random.default_rng(1).normal(size=X.shape[1]) / np.where(scale > 1e-8, scale, 1e8)
+    m.set_coeffs(c)
+    y, size = X @ c, np.abs(X) @ np.abs(c)
+    cells = np.mgrid[0:reps, 0:reps, 0:reps].reshape(3, -1)
+    n = cells.shape[1]
+    large = (pos[:, None, :] + (s.axis @ cells)[:, :, None]).reshape(3, -1)
+    big = capi.Batch(m, [s.axis * reps], [large], [np.tile(types, n)])
+    assert 54 * n >= 8192 and big.n_pairs // 2 >= 64 * (4096 if name != "alloy" else 2048)
+    E, F, S = capi.eval_batch(m, big, precision)
+    assert abs(E[0] - n * y[0]) <= 1e-11 * n * size[0]
+    assert np.abs(S[0] - n * y[1:7]).max() <= 1e-11 * n * size[1:7].max()
+    assert np.abs(F[0].reshape(n, -1) - y[7:]).max() <= 1e-11 * size[7:].max()
 
 
 @pytest.mark.parametrize("max_p,model_type", [(2, 4), (3, 3)])

@@ -19,14 +19,15 @@ def model(n_gauss, max_l, max_p=2, n_type=1, model_type=4):
 
 
 # (model, structures): 1 tile and few rows; one column short of and past whole
-# tiles with [X | y]; row splits down to 512 rows; more than 512 tiles
-# (4,395 columns) with a rest
+# tiles with [X | y]; row splits down to 512 rows; more than 512 tiles (4,395
+# columns: 630) with one round in whole rows and the rest in three row splits, the
+# last of them shorter (1,856 padded rows: 624, 624 and 608)
 CASES = {
     "one_tile": (model(2, (2,)), 1),
     "two_tiles": (model(4, (2,)), 7),
     "split_512": (model(7, (4,)), 7),
     "split_many": (model(6, (4,)), 60),
-    "many_tiles": (model(14, (4, 4)), 4),
+    "many_tiles": (model(14, (4, 4)), 13),
 }
 
 

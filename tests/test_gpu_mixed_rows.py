@@ -1,4 +1,4 @@
-"""Energy rows of the mixed form are FP32 sums over the atoms in their order, each
+"""Energy rows and column scales of the mixed form. The energy rows are FP32 sums over the atoms in their order, each
 product rounded before it is added. Structures of separate dimers of several
 lengths: both atoms of a dimer have its FP32 pair features, half of what the
 linear columns of the dimer alone hold (a sum of two equal numbers, exact), so
@@ -7,7 +7,7 @@ numpy adds the same products in the same order and every bit is known."""
 import numpy as np
 import pytest
 
-from pypolymlp_amd import capi
+from pypolymlp_amd import capi, datasets, mlp_dev
 from pypolymlp_amd.params import ModelSpec
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +61,22 @@ def test_energy_rows_add_atoms_in_order(sizes, max_p):
             want = want + p[q]
             want = want + p[q]
         assert np.array_equal(g, want.astype(np.float64))
+
+
+def test_scales_of_an_alloy_set_against_64_bits():
+    """A column's scale is the spread of its energy row over the structures, so it
+    moves by no more than the rms of the row's change. The variance is a difference
+    of sums: its rounding is magnified by mean over spread."""
+    ds = datasets.config2_dataset(24)
+    m = capi.Model(datasets.config2_model().as_dict())
+    sts = ds.structures
+    b = capi.Batch(m, [s.axis for s in sts], [s.positions_cartesian for s in sts],
+                   [s.types for s in sts])
+    e64, e32 = (capi.features_x(m, b, p)[:len(sts)] for p in (capi.PLM_FP64, capi.PLM_MIXED))
+    off = np.sqrt(np.mean((e32 - e64) ** 2, axis=0))
+    rms = np.sqrt(np.mean(e64 ** 2, axis=0))
+    spread = e64.std(axis=0)
+    kept = spread > 1e-8
+    scales = mlp_dev.calc_xtx_xty(m, [ds], capi.PLM_MIXED).scales
+    rounding = 1e-14 * rms[kept] ** 2 / spread[kept]
+    assert np.all(np.abs(scales[kept] - spread[kept]) <= off[kept] + rounding)
