@@ -6,6 +6,7 @@
 #include <array>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <numeric>
 #include <stdexcept>
 #include <vector>
@@ -15,10 +16,35 @@
 
 namespace plm {
 
+namespace {
+
+// Host tables of one potential, laid end to end, uploaded by one copy (about 20
+// small arrays a type: one by one they cost 10 us each, most of set_coeffs for a
+// small model).
+struct TableUpload {
+    std::vector<unsigned char> data;
+    std::vector<std::pair<size_t, std::function<void(const unsigned char*)>>> set;
+    template <class V>
+    void put(const V*& dst, const std::vector<V>& v) {
+        const size_t at = (data.size() + 63) / 64 * 64;
+        data.resize(at + std::max<size_t>(1, v.size()) * sizeof(V));
+        if (!v.empty()) std::memcpy(data.data() + at, v.data(), v.size() * sizeof(V));
+        set.push_back({at, [&dst](const unsigned char* p) { dst = reinterpret_cast<const V*>(p); }});
+    }
+    void upload(Store& store) {
+        const unsigned char* base = store.upload(data.data(), data.size());
+        for (auto& s : set) s.second(base + s.first);
+    }
+};
+
+}  // namespace
+
 void upload_potential(ModelHandle& m) {
     const Model& M = m.host;
     if (!M.has_potential()) throw std::runtime_error("coefficients not set");
     m.pot_store.bufs.clear();
+    m.pot_uploaded = false;
+    TableUpload tables;
     const int nt = M.n_type(), ntp = M.n_tp();
     const bool gt = M.input().gtinv;
     m.max_heads = 0;
@@ -113,10 +139,6 @@ void upload_potential(ModelHandle& m) {
                     hj[hoff[tp]] != tp_first[t2][tp])
                     throw std::invalid_argument("evaluation head order");
         }
-        auto upv = [&](const auto& v) {
-            using V = typename std::decay_t<decltype(v)>::value_type;
-            return m.pot_store.upload(v.data(), v.size() * sizeof(V));
-        };
         auto k16 = [](int v) -> unsigned {
             if (v < 0 || v >= 0xffff) throw std::invalid_argument("evaluation table index exceeds 16 bits");
             return (unsigned)v;
@@ -294,22 +316,23 @@ void upload_potential(ModelHandle& m) {
             const int k = order[t][r];
             ha[r] = gt ? T.noconj[k] | (T.nlm[T.noconj[k]].m == 0 ? 1 << 30 : 0) : k;
         }
-        E.hd_a = upv(ha);
-        E.vq_boff = upv(vboff), E.vq_item = upv(vitem), E.vq_key = upv(vkey);
-        E.vq_c = upv(vc), E.vq_cf = upv(vcf);
-        E.pf_boff = upv(pf_boff), E.pf_piece = upv(pf_piece), E.pf_rec = upv(pf_rec), E.pf_lin = upv(pf_lin);
-        E.pf_c = upv(pf_c), E.pf_cf = upv(pf_cf);
-        E.tq_boff = upv(boff), E.tq_item = upv(item), E.tq_key = upv(key);
-        E.tq_c = upv(tc), E.tq_cf = upv(tcf);
+        tables.put(E.hd_a, ha);
+        tables.put(E.vq_boff, vboff), tables.put(E.vq_item, vitem), tables.put(E.vq_key, vkey);
+        tables.put(E.vq_c, vc), tables.put(E.vq_cf, vcf);
+        tables.put(E.pf_boff, pf_boff), tables.put(E.pf_piece, pf_piece);
+        tables.put(E.pf_rec, pf_rec), tables.put(E.pf_lin, pf_lin);
+        tables.put(E.pf_c, pf_c), tables.put(E.pf_cf, pf_cf);
+        tables.put(E.tq_boff, boff), tables.put(E.tq_item, item), tables.put(E.tq_key, key);
+        tables.put(E.tq_c, tc), tables.put(E.tq_cf, tcf);
         std::vector<int4> rec(std::max<size_t>(1, nid.size()), int4{0, 0, 0, 0});
         for (size_t h = 0; h < nid.size(); ++h) {
             if (hj[h] < 0 || hj[h] >= (1 << 28)) throw std::invalid_argument("head index range");
             rec[h] = int4{nid[h], ylm[h], hi[h],
                           hj[h] | (sj[h] < 0.f ? 1 << 28 : 0) | (m0[h] ? 1 << 29 : 0)};
         }
-        E.hd_off = upv(hoff);
-        E.hd_rec = static_cast<const int4*>(upv(rec));
+        tables.put(E.hd_off, hoff), tables.put(E.hd_rec, rec);
     }
+    tables.upload(m.pot_store);
     m.pot_uploaded = true;
     ++m.pot_version;
 }

@@ -160,9 +160,6 @@ void launch_pair(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& e
                  const void* ps_f, int ps_stride, double* part, double* energy, double* forces,
                  double* stress, int pair_model);
 
-// X^T X with the weighted targets in column F of X (ld >= F + 1, multiple of
-// 128; rows_pad multiple of 64). Mixed: quantise X into the int8 slice buffer
-// (gram_quant_bytes) then accumulate the exact Gram of the quantised X.
 // out[q] = X[src[q]] as doubles for q < rows, F columns each
 void launch_gather_rows(hipStream_t st, bool fp64, const void* X, int ld, const int* src, int rows,
                         int F, double* out);
@@ -172,6 +169,9 @@ void launch_gather_rows(hipStream_t st, bool fp64, const void* X, int ld, const 
 void launch_gram_mirror(hipStream_t st, const double* G, int ldg, int F, int i0, int rows,
                         double* out, double* xty);
 
+// X^T X with the weighted targets in column F of X (ld >= F + 1, multiple of
+// 128; rows_pad multiple of 64). Mixed: quantise X into the int8 slice buffer
+// (gram_quant_bytes) then accumulate the exact Gram of the quantised X.
 void launch_set_column(hipStream_t st, bool fp64, void* X, int ld, int col, const double* y,
                        int rows);
 // part: gram_f64_part_bytes of scratch for the row splits (unused where that is 0)
