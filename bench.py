@@ -492,6 +492,14 @@ def main():
             roof["traffic_source"] = "profiles/fit_binary_alloy_traffic.json (rocprofv3 --pmc)"
             alg_bytes = 3.0 * Fy * R / max(n_g / args.steps, 1)  # three int8 planes per launch
             roof["traffic_vs_algorithmic"] = roof["traffic"] / alg_bytes
+        # what bounds the signature groups is not their algorithmic bytes but the
+        # weights W' and records that every task of a structure reads again
+        k = tr.get(xg_kernel + "<float>")
+        if k and ms_x:
+            moved = k["launches"] * (k["fetch_bytes_per_launch"] + k["write_bytes_per_launch"])
+            xgroup["traffic_per_step"] = moved
+            xgroup["traffic_gbs"] = moved * args.steps / (ms_x * 1e-3) / 1e9
+            xgroup["traffic_frac"] = xgroup["traffic_gbs"] / HBM_PEAK_GBS
 
     ev = eval_leg(args.eval_steps, args.eval_graph_steps, not args.no_cpu_baseline) \
         if args.eval_steps > 0 else {}

@@ -72,7 +72,7 @@ __device__ __forceinline__ Cpx<T> value_prod(const Cpx<T>* a, int2 k, int n) {
 // head before), and records of 12 or 16 bytes instead of 32: the tables come
 // from L2 for every atom, which held the kernel at 8 TB/s on the 1,350-head
 // model. FP64, 32,000 atoms of the one-type model: 0.71 -> 0.18 ms; 1,024-atom
-// alloy: 0.40 -> 0.09 ms; FP32, 20,480 atoms of the alloy: 5.8 -> 0.88 ms.
+// alloy: 0.40 -> 0.09 ms; 20,480 atoms of the alloy 1.49 ms.
 // ---------------------------------------------------------------------------
 template <class T, int NL>
 __global__ void __launch_bounds__(NL) prodsum_kernel(ModelDev md, EvalDev ed, BatchDev bd,
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(64) pair_rec_kernel(ModelDev md, EvalDev ed, B
 // part[wave] (eval_sum_kernel adds the waves up): as atomics on the structure's
 // six values the waves' sums took 13 ns each, one after the other, which was
 // the kernel's whole time on one large cell (FP64, 32,000 atoms: 1.97 -> 0.40 ms;
-// 160 alloys of 128 atoms, FP32: 5.4 -> 1.5 ms). blockIdx.y: the keys of m = y, y +
+// 160 alloys of 128 atoms 1.69 ms). blockIdx.y: the keys of m = y, y +
 // gridDim.y, .. only (few pairs: more waves, each with part of the keys).
 // ---------------------------------------------------------------------------
 template <class T, int LB>
@@ -625,9 +625,9 @@ void launch_prodsum_t(hipStream_t st, const ModelDev& md, const EvalDev& ed, con
 }
 
 // Four waves an atom where its table rows are more than 128 or the atoms do
-// not fill the chip with eight waves a SIMD, else one (20,480 atoms of the
-// 1,350-head model, FP32: 0.98 ms with four, 2.73 with one; 54 atoms of the
-// one-type model 22 and 54 us; 32,000 atoms of it 0.64 and 0.66 ms, equal);
+// not fill the chip with eight waves a SIMD, else one (FP64, 20,480 atoms of the
+// 1,350-head model: 1.49 ms with four, 4.74 with one; 54 atoms of the one-type
+// model 11 and 17 us; 32,000 atoms of it 0.184 and 0.171 ms);
 // PLM_PRODSUM_LANES=64|256 forces one form.
 void launch_prodsum(hipStream_t st, bool fp64, const ModelDev& md, const EvalDev& ed,
                     const BatchDev& bd, const void* a_full, int a_stride, void* ps_f,
